@@ -72,6 +72,29 @@ __device__ __forceinline__ float block_lse(float m, float s) {
   return M + __logf(S);
 }
 
+// A row of V bf16 values at p as 16-byte words: `head` values before the first
+// 16-byte boundary, n8 whole words from there, then the rest.  Rows of an odd
+// vocabulary start at any even address, so a row's head differs from the next
+// one's; the few head and tail values are read one by one, each by a thread of
+// its own (their loads go out beside the words').  2048 x 50257, HBM-bound:
+// forward 40 us (5.1 TB/s), backward 90 us (4.6 TB/s); with 2-byte accesses for
+// every row that is not 16-byte aligned they took 112 and 181 us.
+struct RowSplit {
+  int head;            // values before the words
+  int64_t n8, tail0;   // words; first value after them
+  __device__ __forceinline__ RowSplit(const uint16_t* p, int64_t V) {
+    const int64_t h = (int64_t)((0u - (uint32_t)(reinterpret_cast<uintptr_t>(p) >> 1)) & 7u);
+    head = (int)(h < V ? h : V);
+    n8 = (V - head) >> 3;
+    tail0 = head + 8 * n8;
+  }
+  // the single value of this thread, or -1: threads 0 .. 7 take the head, 8 .. 15 the tail
+  __device__ __forceinline__ int64_t single(int64_t V) const {
+    const int64_t i = threadIdx.x < 8 ? (int64_t)threadIdx.x : tail0 + (int64_t)threadIdx.x - 8;
+    return (threadIdx.x < 8 ? i < head : threadIdx.x < 16 && i < V) ? i : -1;
+  }
+};
+
 // z of the 8 bf16 values of one 16-byte word
 __device__ __forceinline__ void capped8(const uint4& w, float cap, float inv_cap, float* z) {
   const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
@@ -93,7 +116,6 @@ __device__ __forceinline__ void lse_accum(const float* z, float& m, float& s) {
   lse_merge(m, s, zm, part);
 }
 
-template <bool VEC>
 __global__ __launch_bounds__(kXentThreads) void xent_fwd_kernel(const uint16_t* __restrict__ logits,
                                                                const int64_t* __restrict__ tgt,
                                                                int64_t V, float cap, float inv_cap,
@@ -102,29 +124,25 @@ __global__ __launch_bounds__(kXentThreads) void xent_fwd_kernel(const uint16_t* 
   const int64_t row = blockIdx.x;
   const uint16_t* lr = logits + row * V;
   float m = -__builtin_inff(), s = 0.0f;
-  if (VEC) {
-    const uint4* p = reinterpret_cast<const uint4*>(lr);
-    const int64_t n8 = V / 8;
-    int64_t c = threadIdx.x;
-    for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
-      uint4 w[kXentUnroll];
+  const RowSplit rs(lr, V);
+  const int64_t si = rs.single(V);
+  if (si >= 0) lse_merge(m, s, capped(__uint_as_float((uint32_t)lr[si] << 16), cap, inv_cap), 1.0f);
+  const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
+  const int64_t n8 = rs.n8;
+  int64_t c = threadIdx.x;
+  for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
+    uint4 w[kXentUnroll];
 #pragma unroll
-      for (int u = 0; u < kXentUnroll; ++u) w[u] = ldg_stream(p + c + u * kXentThreads);
-      float z[8 * kXentUnroll];
+    for (int u = 0; u < kXentUnroll; ++u) w[u] = ldg_stream(p + c + u * kXentThreads);
+    float z[8 * kXentUnroll];
 #pragma unroll
-      for (int u = 0; u < kXentUnroll; ++u) capped8(w[u], cap, inv_cap, z + 8 * u);
-      lse_accum<8 * kXentUnroll>(z, m, s);
-    }
-    for (; c < n8; c += kXentThreads) {
-      float z[8];
-      capped8(ldg_stream(p + c), cap, inv_cap, z);
-      lse_accum<8>(z, m, s);
-    }
-  } else {
-    for (int64_t i = threadIdx.x; i < V; i += kXentThreads) {
-      const float z = capped(__uint_as_float((uint32_t)lr[i] << 16), cap, inv_cap);
-      lse_merge(m, s, z, 1.0f);
-    }
+    for (int u = 0; u < kXentUnroll; ++u) capped8(w[u], cap, inv_cap, z + 8 * u);
+    lse_accum<8 * kXentUnroll>(z, m, s);
+  }
+  for (; c < n8; c += kXentThreads) {
+    float z[8];
+    capped8(ldg_stream(p + c), cap, inv_cap, z);
+    lse_accum<8>(z, m, s);
   }
   const float lse = block_lse(m, s);
   if (threadIdx.x == 0) {
@@ -166,10 +184,16 @@ __global__ __launch_bounds__(kXentThreads) void xent_bwd_kernel(const uint16_t* 
       o[e] = pack_bf16x2(grad(bf16lo(ww[e]), i0 + 2 * e), grad(bf16hi(ww[e]), i0 + 2 * e + 1));
     return make_uint4(o[0], o[1], o[2], o[3]);
   };
+  auto put1 = [&](int64_t i) {
+    dr[i] = (uint16_t)(pack_bf16x2(grad(__uint_as_float((uint32_t)lr[i] << 16), i), 0.0f) & 0xFFFFu);
+  };
   if (VEC) {
-    const uint4* p = reinterpret_cast<const uint4*>(lr);
-    uint4* q = reinterpret_cast<uint4*>(dr);
-    const int64_t n8 = V / 8;
+    const RowSplit rs(lr, V);
+    const int64_t si = rs.single(V);
+    if (si >= 0) put1(si);
+    const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
+    uint4* q = reinterpret_cast<uint4*>(dr + rs.head);
+    const int64_t n8 = rs.n8, i0 = rs.head;
     int64_t c = threadIdx.x;
     for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
       uint4 w[kXentUnroll];
@@ -178,15 +202,12 @@ __global__ __launch_bounds__(kXentThreads) void xent_bwd_kernel(const uint16_t* 
 #pragma unroll
       for (int u = 0; u < kXentUnroll; ++u) {
         const int64_t cu = c + u * kXentThreads;
-        stg_stream(q + cu, grad8(w[u], 8 * cu));
+        stg_stream(q + cu, grad8(w[u], i0 + 8 * cu));
       }
     }
-    for (; c < n8; c += kXentThreads) stg_stream(q + c, grad8(ldg_stream(p + c), 8 * c));
+    for (; c < n8; c += kXentThreads) stg_stream(q + c, grad8(ldg_stream(p + c), i0 + 8 * c));
   } else {
-    for (int64_t i = threadIdx.x; i < V; i += kXentThreads) {
-      const float d = grad(__uint_as_float((uint32_t)lr[i] << 16), i);
-      dr[i] = (uint16_t)(pack_bf16x2(d, 0.0f) & 0xFFFFu);
-    }
+    for (int64_t i = threadIdx.x; i < V; i += kXentThreads) put1(i);
   }
 }
 
@@ -255,7 +276,6 @@ __device__ __forceinline__ float block_sum_max(float s, uint32_t& mx, float* red
   return t;
 }
 
-template <bool VEC>
 __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(8))) void xent_fwd_lut_kernel(const uint16_t* __restrict__ logits,
                                                                    const int64_t* __restrict__ tgt,
                                                                    int64_t rows, int64_t V, float cap,
@@ -274,29 +294,28 @@ __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(8)
       s += lut_at(lut, o0) + lut_at(lut, o1);
       mx = max(mx, max(m0, m1));
     };
-    if (VEC) {
-      const uint4* p = reinterpret_cast<const uint4*>(lr);
-      const int64_t n8 = V / 8;
-      int64_t c = threadIdx.x;
-      for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
-        uint4 w[kXentUnroll];
+    const RowSplit rs(lr, V);
+    const int64_t si = rs.single(V);
+    if (si >= 0) {
+      uint32_t m;
+      s += lut_at(lut, lut_off<false>((uint32_t)lr[si], m));
+      mx = m;
+    }
+    const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
+    const int64_t n8 = rs.n8;
+    int64_t c = threadIdx.x;
+    for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
+      uint4 w[kXentUnroll];
 #pragma unroll
-        for (int u = 0; u < kXentUnroll; ++u) w[u] = ldg_stream(p + c + u * kXentThreads);
+      for (int u = 0; u < kXentUnroll; ++u) w[u] = ldg_stream(p + c + u * kXentThreads);
 #pragma unroll
-        for (int u = 0; u < kXentUnroll; ++u) {
-          add_word(w[u].x); add_word(w[u].y); add_word(w[u].z); add_word(w[u].w);
-        }
+      for (int u = 0; u < kXentUnroll; ++u) {
+        add_word(w[u].x); add_word(w[u].y); add_word(w[u].z); add_word(w[u].w);
       }
-      for (; c < n8; c += kXentThreads) {
-        const uint4 w = ldg_stream(p + c);
-        add_word(w.x); add_word(w.y); add_word(w.z); add_word(w.w);
-      }
-    } else {
-      for (int64_t i = threadIdx.x; i < V; i += kXentThreads) {
-        uint32_t m;
-        s += lut_at(lut, lut_off<false>((uint32_t)lr[i], m));
-        mx = max(mx, m);
-      }
+    }
+    for (; c < n8; c += kXentThreads) {
+      const uint4 w = ldg_stream(p + c);
+      add_word(w.x); add_word(w.y); add_word(w.z); add_word(w.w);
     }
     const float S = block_sum_max(s, mx, red);
     if (threadIdx.x == 0) {
@@ -339,19 +358,28 @@ __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(6)
     auto grad_fast = [&](uint32_t off) {
       return lut_at(lut, off) * cg * lut_at(lut + 2 * kLutN, off & 0x3FFFu);
     };
+    auto put1 = [&](int64_t i) {
+      uint32_t m;
+      const float d = grad(lut_off<false>((uint32_t)lr[i], m), i);
+      dr[i] = (uint16_t)(pack_bf16x2(d, 0.0f) & 0xFFFFu);
+    };
     if (VEC) {
-      const uint4* p = reinterpret_cast<const uint4*>(lr);
-      uint4* q = reinterpret_cast<uint4*>(dr);
-      const int64_t n8 = V / 8;
+      const RowSplit rs(lr, V);
+      const int64_t si = rs.single(V);
+      if (si >= 0) put1(si);
+      const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
+      uint4* q = reinterpret_cast<uint4*>(dr + rs.head);
+      const int64_t n8 = rs.n8, tw = t - rs.head;    // the target, counted from the words
       auto grad8 = [&](const uint4& w, int64_t c) {
         const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
         uint32_t o[4];
         uint32_t m;
-        if ((uint64_t)(t - 8 * c) < 8u) {            // the target is in this chunk
+        if ((uint64_t)(tw - 8 * c) < 8u) {           // the target is in this chunk
+          const int64_t i0 = rs.head + 8 * c;
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            o[e] = pack_bf16x2(grad(lut_off<false>(ww[e], m), 8 * c + 2 * e),
-                               grad(lut_off<true>(ww[e], m), 8 * c + 2 * e + 1));
+            o[e] = pack_bf16x2(grad(lut_off<false>(ww[e], m), i0 + 2 * e),
+                               grad(lut_off<true>(ww[e], m), i0 + 2 * e + 1));
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -372,11 +400,7 @@ __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(6)
       }
       for (; c < n8; c += kXentThreads) stg_stream(q + c, grad8(ldg_stream(p + c), c));
     } else {
-      for (int64_t i = threadIdx.x; i < V; i += kXentThreads) {
-        uint32_t m;
-        const float d = grad(lut_off<false>((uint32_t)lr[i], m), i);
-        dr[i] = (uint16_t)(pack_bf16x2(d, 0.0f) & 0xFFFFu);
-      }
+      for (int64_t i = threadIdx.x; i < V; i += kXentThreads) put1(i);
     }
   }
 }
@@ -422,24 +446,13 @@ extern "C" int tg_logit_cap_xent_fwd(const void* logits, const int64_t* targets,
   TG_TRY(xent_check(logits, targets, rows, vocab, cap));
   if (rows == 0) return TG_OK;
   if (!row_loss || !row_lse) return einval("logit_cap_xent_fwd: null pointer");
-  const bool vec = vocab % 8 == 0 && aligned(logits, 16);
   auto L = reinterpret_cast<const uint16_t*>(logits);
-  if (cap <= kLutCapMax) {
-    const dim3 grid((unsigned)(rows < kLutGridFwd ? rows : kLutGridFwd));
-    if (vec)
-      hipLaunchKernelGGL(xent_fwd_lut_kernel<true>, grid, dim3(kXentThreads), 0, as_stream(stream), L,
-                         targets, rows, vocab, cap, row_loss, row_lse);
-    else
-      hipLaunchKernelGGL(xent_fwd_lut_kernel<false>, grid, dim3(kXentThreads), 0, as_stream(stream), L,
-                         targets, rows, vocab, cap, row_loss, row_lse);
-    return check_launch("logit_cap_xent_fwd");
-  }
-  if (vec)
-    hipLaunchKernelGGL(xent_fwd_kernel<true>, dim3((unsigned)rows), dim3(kXentThreads), 0,
-                       as_stream(stream), L, targets, vocab, cap, 1.0f / cap, row_loss, row_lse);
+  if (cap <= kLutCapMax)
+    hipLaunchKernelGGL(xent_fwd_lut_kernel, dim3((unsigned)(rows < kLutGridFwd ? rows : kLutGridFwd)),
+                       dim3(kXentThreads), 0, as_stream(stream), L, targets, rows, vocab, cap, row_loss, row_lse);
   else
-    hipLaunchKernelGGL(xent_fwd_kernel<false>, dim3((unsigned)rows), dim3(kXentThreads), 0,
-                       as_stream(stream), L, targets, vocab, cap, 1.0f / cap, row_loss, row_lse);
+    hipLaunchKernelGGL(xent_fwd_kernel, dim3((unsigned)rows), dim3(kXentThreads), 0, as_stream(stream), L,
+                       targets, vocab, cap, 1.0f / cap, row_loss, row_lse);
   return check_launch("logit_cap_xent_fwd");
 }
 
@@ -450,7 +463,12 @@ extern "C" int tg_logit_cap_xent_bwd(const void* logits, const int64_t* targets,
   TG_TRY(xent_check(logits, targets, rows, vocab, cap));
   if (rows == 0) return TG_OK;
   if (!row_lse || !g || !dlogits) return einval("logit_cap_xent_bwd: null pointer");
-  const bool vec = vocab % 8 == 0 && aligned(logits, 16) && aligned(dlogits, 16);
+  // 16-byte accesses need the logits' and the gradient's rows to cross 16-byte
+  // boundaries at the same elements: true of any two 16-byte-aligned arrays
+  // (torch's), whatever the vocabulary; buffers offset from each other keep
+  // the element-wise loop
+  const bool vec = ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(dlogits)) & 15u) == 0 &&
+                   aligned(logits, 2);
   auto L = reinterpret_cast<const uint16_t*>(logits);
   auto D = reinterpret_cast<uint16_t*>(dlogits);
   if (cap <= kLutCapMax) {
