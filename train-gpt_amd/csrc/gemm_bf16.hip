@@ -15,8 +15,10 @@
 //   * Operands travel HBM -> LDS by buffer_load ... lds through a ring of four
 //     K32 stages (one barrier per stage), issued by one wave per SIMD.
 //   * dW contracts over the token axis, which is the row axis of both a and
-//     g, so the backward first packs a.T and g.T (bf16, rows padded to a
-//     multiple of 64 with zeros) and runs the same NT kernel.
+//     g: the contraction-major kernel reads them in place (g from its packed
+//     copy where its rows are not 16-byte aligned); only an f32 or unaligned
+//     a has a.T and g.T packed for the NT kernel.
+//   * Outputs with few tiles split the contraction over workgroups (q4_split_of).
 #include "tg_device.h"
 #include "tg_host.h"
 #include "gemm_tile.h"
@@ -190,6 +192,46 @@ __device__ __forceinline__ void q4_main_loop(const Q4Ctx& c, v4f (&acc)[4][8]) {
   }
 }
 
+// R rows of 128 bf16 from LDS (256-byte rows, chunk c of row r at
+// c ^ (r & 15)), rows r0 .. r0 + R - 1, to C rows mw + r, columns nw .. nw + 127,
+// by one wave.  Rows of N % 8 == 0 go out as 16-byte pieces, 16 lanes per row.
+// Other rows start at any even address: one row per instruction as 64
+// consecutive 4-byte words from its first 4-byte boundary, and a single value
+// at either end where one is left over (2-byte stores of whole pieces touched
+// every line eight times).
+template <int R, int PITCH>
+__device__ __forceinline__ void q4_store_rows(const uint8_t* l, __bf16* __restrict__ C, int M, int N, int mw, int nw,
+                                              int lane, int r0) {
+  if (N % 8 == 0) {
+    const int k = lane & 15;
+#pragma unroll
+    for (int q = 0; q < R / 4; ++q) {
+      const int r = r0 + q * 4 + (lane >> 4);
+      const int m = mw + r, n = nw + k * 8;
+      const uint4 v = *reinterpret_cast<const uint4*>(l + r * PITCH + ((k ^ (r & 15)) * 16));
+      if (m < M && n < N) *reinterpret_cast<uint4*>(C + (int64_t)m * N + n) = v;
+    }
+    return;
+  }
+  const int cnt = min(128, N - nw);
+  if (cnt <= 0) return;
+  auto at = [&](int r, int e) {
+    return *reinterpret_cast<const uint16_t*>(l + r * PITCH + (((e >> 3) ^ (r & 15)) * 16) + (e & 7) * 2);
+  };
+#pragma unroll 4
+  for (int q = 0; q < R; ++q) {
+    const int r = r0 + q;
+    if (mw + r >= M) break;
+    uint16_t* dst = reinterpret_cast<uint16_t*>(C) + (int64_t)(mw + r) * N + nw;
+    const int o = (int)((reinterpret_cast<uintptr_t>(dst) >> 1) & 1);
+    const int e = 2 * lane + o;
+    const uint32_t lo = at(r, min(e, 127)), hi = at(r, min(e + 1, 127));
+    if (e + 1 < cnt) *reinterpret_cast<uint32_t*>(dst + e) = lo | (hi << 16);
+    else if (e < cnt) dst[e] = (uint16_t)lo;
+    if (o && lane == 0) dst[0] = at(r, 0);
+  }
+}
+
 // Epilogue of the 256 x 256 bf16 kernels: lane (fr, fg) holds row i * 16 + fr
 // and columns j * 16 + 4 fg .. +3 of the wave tile; stage it in this wave's
 // 16 KiB (256-byte rows, chunk c of row r at c ^ (r & 15)), then 16 lanes
@@ -212,40 +254,83 @@ __device__ __forceinline__ void q4_store_tile(const v4f (&acc)[4][8], __bf16* __
           make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  const bool vec_ok = (N % 8) == 0;
-  const int k = lane & 15;
+  q4_store_rows<64, 256>(wbuf, C, M, N, m0 + wm * 64, n0 + wn * 128, lane, 0);
+}
+
+// Split-K: the workgroup's f32 tile in register order, one contiguous 8 KiB
+// per (i, j), for q4_reduce_kernel.  The copies issued past the last slice
+// still write LDS, so they are waited for before the wave ends.
+__device__ __forceinline__ void q4_store_part(const v4f (&acc)[4][8], float* __restrict__ part) {
+  float4* p = reinterpret_cast<float4*>(part) + (size_t)blockIdx.x * (32 * 512) + threadIdx.x;
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int r = q * 4 + (lane >> 4);
-    const int m = m0 + wm * 64 + r;
-    const int n = n0 + wn * 128 + k * 8;
-    const uint4 v = *reinterpret_cast<const uint4*>(wbuf + r * 256 + ((k ^ (r & 15)) * 16));
-    if (m < M && n < N) {
-      __bf16* dst = C + (int64_t)m * N + n;
-      if (vec_ok) {
-        *reinterpret_cast<uint4*>(dst) = v;
-      } else {
-        const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
-          if (n + t < N) reinterpret_cast<uint16_t*>(dst)[t] = e[t];
-      }
+    for (int j = 0; j < 8; ++j)
+      p[(i * 8 + j) * 512] = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// Sum of the splits' partial tiles in split order, rounded once to bf16.  One
+// workgroup per 64 x 128 wave tile (8 per 256 x 256 tile): wave i sums the
+// fragments of rows 16 i .. +15 as the GEMM's lanes held them, and the bf16
+// rows leave through LDS as whole 256-byte pieces.
+__global__ __launch_bounds__(256) void q4_reduce_kernel(const float4* __restrict__ part, __bf16* __restrict__ C,
+                                                        int M, int N, int tiles_m, int tiles_n, int nsplit) {
+  __shared__ __attribute__((aligned(16))) uint8_t rows[64 * 256];
+  const int tile = blockIdx.x >> 3, w = blockIdx.x & 7;
+  int tmi, tni;
+  tile_of(tile, tiles_m, tiles_n, tmi, tni);
+  const int mw = tmi * 256 + (w >> 1) * 64, nw = tni * 256 + (w & 1) * 128;
+  if (mw >= M || nw >= N) return;
+  const int lane = threadIdx.x & 63, i = threadIdx.x >> 6, fr = lane & 15, fg = lane >> 4;
+  const size_t ntiles = (size_t)tiles_m * tiles_n;
+  const float4* p = part + ((size_t)tile * 32 + i * 8) * 512 + w * 64 + lane;
+  float4 t[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) t[j] = p[j * 512];
+  for (int s = 1; s < nsplit; ++s) {
+    p += ntiles * (32 * 512);
+    float4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = p[j * 512];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      t[j].x += v[j].x; t[j].y += v[j].y; t[j].z += v[j].z; t[j].w += v[j].w;
     }
   }
+  const int r = i * 16 + fr;
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    *reinterpret_cast<uint2*>(rows + r * 256 + (((j * 2 + (fg >> 1)) ^ (r & 15)) * 16) + (fg & 1) * 8) =
+        make_uint2(pack_bf16x2(t[j].x, t[j].y), pack_bf16x2(t[j].z, t[j].w));
+  __syncthreads();
+  q4_store_rows<16, 256>(rows, C, M, N, mw, nw, lane, 16 * i);
+}
+
+// The K slices of this workgroup's split: first slice and count (per slices
+// each, the last split takes what is left), and the tile slot within it.
+__device__ __forceinline__ int q4_split(int nks, int tiles_m, int tiles_n, int nsplit, int per, int& ks0, int& cnt) {
+  const int ntiles = tiles_m * tiles_n;
+  const int sp = nsplit > 1 ? (int)blockIdx.x / ntiles : 0;
+  ks0 = sp * per;
+  cnt = (sp == nsplit - 1 ? nks : ks0 + per) - ks0;
+  return (int)blockIdx.x - sp * ntiles;
 }
 
 __global__ __launch_bounds__(512, 1) void gemm_bf16_nt_q4_kernel(const __bf16* __restrict__ A,
                                                                  const __bf16* __restrict__ B,
                                                                  __bf16* __restrict__ C, int M, int N,
-                                                                 int K, int tiles_m, int tiles_n) {
+                                                                 int K, int tiles_m, int tiles_n, int nsplit,
+                                                                 int per, float* __restrict__ part) {
   Q4Ctx c;
   const int tid = threadIdx.x, lane = tid & 63;
   c.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  c.nks = K >> 5;
+  int ks0;
+  const int slot = q4_split(K >> 5, tiles_m, tiles_n, nsplit, per, ks0, c.nks);
   const int fr = lane & 15, fg = lane >> 4;
   const int wm = c.wave >> 1, wn = c.wave & 1;
   int tmi, tni;
-  tile_of(blockIdx.x, tiles_m, tiles_n, tmi, tni);
+  tile_of(slot, tiles_m, tiles_n, tmi, tni);
   const int m0 = tmi * 256, n0 = tni * 256;
   const uint32_t rowb = 2u * (uint32_t)K;
   c.ra = make_rsrc(A, (uint32_t)M * rowb);
@@ -255,8 +340,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_nt_q4_kernel(const __bf16* _
   // physical chunk L % 4, which holds logical chunk (L % 4) ^ ((L >> 3) & 3)
   const int lrow = c.wave * 64 + (lane >> 2);   // loader waves 0-3
   const uint32_t lch = (uint32_t)((lane & 3) ^ ((lane >> 3) & 3)) * 16u;
-  c.voa = (uint32_t)(m0 + lrow) * rowb + lch;
-  c.vob = (uint32_t)(n0 + lrow) * rowb + lch;
+  c.voa = (uint32_t)(m0 + lrow) * rowb + lch + (uint32_t)ks0 * 64u;
+  c.vob = (uint32_t)(n0 + lrow) * rowb + lch + (uint32_t)ks0 * 64u;
   // fragment: lane (fr, fg) reads logical chunk fg (k 8fg .. 8fg+7) of row
   // (wave tile row) + 16 t + fr, at physical chunk fg ^ ((fr >> 1) & 3)
   const uint32_t ch = (uint32_t)(fg ^ ((fr >> 1) & 3)) * 16u;
@@ -272,7 +357,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_nt_q4_kernel(const __bf16* _
   if (c.wave < 4) q4_main_loop<true, false>(c, acc);
   else q4_main_loop<false, false>(c, acc);
 
-  q4_store_tile(acc, C, M, N, m0, n0, wm, wn, c.wave, lane);
+  if (nsplit > 1) q4_store_part(acc, part);
+  else q4_store_tile(acc, C, M, N, m0, n0, wm, wn, c.wave, lane);
 }
 
 // C (M, N) = A^T B on contraction-major operands: A (Kc, M) and B (Kc, N)
@@ -287,15 +373,17 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_nt_q4_kernel(const __bf16* _
 __global__ __launch_bounds__(512, 1) void gemm_bf16_tn_q4_kernel(const __bf16* __restrict__ A,
                                                                  const __bf16* __restrict__ B,
                                                                  __bf16* __restrict__ C, int M, int N, int Kc,
-                                                                 int lda, int ldb, int tiles_m, int tiles_n) {
+                                                                 int lda, int ldb, int tiles_m, int tiles_n,
+                                                                 int nsplit, int per, float* __restrict__ part) {
   Q4Ctx c;
   const int tid = threadIdx.x, lane = tid & 63;
   c.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  c.nks = (Kc + 31) >> 5;
+  int ks0;
+  const int slot = q4_split((Kc + 31) >> 5, tiles_m, tiles_n, nsplit, per, ks0, c.nks);
   const int fr = lane & 15, fg = lane >> 4;
   const int wm = c.wave >> 1, wn = c.wave & 1;
   int tmi, tni;
-  tile_of(blockIdx.x, tiles_m, tiles_n, tmi, tni);
+  tile_of(slot, tiles_m, tiles_n, tmi, tni);
   const int m0 = tmi * 256, n0 = tni * 256;
   const uint32_t pa = 2u * (uint32_t)lda, pb = 2u * (uint32_t)ldb;
   c.ra = make_rsrc(A, (uint32_t)Kc * pa);
@@ -309,8 +397,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_tn_q4_kernel(const __bf16* _
   for (int p = 0; p < 4; ++p) {
     const uint32_t r = (uint32_t)(8 * c.wave + 2 * p + (lane >> 5));
     const uint32_t lc = (uint32_t)(lane & 31) ^ tn_swz(r);
-    c.voa4[p] = r * pa + (uint32_t)m0 * 2u + lc * 16u;
-    c.vob4[p] = r * pb + (uint32_t)n0 * 2u + lc * 16u;
+    c.voa4[p] = ((uint32_t)ks0 * 32u + r) * pa + (uint32_t)m0 * 2u + lc * 16u;
+    c.vob4[p] = ((uint32_t)ks0 * 32u + r) * pb + (uint32_t)n0 * 2u + lc * 16u;
   }
   // transposed reads: lane (fr, fg) reads row 8 fg + fr / 4 (+ 4) at columns
   // 4 (fr % 4) .. +3 of a subtile: chunk (fr % 4) / 2 of it, byte 8 (fr % 2)
@@ -333,7 +421,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_tn_q4_kernel(const __bf16* _
   if (c.wave < 4) q4_main_loop<true, true>(c, acc);
   else q4_main_loop<false, true>(c, acc);
 
-  q4_store_tile(acc, C, M, N, m0, n0, wm, wn, c.wave, lane);
+  if (nsplit > 1) q4_store_part(acc, part);
+  else q4_store_tile(acc, C, M, N, m0, n0, wm, wn, c.wave, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -382,16 +471,74 @@ __global__ __launch_bounds__(256) void pack_bf16_kernel(const void* __restrict__
   }
 }
 
-// Transposing pack of 16-byte-aligned bf16 rows (the common case, x_dtype bf16,
-// cols % 8 == 0): a 128 x 128 tile is loaded with 16-byte row loads into LDS
+// 8 consecutive bf16 at any even byte offset of a buffer: the 20 bytes from the
+// 4-byte boundary at or before it (raw buffer loads need no more than 4-byte
+// alignment, and what lies past the buffer reads zero), shifted into place.
+struct U8Load {
+  u32x4_t v;
+  uint32_t w;
+};
+__device__ __forceinline__ U8Load u8_load(const __amdgpu_buffer_rsrc_t& r, uint32_t off) {
+  const uint32_t o = off & ~3u;
+  return U8Load{__builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0), __builtin_amdgcn_raw_buffer_load_b32(r, o + 16u, 0, 0)};
+}
+__device__ __forceinline__ uint4 u8_value(const U8Load& l, uint32_t off) {
+  const uint32_t sh = (off & 2u) * 8u;   // 0 or 16 bits
+  return make_uint4(__builtin_amdgcn_alignbit(l.v.y, l.v.x, sh), __builtin_amdgcn_alignbit(l.v.z, l.v.y, sh),
+                    __builtin_amdgcn_alignbit(l.v.w, l.v.z, sh), __builtin_amdgcn_alignbit(l.w, l.v.w, sh));
+}
+// The first `n` of the 8 values, zeros after them.
+__device__ __forceinline__ uint4 u8_first(const uint4& v, int64_t n) {
+  uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] &= n >= 2 * i + 2 ? 0xFFFFFFFFu : n == 2 * i + 1 ? 0xFFFFu : 0u;
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+// Descriptor of bytes [x, x + bytes) from the 4-byte boundary at or before x,
+// and x's offset in it (0 or 2).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t u8_rsrc(const void* x, uint64_t bytes, uint32_t& base) {
+  base = (uint32_t)(reinterpret_cast<uintptr_t>(x) & 3u);
+  return make_rsrc(reinterpret_cast<const uint8_t*>(x) - base, (uint32_t)((bytes + base + 3u) & ~3ull));
+}
+
+// Row copy of bf16 rows at any even address to rows of `pitch` elements, zeros
+// past the row (pitch % 8 == 0, y 16-byte aligned): each thread four 16-byte
+// pieces of one output row, 256 pieces apart.  HBM-bound (2 bytes read, 2
+// written per element): with the 64 x 64 tiles of 2-byte accesses above,
+// 2048 x 50257 took 162 us (2.5 TB/s).
+constexpr int kRowPieces = 4;
+__global__ __launch_bounds__(256) void pack_bf16_rows_kernel(const uint16_t* __restrict__ x,
+                                                             uint16_t* __restrict__ y, int rows, int cols,
+                                                             int pitch) {
+  uint32_t base;
+  const __amdgpu_buffer_rsrc_t rx = u8_rsrc(x, (uint64_t)rows * (uint64_t)cols * 2u, base);
+  const int np = pitch >> 3;
+  for (int r = blockIdx.y; r < rows; r += gridDim.y) {
+    const int p0 = blockIdx.x * (256 * kRowPieces) + threadIdx.x;
+    const uint32_t ro = base + (uint32_t)r * (uint32_t)cols * 2u;
+    U8Load l[kRowPieces];
+#pragma unroll
+    for (int u = 0; u < kRowPieces; ++u) l[u] = u8_load(rx, ro + (uint32_t)(p0 + 256 * u) * 16u);
+#pragma unroll
+    for (int u = 0; u < kRowPieces; ++u) {
+      const int p = p0 + 256 * u;
+      if (p < np)
+        *reinterpret_cast<uint4*>(y + (int64_t)r * pitch + p * 8) = u8_first(u8_value(l[u], ro), (int64_t)cols - 8 * p);
+    }
+  }
+}
+
+// Transposing pack of bf16 rows (16-byte-aligned ones, or with UA rows at any
+// even address, such as an odd vocabulary's): a 128 x 128 tile is loaded with 16-byte row loads into LDS
 // (pitch 272 B); lane p of a wave reads the column pair 2p, 2p + 1 one 32-bit
 // word per row (conflict-free), the tile is re-staged in LDS as output rows
 // (pitch 264 B) and 16 lanes write each output row's 256 bytes, so every store
 // instruction covers four whole row segments.  (Writing each lane's 16-byte
 // pieces straight out left every output line to be assembled from sixteen
-// stores of four waves: 2.4 TB/s instead of 4.5 at 8192 x 50304.)  NT: non-
+// stores of four waves: 2.4 TB/s instead of 4.5 at 8192 x 50304.)  UA at
+// 2304 x 50257: 87 us; the 64 x 64 tiles took 164.  NT: non-
 // temporal stores, for outputs larger than the Infinity Cache.
-template <bool NT>
+template <bool NT, bool UA>
 __global__ __launch_bounds__(256) void pack_bf16_t128_kernel(const uint4* __restrict__ x,
                                                              uint16_t* __restrict__ y, int rows,
                                                              int cols, int pitch) {
@@ -401,12 +548,30 @@ __global__ __launch_bounds__(256) void pack_bf16_t128_kernel(const uint4* __rest
   const int ch = tid & 15, rr = tid >> 4;
   const int cchunks = cols >> 3;
   const bool ch_ok = (c0 >> 3) + ch < cchunks;
+  if constexpr (UA) {
+    // values past a row's end only reach output rows that are not stored, and
+    // rows past the last read zero
+    uint32_t base;
+    const __amdgpu_buffer_rsrc_t rx = u8_rsrc(x, (uint64_t)rows * (uint64_t)cols * 2u, base);
+    U8Load l[8];
+    uint32_t off[8];
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int r = r0 + rr + 16 * u;
-    const uint4 v = (ch_ok && r < rows) ? ldg_stream(x + (int64_t)r * cchunks + (c0 >> 3) + ch)
-                                        : make_uint4(0, 0, 0, 0);
-    *reinterpret_cast<uint4*>(&tile[(rr + 16 * u) * 68 + ch * 4]) = v;
+    for (int u = 0; u < 8; ++u) {
+      off[u] = base + ((uint32_t)(r0 + rr + 16 * u) * (uint32_t)cols + (uint32_t)(c0 + 8 * ch)) * 2u;
+      l[u] = u8_load(rx, off[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      *reinterpret_cast<uint4*>(&tile[(rr + 16 * u) * 68 + ch * 4]) =
+          u8_first(u8_value(l[u], off[u]), r0 + rr + 16 * u < rows ? 8 : 0);
+  } else {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int r = r0 + rr + 16 * u;
+      const uint4 v = (ch_ok && r < rows) ? ldg_stream(x + (int64_t)r * cchunks + (c0 >> 3) + ch)
+                                          : make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(&tile[(rr + 16 * u) * 68 + ch * 4]) = v;
+    }
   }
   __syncthreads();
   // lane p: input columns 2p, 2p + 1 (output rows), input rows 32g + 8c .. +7
@@ -452,16 +617,34 @@ int launch_pack_bf16(const void* x, int x_dtype, int64_t rows, int64_t cols, int
   const int64_t ext_r = transpose ? pitch : rows, ext_c = transpose ? cols : pitch;
   const dim3 grid((unsigned)((ext_c + 63) / 64), (unsigned)((ext_r + 63) / 64));
   const int r = (int)rows, c = (int)cols, p = (int)pitch;
-  if (transpose && x_dtype == TG_DTYPE_BF16 && cols % 8 == 0 && pitch % 8 == 0 &&
-      (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
+  // bf16 to 16-byte-aligned output rows: 16-byte stores, and 16-byte loads at
+  // any even address (32-bit buffer offsets, the last tile's overhang included);
+  // what is left (f32, an unaligned pitch or output) takes the 64 x 64 tiles
+  const bool wide = x_dtype == TG_DTYPE_BF16 && pitch % 8 == 0 && aligned(y, 16) && aligned(x, 2);
+  const bool off32 = ((uint64_t)rows + 128) * (uint64_t)cols * 2 + 512 < (1ull << 32);
+  const bool in16 = cols % 8 == 0 && aligned(x, 16);
+  if (transpose && wide && (in16 || off32)) {
     const dim3 g128((unsigned)((cols + 127) / 128), (unsigned)((pitch + 127) / 128));
     auto X = reinterpret_cast<const uint4*>(x);
     auto Y = reinterpret_cast<uint16_t*>(y);
-    if ((uint64_t)cols * (uint64_t)pitch * 2 > (256ull << 20))   // larger than the Infinity Cache
-      hipLaunchKernelGGL(pack_bf16_t128_kernel<true>, g128, dim3(256), 0, st, X, Y, r, c, p);
-    else
-      hipLaunchKernelGGL(pack_bf16_t128_kernel<false>, g128, dim3(256), 0, st, X, Y, r, c, p);
+    const bool nt = (uint64_t)cols * (uint64_t)pitch * 2 > (256ull << 20);   // larger than the Infinity Cache
+#define TG_PACK_T128(NT, UA) hipLaunchKernelGGL((pack_bf16_t128_kernel<NT, UA>), g128, dim3(256), 0, st, X, Y, r, c, p)
+    if (in16) {
+      if (nt) TG_PACK_T128(true, false);
+      else TG_PACK_T128(false, false);
+    } else {
+      if (nt) TG_PACK_T128(true, true);
+      else TG_PACK_T128(false, true);
+    }
+#undef TG_PACK_T128
     return check_launch("pack_bf16_t128");
+  }
+  if (!transpose && wide && off32) {
+    const dim3 gr((unsigned)((pitch / 8 + 256 * kRowPieces - 1) / (256 * kRowPieces)),
+                  (unsigned)(rows < 65535 ? rows : 65535));
+    hipLaunchKernelGGL(pack_bf16_rows_kernel, gr, dim3(256), 0, st, reinterpret_cast<const uint16_t*>(x),
+                       reinterpret_cast<uint16_t*>(y), r, c, p);
+    return check_launch("pack_bf16_rows");
   }
   if (x_dtype == TG_DTYPE_F32) {
     if (transpose) hipLaunchKernelGGL((pack_bf16_kernel<true, true>), grid, dim3(256), 0, st, x, y, r, c, p);
@@ -486,23 +669,67 @@ int launch_fill_zero_bf16(void* p, int64_t n, hipStream_t st) {
   return check_launch("fill_zero_bf16");
 }
 
-// C (M, N) = A^T B, A (Kc, M) pitch lda, B (Kc, N) pitch ldb (gemm_bf16_tn_q4_kernel)
+// Split of a contraction of nks 32-wide slices over workgroups, for outputs
+// whose 256 x 256 tiles leave CUs idle (a head's dX at 2048 x 2304: 72 tiles
+// on 256 CUs) or fill a last round badly.
+struct Q4Split {
+  int n, per;   // splits, slices per split
+};
+// The split with the least modelled time, in slices (~0.5 us each): rounds of
+// 256 workgroups times a split's slices plus 8 for its first round trip and
+// its tile's store, and for n > 1 the partial tiles written and read back
+// (8 bytes per output and split at ~5 TB/s) and the reduction's launch.
+// Measured: dX 2048 x 2304 over 50304, three splits on 216 CUs, 1219 us on 72
+// CUs -> 479 + 12 (reduction); dX 4096 x 2304 over 6912 (144 tiles, 176 us)
+// stays whole: three splits would move 226 MB of partial tiles.  A function of the shape alone: the workspace size and the launch agree on
+// every device, and the split (so the sum's order) is the same on every call.
+static Q4Split q4_split_of(int64_t M, int64_t N, int64_t Kc) {
+  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), nks = (Kc + 31) / 32;
+  Q4Split best{1, (int)nks};
+  double cost = 1e300;
+  for (int64_t n = 1; n <= 16; ++n) {
+    const int64_t per = (nks + n - 1) / n;
+    if (n > 1 && (per < 16 || (nks + per - 1) / per != n)) continue;
+    const double c = (double)((tiles * n + 255) / 256) * (double)(per + 8) +
+                     (n > 1 ? 6.0 + (double)(tiles * n) * (65536.0 * 8.0 / 2.5e6) : 0.0);
+    if (c < cost * 0.97) {
+      cost = c;
+      best = Q4Split{(int)n, (int)per};
+    }
+  }
+  return best;
+}
+static size_t q4_part_bytes(const Q4Split& sp, int64_t M, int64_t N) {
+  return sp.n > 1 ? (size_t)sp.n * (size_t)(((M + 255) / 256) * ((N + 255) / 256)) * 65536 * 4 : 0;
+}
+
+static int launch_q4_reduce(const float* part, __bf16* c, int64_t M, int64_t N, int tiles_m, int tiles_n, int n,
+                            hipStream_t st) {
+  hipLaunchKernelGGL(q4_reduce_kernel, dim3((unsigned)(tiles_m * tiles_n * 8)), dim3(256), 0, st,
+                     reinterpret_cast<const float4*>(part), c, (int)M, (int)N, tiles_m, tiles_n, n);
+  return check_launch("gemm_bf16_reduce");
+}
+
+// C (M, N) = A^T B, A (Kc, M) pitch lda, B (Kc, N) pitch ldb (gemm_bf16_tn_q4_kernel);
+// part: q4_part_bytes(sp, M, N) bytes, used when sp.n > 1
 int launch_gemm_bf16_tn(const __bf16* a, int64_t lda, const __bf16* b, int64_t ldb, __bf16* c, int64_t M,
-                        int64_t N, int64_t Kc, hipStream_t st) {
+                        int64_t N, int64_t Kc, const Q4Split& sp, float* part, hipStream_t st) {
   if (M == 0 || N == 0) return TG_OK;
   const int tiles_m = (int)((M + 255) / 256), tiles_n = (int)((N + 255) / 256);
-  hipLaunchKernelGGL(gemm_bf16_tn_q4_kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, st, a, b, c,
-                     (int)M, (int)N, (int)Kc, (int)lda, (int)ldb, tiles_m, tiles_n);
-  return check_launch("gemm_bf16_tn_256");
+  hipLaunchKernelGGL(gemm_bf16_tn_q4_kernel, dim3((unsigned)(tiles_m * tiles_n * sp.n)), dim3(512), 0, st, a, b, c,
+                     (int)M, (int)N, (int)Kc, (int)lda, (int)ldb, tiles_m, tiles_n, sp.n, sp.per, part);
+  TG_TRY(check_launch("gemm_bf16_tn_256"));
+  return sp.n > 1 ? launch_q4_reduce(part, c, M, N, tiles_m, tiles_n, sp.n, st) : TG_OK;
 }
 
 int launch_gemm_bf16(const __bf16* a, const __bf16* b, __bf16* c, int64_t M, int64_t N, int64_t K,
-                     hipStream_t st) {
+                     const Q4Split& sp, float* part, hipStream_t st) {
   if (M == 0 || N == 0) return TG_OK;
   const int tiles_m = (int)((M + 255) / 256), tiles_n = (int)((N + 255) / 256);
-  hipLaunchKernelGGL(gemm_bf16_nt_q4_kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, st,
-                     a, b, c, (int)M, (int)N, (int)K, tiles_m, tiles_n);
-  return check_launch("gemm_bf16_nt_256");
+  hipLaunchKernelGGL(gemm_bf16_nt_q4_kernel, dim3((unsigned)(tiles_m * tiles_n * sp.n)), dim3(512), 0, st,
+                     a, b, c, (int)M, (int)N, (int)K, tiles_m, tiles_n, sp.n, sp.per, part);
+  TG_TRY(check_launch("gemm_bf16_nt_256"));
+  return sp.n > 1 ? launch_q4_reduce(part, c, M, N, tiles_m, tiles_n, sp.n, st) : TG_OK;
 }
 
 }  // namespace tg
@@ -529,7 +756,8 @@ extern "C" int tg_gemm_bf16_nt(const void* a, const void* b, void* c, int64_t M,
   if (!a || !b || !c) return einval("gemm_bf16_nt: null pointer");
   if (!aligned(a, 16) || !aligned(b, 16)) return einval("gemm_bf16_nt: operands must be 16-byte aligned");
   return launch_gemm_bf16(reinterpret_cast<const __bf16*>(a), reinterpret_cast<const __bf16*>(b),
-                          reinterpret_cast<__bf16*>(c), M, N, K, as_stream(stream));
+                          reinterpret_cast<__bf16*>(c), M, N, K, Q4Split{1, (int)(K / 32)}, nullptr,
+                          as_stream(stream));
 }
 
 extern "C" int tg_pack_bf16(const void* x, int x_dtype, int64_t rows, int64_t cols, int transpose,
@@ -547,8 +775,11 @@ extern "C" int tg_pack_bf16(const void* x, int x_dtype, int64_t rows, int64_t co
 extern "C" size_t tg_block_scaled_matmul_bwd_bf16_workspace(int64_t M, int64_t N, int64_t K) {
   if (M < 0 || N < 0 || K < 0) return 0;
   const size_t np = (size_t)round64(N), mp = (size_t)round64(M);
+  const size_t px = q4_part_bytes(q4_split_of(M, K, (int64_t)np), M, K);
+  const size_t pw = q4_part_bytes(q4_split_of(K, N, M), K, N);
   return align256((size_t)M * np * 2) + align256((size_t)K * np * 2) +   // g, b packed along N
-         align256((size_t)K * mp * 2) + align256((size_t)N * mp * 2);    // a.T, g.T packed along M
+         align256((size_t)K * mp * 2) + align256((size_t)N * mp * 2) +   // a.T, g.T packed along M
+         (px > pw ? px : pw);                                            // split-K partial tiles of dX, then of dW
 }
 
 extern "C" int tg_block_scaled_matmul_bwd_bf16(const void* a, int a_dtype, const void* b,
@@ -577,7 +808,9 @@ extern "C" int tg_block_scaled_matmul_bwd_bf16(const void* a, int a_dtype, const
   __bf16* gp = reinterpret_cast<__bf16*>(p);   p += align256((size_t)M * np * 2);
   __bf16* bp = reinterpret_cast<__bf16*>(p);   p += align256((size_t)K * np * 2);
   __bf16* at = reinterpret_cast<__bf16*>(p);   p += align256((size_t)K * mp * 2);
-  __bf16* gt = reinterpret_cast<__bf16*>(p);
+  __bf16* gt = reinterpret_cast<__bf16*>(p);   p += align256((size_t)N * mp * 2);
+  float* part = reinterpret_cast<float*>(p);
+  const Q4Split spx = q4_split_of(M, K, np), spw = q4_split_of(K, N, M);
   // dX operands: used in place when already bf16, 64-aligned along N and 16-byte aligned
   const __bf16* gx = reinterpret_cast<const __bf16*>(g);
   const __bf16* bx = reinterpret_cast<const __bf16*>(b);
@@ -589,13 +822,15 @@ extern "C" int tg_block_scaled_matmul_bwd_bf16(const void* a, int a_dtype, const
     TG_TRY(launch_pack_bf16(b, b_dtype, K, N, 0, bp, np, st));
     bx = bp;
   }
-  TG_TRY(launch_gemm_bf16(gx, bx, reinterpret_cast<__bf16*>(da), M, K, np, st));   // fp8.py:95
-  if (a_dtype == TG_DTYPE_BF16 && g_dtype == TG_DTYPE_BF16 && K % 8 == 0 && N % 8 == 0 && aligned(a, 16) &&
-      aligned(g, 16))
-    // db = a.T . g read straight from a and g (contraction-major operands)
-    return launch_gemm_bf16_tn(reinterpret_cast<const __bf16*>(a), K, reinterpret_cast<const __bf16*>(g), N,
-                               reinterpret_cast<__bf16*>(db), K, N, M, st);                // fp8.py:96
+  TG_TRY(launch_gemm_bf16(gx, bx, reinterpret_cast<__bf16*>(da), M, K, np, spx, part, st));   // fp8.py:95
+  // db = a.T . g read straight from a and g (contraction-major operands): rows
+  // of a and g are read in 16-byte pieces, g's from its packed copy where its
+  // own rows are not aligned (an odd vocabulary)
+  const bool g_in_place = gx != gp && N % 8 == 0;
+  if (a_dtype == TG_DTYPE_BF16 && K % 8 == 0 && aligned(a, 16) && (gx == gp || g_in_place))
+    return launch_gemm_bf16_tn(reinterpret_cast<const __bf16*>(a), K, gx, gx == gp ? np : N,
+                               reinterpret_cast<__bf16*>(db), K, N, M, spw, part, st);         // fp8.py:96
   TG_TRY(launch_pack_bf16(a, a_dtype, M, K, 1, at, mp, st));
   TG_TRY(launch_pack_bf16(g, g_dtype, M, N, 1, gt, mp, st));
-  return launch_gemm_bf16(at, gt, reinterpret_cast<__bf16*>(db), K, N, mp, st);      // fp8.py:96
+  return launch_gemm_bf16(at, gt, reinterpret_cast<__bf16*>(db), K, N, mp, spw, part, st);      // fp8.py:96
 }
