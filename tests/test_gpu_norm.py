@@ -36,6 +36,21 @@ def test_rms_norm_pure_bit_exact(dev, shape):
     np.testing.assert_array_equal(bf16_bits(y), yo)
 
 
+# one past and exactly at 512 J elements for each J the kernels are built for
+# between the powers of two, and fewer and more rows than waves
+@pytest.mark.parametrize("rows,D", [(1, 1032), (9, 1536), (2, 2056), (700, 2560), (3, 2568), (4099, 3072), (5, 3080)])
+def test_rms_norm_chunk_count_edges(dev, rows, D):
+    rng = np.random.default_rng(rows + D)
+    x, g = _inputs(rng, (rows, D))
+    y = kernels.rms_norm(to_dev(x, dev), to_dev(g, dev), 1e-6)
+    assert np.array_equal(bf16_bits(y), norm_ref.rms_norm_pure(x, g, 1e-6))
+    if D % 128 == 0:
+        y, q, s = kernels.rms_norm_fp8(to_dev(x, dev), to_dev(g, dev), 1e-6)
+        yo, qo, so = norm_ref.rms_norm_fp8(x, g, 1e-6)
+        assert np.array_equal(bf16_bits(y), yo) and np.array_equal(u8(q), qo)
+        assert np.array_equal(f32_bits(s), so.view(np.uint32))
+
+
 @pytest.mark.parametrize("D", [8, 200, 1000])
 def test_rms_norm_dims_not_multiple_of_128(dev, D):
     rng = np.random.default_rng(D)

@@ -46,7 +46,9 @@ def _rne_equal(got_bits, ref):
 
 
 @pytest.mark.parametrize("shape", [(1, 128), (5, 768), (64, 2048), (3, 7, 256), (8, 1024, 2048),
-                                   (40, 520), (9, 1000), (33, 4096), (6, 3000)])
+                                   (40, 520), (9, 1000), (33, 4096), (6, 3000),
+                                   # the edges of 5 and 6 chunks per lane; rows around two per wave
+                                   (1, 2056), (2049, 2304), (17, 2560), (8, 2568), (9, 3072), (7, 3080)])
 def test_rms_norm_bwd_matches_oracle(dev, shape):
     rng = np.random.default_rng(sum(shape) + 7)
     x, g, dy = _inputs(rng, shape)

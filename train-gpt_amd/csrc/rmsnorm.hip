@@ -119,6 +119,10 @@ static int launch_rmsnorm(const void* x, const void* gamma, void* y, uint8_t* q,
   const float dimf = (float)dim;
   auto D = reinterpret_cast<const uint4*>(delta);
   auto XO = reinterpret_cast<uint4*>(xout);
+  // the chunks per lane that the width needs, not the next power of two: a lane
+  // without a chunk still costs its arithmetic and registers (fused with the
+  // quantizer, 3000 x 2304 9.2 us at J = 5 against 11.0 at 8; 4096 x 3072 12.9
+  // at 6 against 16.0)
 #define TG_NORM_CASE(JJ)                                                                        \
   if (jneed <= JJ) {                                                                             \
     if (nch == JJ * 64)                                                                          \
@@ -131,7 +135,10 @@ static int launch_rmsnorm(const void* x, const void* gamma, void* y, uint8_t* q,
   }
   TG_NORM_CASE(1)
   TG_NORM_CASE(2)
+  TG_NORM_CASE(3)
   TG_NORM_CASE(4)
+  TG_NORM_CASE(5)
+  TG_NORM_CASE(6)
   TG_NORM_CASE(8)
   TG_NORM_CASE(16)
   TG_NORM_CASE(32)
@@ -154,8 +161,11 @@ static int launch_rmsnorm(const void* x, const void* gamma, void* y, uint8_t* q,
 // order and the workgroup writes one partial row (slice-major, see
 // kNormBwdSlice), which rmsnorm_bwd_reduce_sm adds up in a fixed order.
 // Both orders are fixed, so dscale is the same on every run.
-// GREG: gamma in registers (J <= 4); PF: two rows' loads in flight per wave
-// (J <= 4).
+// GREG: gamma in registers; PF: two rows' loads in flight per wave.  Both up
+// to J = 6 (width 3072), where one wave per SIMD still holds a row twice over
+// without spilling (at 8 chunks, two rows spill: 57 -> 85 us at 8192 x 4096).
+// Widths 2049 .. 3072 have J = 5 or 6 of their own: 3000 x 2304 15.7 us against
+// 26.8 in the 8-chunk form (dx and the reduction), 16384 x 3072 56 against 89.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void unpack_bf16x8(const uint4& v, float (&f)[8]) {
   f[0] = bf16lo(v.x); f[1] = bf16hi(v.x); f[2] = bf16lo(v.y); f[3] = bf16hi(v.y);
@@ -183,7 +193,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const uint4* __restric
                                                           float* __restrict__ partial,
                                                           int64_t rows, int nch, float dimf,
                                                           float eps) {
-  constexpr bool GREG = J <= 4, PF = J <= 4;
+  constexpr bool GREG = J <= 6, PF = J <= 6;
   extern __shared__ float colsum[];   // nch * 8 floats
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t wave0 = (int64_t)blockIdx.x * 4 + wave;
@@ -543,9 +553,10 @@ __global__ __launch_bounds__(TG_NBWD_RTHREADS) void rmsnorm_bwd_reduce_sm(const 
 static int64_t norm_bwd_slices(int64_t dim) { return (dim + kNormBwdSlice - 1) / kNormBwdSlice; }
 
 static int64_t norm_bwd_grid(int64_t rows) {
-  // about four rows per wave, at most one workgroup per CU (256 partial rows
-  // at C2's 8192: 0.5 us less than 512 over both kernels, measured)
-  int64_t g = (rows + 15) / 16;
+  // two rows per wave (its two rows in flight), at most one workgroup per CU
+  // (256 partial rows at C2's 8192: 0.5 us less than 512 over both kernels,
+  // measured; at 100 x 768 two rows per wave 6.3 us, four 7.6)
+  int64_t g = (rows + 7) / 8;
   if (g > kNormBwdMaxGrid) g = kNormBwdMaxGrid;
   return g;
 }
@@ -564,6 +575,7 @@ static int launch_rmsnorm_bwd(const void* x, const void* gamma, const void* dy, 
   const size_t lds = (size_t)dim * 4;
   if (grid > 0) {
     bool launched = false;
+    // no J = 3: it takes the registers of J = 4 and ran 3% slower at 8192 x 1280
 #define TG_NORM_BWD_CASE(JJ)                                                                       \
     if (!launched && jneed <= JJ) {                                                                \
       if (nch == JJ * 64)                                                                          \
@@ -577,6 +589,8 @@ static int launch_rmsnorm_bwd(const void* x, const void* gamma, const void* dy, 
     TG_NORM_BWD_CASE(1)
     TG_NORM_BWD_CASE(2)
     TG_NORM_BWD_CASE(4)
+    TG_NORM_BWD_CASE(5)
+    TG_NORM_BWD_CASE(6)
     TG_NORM_BWD_CASE(8)
 #undef TG_NORM_BWD_CASE
     if (!launched) return einval("rms_norm_bwd: dim must be <= 4096");
