@@ -1,0 +1,114 @@
+"""GPU parity of the training step's FP8 linear (tg_linear_fwd, tg_linear_bwd,
+tg_linear_bwd_kept) on the extents and types that no block divides: bit for bit
+the general path's result, that is quantize_fp8 of zero-padded f32 copies and
+scaled_matmul (bf16 values widen to f32 exactly, so the bytes are the same)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import _tglib as L
+import fp8
+
+pytestmark = pytest.mark.gpu
+
+BF, F32 = torch.bfloat16, torch.float32
+
+
+def _pad(x, r, c):
+    x = x.float()
+    return F.pad(x, (0, c - x.shape[1], 0, r - x.shape[0])).contiguous()
+
+
+def _general(a, b, g):
+    """y, da, db (bf16) through padded copies, separate quantizers and row-major scales."""
+    (M, K), N = a.shape, b.shape[1]
+    mp, np_ = -(-M // 128) * 128, -(-N // 128) * 128
+    u8 = torch.uint8
+    ap, bp, gp = _pad(a, mp, K), _pad(b, K, np_), _pad(g, mp, np_)
+
+    def mm(x, y):            # x (R, C), y (S, C) quantized along C
+        return fp8.scaled_matmul(x[0].view(u8), x[1], y[0].view(u8), y[1])
+
+    def rows(x):
+        return fp8.quantize_fp8(x)
+
+    def cols(x):             # of x.T: the row quantizer on the transposed copy
+        return fp8.quantize_fp8(x.t().contiguous())
+
+    y = mm(rows(ap), cols(bp))[:M, :N]
+    da = mm(rows(gp), rows(bp))[:M]
+    db = mm(cols(ap), cols(gp))[:, :N]
+    return y, da, db
+
+
+def _inputs(dev, M, K, N, adt, bdt, seed=0, off=0):
+    gen = torch.Generator(device=dev).manual_seed(seed + M + K + N)
+
+    def make(r, c, std, dt):
+        buf = torch.zeros(r * c + off, dtype=dt, device=dev)
+        buf[off:] = (torch.randn(r * c, generator=gen, device=dev) * std).to(dt)
+        return buf[off:].reshape(r, c)
+
+    return make(M, K, 1.0, adt), make(K, N, 0.02, bdt), make(M, N, 1e-3, BF)
+
+
+# tile edges (128), one row or column past and short of them, odd widths, a
+# single row and a single column; every pairing of types
+@pytest.mark.parametrize("adt,bdt", [(BF, BF), (F32, F32), (F32, BF), (BF, F32)])
+@pytest.mark.parametrize("M,K,N", [(1, 128, 1), (127, 128, 130), (129, 384, 257), (300, 256, 128), (128, 128, 1001),
+                                   (256, 384, 256), (1000, 640, 520)])
+def test_linear_same_bits_as_general_path(dev, M, K, N, adt, bdt):
+    a, b, g = _inputs(dev, M, K, N, adt, bdt)
+    a.requires_grad_()
+    b.requires_grad_()
+    y = fp8.block_scaled_matmul(a, b)
+    da, db = torch.autograd.grad(y, (a, b), g)
+    assert (da.dtype, db.dtype) == (adt, bdt)
+    ry, rda, rdb = _general(a.detach(), b.detach(), g)
+    assert torch.equal(y, ry) and torch.equal(da, rda.to(adt)) and torch.equal(db, rdb.to(bdt))
+    assert torch.equal(fp8._fp8_forward(a.detach(), b.detach(), 128), ry)
+
+
+@pytest.mark.parametrize("M,N", [(130, 257), (128, 256)])
+def test_linear_bwd_from_element_aligned_operands(dev, M, N):
+    """tg_linear_bwd takes operands at any element address (odd bf16 offsets included)."""
+    a, b, g = _inputs(dev, M, 256, N, BF, BF, off=1)
+    da, db = fp8._linear_bwd(a, b, g)
+    _, rda, rdb = _general(a, b, g)
+    assert torch.equal(da, rda) and torch.equal(db, rdb)
+
+
+def test_linear_bwd_one_gradient(dev):
+    a, b, g = _inputs(dev, 200, 256, 136, BF, F32)
+    _, rda, rdb = _general(a, b, g)
+    M, K, N = 200, 256, 136
+    ws_bytes = L.lib().tg_linear_bwd_workspace(M, N, K)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    for want in ("da", "db"):
+        out = torch.full((M, K) if want == "da" else (K, N), 7.0, dtype=BF if want == "da" else F32, device=dev)
+        L.check(L.lib().tg_linear_bwd(L.ptr(a), 0, L.ptr(b), 1, L.ptr(g), 0, L.ptr(out) if want == "da" else None,
+                                      L.ptr(out) if want == "db" else None, M, N, K, L.ptr(ws), ws_bytes,
+                                      L.stream_of(a)))
+        assert torch.equal(out, rda if want == "da" else rdb.float())
+
+
+@pytest.mark.parametrize("dt", [BF, F32])
+def test_linear_non_finite_rows_ragged(dev, dt):
+    """A NaN and an infinity in a and g: the same positions as the general path."""
+    a, b, g = _inputs(dev, 140, 256, 200, dt, dt)
+    a[3, 5], a[139, 255], g[7, 199], g[131, 0] = float("nan"), float("inf"), float("nan"), float("-inf")
+    da, db = fp8._linear_bwd(a, b, g)
+    ry, rda, rdb = _general(a, b, g)
+    y = fp8._fp8_forward(a, b, 128)
+    for got, ref in ((y, ry), (da, rda), (db, rdb)):
+        ok = (got.float() == ref.float()) | (torch.isnan(got.float()) & torch.isnan(ref.float()))
+        assert bool(ok.all())
+
+
+@pytest.mark.parametrize("cols", [1, 3, 130, 2304])
+def test_quantize_cols_f32_same_bits_as_rows_of_the_transpose(dev, cols):
+    gen = torch.Generator(device=dev).manual_seed(cols)
+    x = torch.randn((384, cols), generator=gen, device=dev)
+    q, s = fp8.quantize_fp8(x, transpose=True)
+    rq, rs = fp8.quantize_fp8(x.t().contiguous())
+    assert torch.equal(q.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(s, rs)

@@ -71,6 +71,18 @@ SIGNATURES = {
     "tg_selftest_divide": (_int, [_vp, _vp]),
 }
 
+# include/tg_fp8_train.h: the FP8 linear of a training step
+TG_KEEP_A, TG_KEEP_B = 1, 2
+TRAIN_SIGNATURES = {
+    "tg_linear_kept_bytes": (_sz, [_i64, _i64, _i64, _int]),
+    "tg_linear_fwd_workspace": (_sz, [_i64, _i64, _i64]),
+    "tg_linear_fwd": (_int, [_vp, _int, _vp, _int, _vp, _i64, _i64, _i64, _int, _vp, _vp, _sz, _vp]),
+    "tg_linear_bwd_kept_workspace": (_sz, [_i64, _i64]),
+    "tg_linear_bwd_kept": (_int, [_vp, _int, _vp, _int, _vp, _int, _vp, _int, _i64, _i64, _i64, _vp, _sz, _vp]),
+    "tg_linear_bwd_workspace": (_sz, [_i64, _i64, _i64]),
+    "tg_linear_bwd": (_int, [_vp, _int, _vp, _int, _vp, _int, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp]),
+}
+
 _lib = None
 
 
@@ -83,7 +95,7 @@ def lib():
                 f"{LIB_PATH} is missing: build it with `python train-gpt_amd/build.py` "
                 "(the FP8 hot path has no non-HIP implementation)")
         L = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in (*SIGNATURES.items(), *TRAIN_SIGNATURES.items()):
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args

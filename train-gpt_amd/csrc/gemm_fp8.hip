@@ -59,7 +59,7 @@ template <int TM, int TN, int BNS, bool OUT_F32, bool SKM>
 __global__ __launch_bounds__(256, 2) void gemm_fp8_nt_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ SA, const uint8_t* __restrict__ B,
     const float* __restrict__ SB, void* __restrict__ C, int M, int N, int K, int tiles_m,
-    int tiles_n) {
+    int tiles_n, int round16) {
   constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
   constexpr int LA = BM / 32, LB = BN / 32;          // 16-byte chunks per thread per K block
   constexpr int STAGE = (BM + BN) * 8;               // uint4 per stage (128 B per row)
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fp8_nt_kernel(
         const int m = m0 + wm * TM * 16 + i * 16 + 4 * fg + r;
         if (m < M && n < N) {
           if (OUT_F32)
-            reinterpret_cast<float*>(C)[(int64_t)m * N + n] = acc[i][j][r];
+            reinterpret_cast<float*>(C)[(int64_t)m * N + n] = round16 ? round_bf16(acc[i][j][r]) : acc[i][j][r];
           else
             reinterpret_cast<__bf16*>(C)[(int64_t)m * N + n] = (__bf16)acc[i][j][r];
         }
@@ -337,7 +337,7 @@ template <int TN, int WN, int BNS, bool OUT_F32, bool SKM>
 __global__ __launch_bounds__(128 * WN, 1) void gemm_fp8_lat_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ SA, const uint8_t* __restrict__ B,
     const float* __restrict__ SB, void* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
-    int vec_out) {
+    int vec_out, int round16) {
   using Cfg = LatCfg<TN, WN>;
   constexpr int TM = Cfg::TM, BM = Cfg::BM, BN = Cfg::BN, NST = Cfg::NST, STAGE = Cfg::STAGE;
   constexpr int TNW = Cfg::TNW, W = Cfg::W;
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_fp8_lat_kernel(
         const int m = mw + i * 16 + 4 * fg + r;
         if (m < M && n < N) {
           if (OUT_F32)
-            reinterpret_cast<float*>(C)[(int64_t)m * N + n] = acc[i][j][r];
+            reinterpret_cast<float*>(C)[(int64_t)m * N + n] = round16 ? round_bf16(acc[i][j][r]) : acc[i][j][r];
           else
             reinterpret_cast<__bf16*>(C)[(int64_t)m * N + n] = (__bf16)acc[i][j][r];
         }
@@ -790,7 +790,7 @@ __device__ __forceinline__ void w32_block(const W32Ctx& c, v16f (&acc)[2][4], W3
 // order, so waiting for its own writes is enough.
 template <int S, bool OUT_F32>
 __device__ __forceinline__ void w32_store_tile(const v16f (&acc)[2][4], void* __restrict__ C, int M, int N,
-                                               int m0w, int n0w, int wave, int lane_in) {
+                                               int m0w, int n0w, int wave, int lane_in, int round16) {
   // an opaque copy of the lane index: the store addresses derive from it, so
   // the compiler cannot hoist them out of the tile loop (where they would
   // stay live across the K loop)
@@ -841,12 +841,15 @@ __device__ __forceinline__ void w32_store_tile(const v16f (&acc)[2][4], void* __
         const v16f& v = acc[i][j];
         if (OUT_F32) {
           float* dst = reinterpret_cast<float*>(C) + (int64_t)m * N + n;
+          float o[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) o[t] = round16 ? round_bf16(v[4 * q + t]) : v[4 * q + t];
           if (vec_ok && n + 4 <= N) {
-            *reinterpret_cast<float4*>(dst) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+            *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
           } else {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-              if (n + t < N) dst[t] = v[4 * q + t];
+              if (n + t < N) dst[t] = o[t];
           }
         } else {
           __bf16* dst = reinterpret_cast<__bf16*>(C) + (int64_t)m * N + n;
@@ -877,7 +880,7 @@ template <int BNS, bool OUT_F32, bool SKM>
 __global__ __launch_bounds__(512, 1) void gemm_fp8_nt_256_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ SA, const uint8_t* __restrict__ B,
     const float* __restrict__ SB, void* __restrict__ C, int M, int N, int K, int tiles_m,
-    int tiles_n) {
+    int tiles_n, int round16) {
   W32Ctx c;
   const int tid = threadIdx.x, lane = tid & 63;
   c.wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: keeps descriptors in SGPRs
@@ -1014,7 +1017,7 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_nt_256_kernel(
     prev.sa = 0.0f;
     prev.sb = make_float4(0.f, 0.f, 0.f, 0.f);
     w32_store_tile<S, OUT_F32>(acc, C, M, N, tm_cur * 256 + wm * 64, tn_cur * 256 + wn * 128, c.wave,
-                               lane);
+                               lane, round16);
     if (more) {
       // every wave is done with stage S before the next block's copies land there
       __syncthreads();
@@ -1036,7 +1039,7 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_nt_256_kernel(
 
 template <int BNS, bool OUT_F32, bool SKM>
 static int launch_gemm_256(const uint8_t* a_q, const float* a_s, const uint8_t* b_q,
-                           const float* b_s, void* c, int M, int N, int K, hipStream_t st) {
+                           const float* b_s, void* c, int M, int N, int K, int r16, hipStream_t st) {
   const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
   // one workgroup per CU (135 KiB of LDS each), looping over its tiles; the
   // grid stays a multiple of 8 so that a workgroup's slots share its XCD
@@ -1044,13 +1047,13 @@ static int launch_gemm_256(const uint8_t* a_q, const float* a_s, const uint8_t* 
   const int slots = device_cus() & ~7;
   const int grid = ntiles <= slots || slots == 0 ? ntiles : slots;
   hipLaunchKernelGGL((gemm_fp8_nt_256_kernel<BNS, OUT_F32, SKM>), dim3((unsigned)grid), dim3(512), 0, st,
-                     a_q, a_s, b_q, b_s, c, M, N, K, tiles_m, tiles_n);
+                     a_q, a_s, b_q, b_s, c, M, N, K, tiles_m, tiles_n, r16);
   return check_launch("gemm_fp8_nt_256");
 }
 
 template <int TM, int TN, int BNS, bool OUT_F32, bool SKM>
 static int launch_gemm_cfg(const uint8_t* a_q, const float* a_s, const uint8_t* b_q,
-                           const float* b_s, void* c, int M, int N, int K, hipStream_t st) {
+                           const float* b_s, void* c, int M, int N, int K, int r16, hipStream_t st) {
   constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const size_t lds = (size_t)2 * (BM + BN) * 128 + (size_t)2 * (BM + BN) * 4;
@@ -1071,7 +1074,7 @@ static int launch_gemm_cfg(const uint8_t* a_q, const float* a_s, const uint8_t* 
     return TG_EHIP;
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), lds, st, a_q, a_s, b_q,
-                     b_s, c, M, N, K, tiles_m, tiles_n);
+                     b_s, c, M, N, K, tiles_m, tiles_n, r16);
   return check_launch("gemm_fp8_nt");
 }
 
@@ -1080,7 +1083,7 @@ static int launch_gemm_cfg(const uint8_t* a_q, const float* a_s, const uint8_t* 
 #endif
 template <int TN, bool SKM>
 static int launch_gemm_lat(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, const float* b_s,
-                           int b_scale_bn, void* c, bool f32, int M, int N, int K, hipStream_t st) {
+                           int b_scale_bn, void* c, bool f32, int M, int N, int K, int r16, hipStream_t st) {
   constexpr int BM = 128, BN = 32 * TN, WN = TG_LAT_WN;
   if constexpr ((2 * TN) % WN != 0) {
     return einval("gemm_fp8_lat: tile width not split over the waves");
@@ -1090,7 +1093,7 @@ static int launch_gemm_lat(const uint8_t* a_q, const float* a_s, const uint8_t* 
   const dim3 grid((unsigned)(tiles_m * tiles_n));
 #define TG_LAT(BNS, F32)                                                                                    \
   hipLaunchKernelGGL((gemm_fp8_lat_kernel<TN, WN, BNS, F32, SKM>), grid, dim3(128 * WN), 0, st, a_q, a_s, b_q, \
-                     b_s, c, M, N, K, tiles_m, tiles_n, vec)
+                     b_s, c, M, N, K, tiles_m, tiles_n, vec, r16)
   if (b_scale_bn == 1) {
     if (f32) TG_LAT(1, true); else TG_LAT(1, false);
   } else {
@@ -1131,21 +1134,21 @@ static int lat_tile_n(int m, int n) {
 template <bool SKM>
 static int launch_gemm_fp8_layout(const uint8_t* a_q, const float* a_s, const uint8_t* b_q,
                                   const float* b_s, int b_scale_bn, void* c, bool f32, int m, int n,
-                                  int k, bool big, bool lat, hipStream_t st) {
+                                  int k, int r16, bool big, bool lat, hipStream_t st) {
   if (lat) {
     switch (lat_tile_n(m, n)) {
-      case 6: return launch_gemm_lat<6, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, st);
-      case 4: return launch_gemm_lat<4, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, st);
-      case 3: return launch_gemm_lat<3, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, st);
-      default: return launch_gemm_lat<2, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, st);
+      case 6: return launch_gemm_lat<6, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st);
+      case 4: return launch_gemm_lat<4, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st);
+      case 3: return launch_gemm_lat<3, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st);
+      default: return launch_gemm_lat<2, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st);
     }
   }
   if (big) {
     if (b_scale_bn == 1)
-      return f32 ? launch_gemm_256<1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
-                 : launch_gemm_256<1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
-    return f32 ? launch_gemm_256<128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
-               : launch_gemm_256<128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
+      return f32 ? launch_gemm_256<1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
+                 : launch_gemm_256<1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
+    return f32 ? launch_gemm_256<128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
+               : launch_gemm_256<128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
   }
   // 128 x 128 or 128 x 96 tiles, whichever leaves the busiest CU the fewer
   // outputs (tiles per CU, rounded up, times the tile's columns): C1's 2048 x
@@ -1157,16 +1160,16 @@ static int launch_gemm_fp8_layout(const uint8_t* a_q, const float* a_s, const ui
   const int64_t load96 = (tm * ((n + 95) / 96) + cus - 1) / cus * 96;
   if (load96 < load128) {
     if (b_scale_bn == 1)
-      return f32 ? launch_gemm_cfg<4, 3, 1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
-                 : launch_gemm_cfg<4, 3, 1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
-    return f32 ? launch_gemm_cfg<4, 3, 128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
-               : launch_gemm_cfg<4, 3, 128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
+      return f32 ? launch_gemm_cfg<4, 3, 1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
+                 : launch_gemm_cfg<4, 3, 1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
+    return f32 ? launch_gemm_cfg<4, 3, 128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
+               : launch_gemm_cfg<4, 3, 128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
   }
   if (b_scale_bn == 1)
-    return f32 ? launch_gemm_cfg<4, 4, 1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
-               : launch_gemm_cfg<4, 4, 1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
-  return f32 ? launch_gemm_cfg<4, 4, 128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
-             : launch_gemm_cfg<4, 4, 128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
+    return f32 ? launch_gemm_cfg<4, 4, 1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
+               : launch_gemm_cfg<4, 4, 1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
+  return f32 ? launch_gemm_cfg<4, 4, 128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
+             : launch_gemm_cfg<4, 4, 128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
 }
 
 int launch_gemm_fp8(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, const float* b_s,
@@ -1174,14 +1177,15 @@ int launch_gemm_fp8(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, co
                     hipStream_t st, bool skm) {
   if (M == 0 || N == 0) return TG_OK;
   const int m = (int)M, n = (int)N, k = (int)K;
-  const bool f32 = c_dtype == TG_DTYPE_F32;
+  const int r16 = c_dtype == kOutF32OfBf16;   // f32 output holding the bf16 result
+  const bool f32 = c_dtype == TG_DTYPE_F32 || r16;
   // 256 x 256 tiles once they fill the chip (>= 128 workgroups), else 128 x 128
   const bool fits32 = (uint64_t)M * (uint64_t)K < (1ull << 31) && (uint64_t)N * (uint64_t)K < (1ull << 31);
   const bool big = fits32 && ((M + 255) / 256) * ((N + 255) / 256) >= 128;
   // below that, the short-K ring kernel (32-bit buffer offsets, as the 256 kernel)
   const bool lat = fits32 && !big && lat_kernel_enabled();
-  return skm ? launch_gemm_fp8_layout<true>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, big, lat, st)
-             : launch_gemm_fp8_layout<false>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, big, lat, st);
+  return skm ? launch_gemm_fp8_layout<true>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, big, lat, st)
+             : launch_gemm_fp8_layout<false>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, big, lat, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -2197,13 +2201,14 @@ int tg::block_scaled_matmul_on(const void* a, const void* b, void* out, int64_t 
   uint8_t* qb = p;                 p += align256((size_t)N * K);
   float* sb = reinterpret_cast<float*>(p);
   // the composite's own workspace: scales K-block-major (the GEMM's cheaper scale reads)
+  // both quantizations in one launch (fp8.py:66, 68): one kernel's fixed cost
+  // instead of two's, which is most of the time at small shapes
   if (M % 128 == 0 && N % 128 == 0) {
-    // both quantizations in one launch (fp8.py:66, 68): one kernel's fixed
-    // cost instead of two's, which is most of the time at small shapes
     TG_TRY(launch_quant_rows_cols(a, M, K, qa, sa, b, N, qb, sb, st, true));
   } else {
-    TG_TRY(launch_quant_rows(a, TG_DTYPE_BF16, M, K, qa, sa, st, true));     // fp8.py:66
-    TG_TRY(launch_quant_cols(b, K, N, qb, sb, st, true));                     // fp8.py:68
+    const QuantTensor t[2] = {{a, TG_DTYPE_BF16, M, K, 1, qa, sa, nullptr, nullptr},
+                              {b, TG_DTYPE_BF16, K, N, 2, nullptr, nullptr, qb, sb}};
+    TG_TRY(launch_quant_tensors(t, 2, true, st));
   }
   return launch_gemm_fp8(qa, sa, qb, sb, 1, out, TG_DTYPE_BF16, M, N, K, st, true);   // fp8.py:70-78
 }

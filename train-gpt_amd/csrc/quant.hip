@@ -1,7 +1,6 @@
 // FP8 e4m3fn quantization kernels for gfx950 (HBM-bound byte work).
 //
 //   quant_rows_kernel   _quantize_to_fp8 along the last axis (fp8.py:39-47)
-//   quant_cols_kernel   _quantize_to_fp8 of x.T (fp8.py:68) for unaligned rows
 //   quant_dual_kernel   rows and / or x.T from one read, transposed through LDS
 //   quant_w128_kernel   128x128-tile weight quantization for the GEMV format
 //   selftest_cvt_kernel hardware e4m3fn convert vs the integer encoder
@@ -114,86 +113,6 @@ int launch_quant_rows_relu2(const void* x, int64_t rows, int64_t cols, uint8_t* 
   return check_launch("quant_rows_relu2");
 }
 
-// ---------------------------------------------------------------------------
-// Column quantization with transpose for rows that are not 16-byte aligned
-// (cols % 8 != 0; element loads, VEC = false).  Aligned rows take
-// quant_dual_kernel<false, ...> below.  Tile = 128 rows (one scale block of the
-// output) x 64 columns.  Load coalesced rows into LDS (row pitch 136 B), let
-// 4 lanes share each column (rows 16i + 4j + r for lane j, so a DPP quad holds
-// the block), stage the e4m3 bytes in a second LDS tile (pitch 144 B) and
-// store 32 contiguous bytes per lane.  Both pitches keep the column reads and
-// the 16-byte reads bank-conflict free for 32- and 64-bank LDS.
-// ---------------------------------------------------------------------------
-template <bool VEC>
-__global__ __launch_bounds__(256) void quant_cols_kernel(const uint16_t* __restrict__ x,
-                                                         int64_t rows, int64_t cols,
-                                                         uint8_t* __restrict__ qt,
-                                                         float* __restrict__ st, bool skm = false) {
-  __shared__ uint32_t tile[128 * 34];
-  __shared__ uint32_t tq[64 * 36];
-  const int tid = threadIdx.x;
-  const int64_t c0 = (int64_t)blockIdx.x * 64;
-  const int64_t r0 = (int64_t)blockIdx.y * 128;
-
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int id = tid + 256 * u;
-    const int row = id >> 3, ch = id & 7;
-    const int64_t col = c0 + ch * 8;
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (VEC) {
-      if (col < cols) v = ldg_stream(x + (r0 + row) * cols + col);
-    } else {
-      // rows are not 16-byte aligned when cols % 8 != 0: element loads
-      uint32_t e[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) e[k] = (col + k < cols) ? x[(r0 + row) * cols + col + k] : 0u;
-      v = make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16));
-    }
-    uint2* p = reinterpret_cast<uint2*>(&tile[row * 34 + ch * 4]);
-    p[0] = make_uint2(v.x, v.y);
-    p[1] = make_uint2(v.z, v.w);
-  }
-  __syncthreads();
-
-  const int n = tid >> 2, j = tid & 3;
-  const uint16_t* t16 = reinterpret_cast<const uint16_t*>(tile);
-  float f[32];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      f[i * 4 + r] = __uint_as_float(((uint32_t)t16[(16 * i + 4 * j + r) * 68 + n]) << 16);
-  uint32_t m = 0;
-#pragma unroll
-  for (int i = 0; i < 32; ++i) m = max(m, __float_as_uint(f[i]) & 0x7FFFFFFFu);
-  m = quad_max_u32(m);
-  const float sc = block_scale_bf16(m);
-  Divider d(sc);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    uint32_t w;
-    if (d.fast) {
-      w = e4m3x4(d.div(f[4 * i]), d.div(f[4 * i + 1]), d.div(f[4 * i + 2]), d.div(f[4 * i + 3]));
-    } else {
-      w = e4m3_nonfinite_scale(f[4 * i], sc) | (e4m3_nonfinite_scale(f[4 * i + 1], sc) << 8) |
-          (e4m3_nonfinite_scale(f[4 * i + 2], sc) << 16) |
-          (e4m3_nonfinite_scale(f[4 * i + 3], sc) << 24);
-    }
-    tq[n * 36 + 4 * i + j] = w;
-  }
-  const bool col_ok = (c0 + n) < cols;
-  if (j == 0 && col_ok) st[skm ? (int64_t)blockIdx.y * cols + c0 + n : (c0 + n) * (rows >> 7) + blockIdx.y] = sc;
-  __syncthreads();
-  if (col_ok) {
-    const uint4* src = reinterpret_cast<const uint4*>(&tq[n * 36 + 8 * j]);
-    uint4* dst = reinterpret_cast<uint4*>(qt + (c0 + n) * rows + r0 + 32 * j);
-    dst[0] = src[0];
-    dst[1] = src[1];
-  }
-}
-
-
 // The dual kernel (rows and / or x.T from one read) lives in quant_dual.h,
 // shared with the I/O-floor probe csrc/probe/quant_floor.hip.
 
@@ -213,11 +132,53 @@ int launch_quant_cols(const void* x, int64_t rows, int64_t cols, uint8_t* q_t, f
       hipLaunchKernelGGL((quant_dual_kernel<false, true>), grid, dim3(kDualThreads), 0, st, jobs);
     return check_launch("quant_cols");
   }
-  // rows not 16-byte aligned: the element-load kernel
-  const dim3 grid((unsigned)((cols + 63) / 64), (unsigned)(rows / 128));
-  hipLaunchKernelGGL(quant_cols_kernel<false>, grid, dim3(256), 0, st,
-                     reinterpret_cast<const uint16_t*>(x), rows, cols, q_t, s_t, skm);
-  return check_launch("quant_cols");
+  // rows not 16-byte aligned
+  const QuantTensor t{x, TG_DTYPE_BF16, rows, cols, 2, nullptr, nullptr, q_t, s_t};
+  return launch_quant_tensors(&t, 1, skm, st);
+}
+
+// The launch for tensors of any extents: all bf16 ones together (up to three,
+// as the backward's g, b and a), read the way the least aligned of them needs,
+// and all f32 ones together.  Whole-tile bf16 tensors take the plain kernel
+// when they are at most two.
+int launch_quant_tensors(const QuantTensor* t, int n, bool skm, hipStream_t st) {
+  for (int f32 = 0; f32 < 2; ++f32) {
+    DualJobs jobs{};
+    int cnt = 0, in = f32 ? kInF32 : kInVec;
+    int64_t total = 0;
+    for (int i = 0; i < n; ++i) {
+      if ((t[i].x_dtype == TG_DTYPE_F32) != (f32 != 0) || t[i].rows == 0 || t[i].cols == 0) continue;
+      if (cnt == 3) return einval("quantize: at most three tensors of a type");
+      if (t[i].cols > kQuantMaxCols) return einval("quantize: rows too wide");
+      TG_TRY(dual_job(jobs.job[cnt], "quantize", t[i].x, t[i].rows, t[i].cols, t[i].q, t[i].s, t[i].qt, t[i].st,
+                      total % 8 == 0, skm));
+      jobs.job[cnt].part = t[i].part;
+      if (!f32) {
+        const bool whole = t[i].rows % 128 == 0 && t[i].cols % 128 == 0 && aligned(t[i].x, 16);
+        const bool words = t[i].cols % 2 == 0 && aligned(t[i].x, 4);
+        const int need = whole ? kInVec : words ? kInBf16 : kInBf16Any;
+        in = need > in ? need : in;
+      }
+      const int64_t blocks = (int64_t)jobs.job[cnt].gx * jobs.job[cnt].gy;
+      total += blocks;
+      if (cnt == 0) jobs.nblk0 = (int)blocks;
+      if (cnt == 1) jobs.nblk1 = (int)blocks;
+      ++cnt;
+    }
+    if (cnt == 0) continue;
+    if (total > kDualMaxTiles) return einval("quantize: too many 128 x 128 tiles");
+    if (cnt == 3 && in == kInVec) in = kInBf16;
+    const dim3 grid((unsigned)total), block(kDualThreads);
+    if (in == kInVec) hipLaunchKernelGGL((quant_dual_kernel<true, false>), grid, block, 0, st, jobs);
+    else if (in == kInBf16)
+      hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInBf16>), grid, block, 0, st, jobs);
+    else if (in == kInBf16Any)
+      hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInBf16Any>), grid, block, 0, st, jobs);
+    else
+      hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInF32>), grid, block, 0, st, jobs);
+    TG_TRY(check_launch("quant_tensors"));
+  }
+  return TG_OK;
 }
 
 int launch_quant_dual(const void* x, int64_t rows, int64_t cols, uint8_t* q, float* s, uint8_t* q_t,
@@ -461,10 +422,16 @@ extern "C" int tg_quantize_cols(const void* x, int x_dtype, int64_t rows, int64_
   if (rows % block_k) return einval("quantize_cols: rows not divisible by block_k");
   if (rows * cols == 0) return TG_OK;
   if (!x || !q_t || !scales_t) return einval("quantize_cols: null pointer");
-  // f32 input (any block_k) and block_k != 128 take the general kernel
   if (block_k != 128 || x_dtype == TG_DTYPE_F32) {
     if (!aligned(x, x_dtype == TG_DTYPE_F32 ? 4 : 2) || !aligned(scales_t, 4))
       return einval("quantize_cols: x and scales_t must be aligned");
+    // f32 in 128-wide blocks: 128 x 128 tiles through LDS; 2304 x 2304 12 us (the
+    // general kernel's thread per column and block: 63 us)
+    if (block_k == 128 && aligned(q_t, 16) && cols <= kQuantMaxCols) {
+      const QuantTensor t{x, x_dtype, rows, cols, 2, nullptr, nullptr, q_t, scales_t};
+      return launch_quant_tensors(&t, 1, false, as_stream(stream));
+    }
+    // other block sizes: the general kernels
     return launch_quant_cols_gb(x, x_dtype == TG_DTYPE_F32, rows, cols, block_k, q_t, scales_t,
                                 as_stream(stream));
   }

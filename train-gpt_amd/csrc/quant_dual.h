@@ -31,6 +31,16 @@
 // ROWS = false gives the column quantization alone (tg_quantize_cols for
 // 16-byte-aligned rows); GUARD handles a last tile narrower than 128 columns.
 //
+// IN: how a tile is read.  kInVec: 16-byte loads of whole 16-byte-aligned rows,
+// every row of the tile inside x.  The others take any row and column count
+// (the FP8 backward on a token count or a width that no block divides): what
+// lies past x reads zero, which is the zero padding of a partial block, so q
+// rows are cp and q_t rows rp bytes wide (rows and cols rounded up to 128) and
+// no padded copy of x is made.  kInBf16: 16-byte-aligned bf16 rows; kInBf16Any:
+// bf16 rows at any even address (an odd width); kInF32: f32 rows, whose scale
+// and quotient are IEEE divides and whose raw tile takes 65 KiB of LDS (row
+// pitch 130 words: the column reads, two values at a time, touch all 64 banks).
+//
 // Scales.  With K-block-major scales (skm) a tile's 128 row scales are 512
 // contiguous bytes (s[tx * rows + r0 ..]) and so are its 128 column scales
 // (st[ty * cols + c0 ..]): they are gathered in LDS and written by two
@@ -59,6 +69,7 @@
 #pragma once
 #include <stdio.h>
 
+#include "gemm_tile.h"
 #include "row_ops.h"
 #include "tg_device.h"
 #include "tg_host.h"
@@ -75,11 +86,14 @@ struct DualJob {
   int gx, gy, xcd_blocks;
   int skm;   // scales K-block-major: s[kb * rows + row], st[kb * cols + col]
   int part;  // 0: rows and x.T; 1: rows only; 2: x.T only (with ROWS)
+  int64_t rp, cp;   // rows and cols rounded up to 128: the row pitches of q_t and q
 };
 struct DualJobs {
-  DualJob job[2];
-  int nblk0;   // tiles of job 0; gridDim.x - nblk0 are job 1's
+  DualJob job[3];
+  int nblk0, nblk1;   // tiles of jobs 0 and 1; the grid's others are job 2's (job 1's with nblk1 = 0)
 };
+
+constexpr int kInVec = 0, kInBf16 = 1, kInBf16Any = 2, kInF32 = 3;
 
 constexpr int kDualThreads = 512;
 
@@ -99,17 +113,21 @@ __device__ __forceinline__ uint32_t oct_max_u32(uint32_t v) {
 // are bit mixes of the loaded words instead of e4m3 bytes and scales, and
 // the amax reductions and divides are gone.  IO_SCALES = false also drops
 // the scale stores.
-template <bool ROWS, bool GUARD, bool IO = false, bool IO_SCALES = true>
+template <bool ROWS, bool GUARD, bool IO = false, bool IO_SCALES = true, int IN = kInVec>
 __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs) {
+  constexpr bool F32 = IN == kInF32, RAGGED = IN != kInVec;
+  static_assert(!RAGGED || (GUARD && !IO), "ragged tiles are guarded");
+  constexpr int kF32Pitch = 130;
   // the raw tile (row pitch 272 B); once every column is in registers the
   // same memory stages the transposed bytes (column pitch 128 B)
-  __shared__ uint32_t tile[128 * 68];
+  __shared__ __attribute__((aligned(16))) uint32_t tile[F32 ? 128 * kF32Pitch : 128 * 68];
   __shared__ float sgather[2][128];   // skm: the tile's row and column scales
   uint32_t* tq = tile;
   constexpr bool kScales = !IO || IO_SCALES;
   const int tid = threadIdx.x;
   const bool second = (int)blockIdx.x >= jobs.nblk0;
-  const DualJob& J = second ? jobs.job[1] : jobs.job[0];
+  const bool third = RAGGED && jobs.nblk1 > 0 && (int)blockIdx.x >= jobs.nblk0 + jobs.nblk1;
+  const DualJob& J = third ? jobs.job[2] : second ? jobs.job[1] : jobs.job[0];
   const uint4* __restrict__ x = J.x;
   const int64_t rows = J.rows, cols = J.cols;
   uint2* __restrict__ q = J.q;
@@ -117,7 +135,7 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
   uint8_t* __restrict__ qt = J.qt;
   float* __restrict__ st = J.st;
   const bool skm = J.skm != 0;
-  const int slot = (int)blockIdx.x - (second ? jobs.nblk0 : 0);
+  const int slot = (int)blockIdx.x - (second ? jobs.nblk0 : 0) - (third ? jobs.nblk1 : 0);
   int tx = slot % J.gx, ty = slot / J.gx;
   if (J.xcd_blocks) {
     // slot % 8 is the XCD: the host sets xcd_blocks only on a job that
@@ -130,20 +148,75 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
   }
   const int64_t c0 = (int64_t)tx * 128, r0 = (int64_t)ty * 128;
   const int ch = tid & 15, rr = tid >> 4;
-  const int64_t cchunks = cols >> 3;
+  // row pitches: q in 8-byte chunks, q_t in bytes
+  const int64_t cchunks = (RAGGED ? J.cp : cols) >> 3, rpitch = RAGGED ? J.rp : rows;
   const bool ch_ok = !GUARD || (c0 >> 3) + ch < cchunks;
   // the job's parts (workgroup-uniform)
   const bool do_rows = ROWS && J.part != 2, do_cols = J.part != 1;
-  uint4 v[4];
+  uint4 v[4], vh[F32 ? 4 : 1];   // F32: v[u], vh[u] the lane's 8 values
+  if constexpr (RAGGED) {
+    // a descriptor per four rows (one wave's), so 32-bit offsets do for any x;
+    // rows past the last fall outside it, columns past the last are cleared
+    constexpr uint32_t kE = F32 ? 4u : 2u;
+    const int64_t ncol = cols - (c0 + 8 * ch);   // of the lane's 8 columns, those inside x
+    uint32_t off[4], tail[IN == kInBf16Any ? 4 : 1];
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
-    v[u] = ch_ok ? ldg_stream(x + (r0 + rr + 32 * u) * cchunks + (c0 >> 3) + ch) : make_uint4(0, 0, 0, 0);
+    for (int u = 0; u < 4; ++u) {
+      const int64_t rb = r0 + 32 * u + 4 * __builtin_amdgcn_readfirstlane(tid >> 6);
+      const int64_t nr = rows - rb < 4 ? rows - rb : 4;
+      const uint8_t* xb = reinterpret_cast<const uint8_t*>(x) + (nr > 0 ? rb : 0) * cols * kE;
+      const uint32_t base = (uint32_t)(reinterpret_cast<uintptr_t>(xb) & 3u);
+      const uint32_t bytes = nr > 0 ? ((uint32_t)(nr * cols * kE) + base + 3u) & ~3u : 0u;
+      const __amdgpu_buffer_rsrc_t rx = make_rsrc(xb - base, bytes);
+      off[u] = base + ((uint32_t)(rr & 3) * (uint32_t)cols + (uint32_t)(c0 + 8 * ch)) * kE;
+      if ((rr & 3) >= nr || ncol <= 0) off[u] = 0x80000000u;   // past any descriptor here
+      const u32x4_t a = __builtin_amdgcn_raw_buffer_load_b128(rx, off[u] & ~3u, 0, 0);
+      v[u] = make_uint4(a.x, a.y, a.z, a.w);
+      if constexpr (F32) {
+        const u32x4_t b = __builtin_amdgcn_raw_buffer_load_b128(rx, off[u] + 16u, 0, 0);
+        vh[u] = make_uint4(b.x, b.y, b.z, b.w);
+      }
+      if constexpr (IN == kInBf16Any) tail[u] = __builtin_amdgcn_raw_buffer_load_b32(rx, (off[u] & ~3u) + 16u, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      uint32_t w[8] = {v[u].x, v[u].y, v[u].z, v[u].w};
+      if constexpr (F32) {
+        w[4] = vh[u].x; w[5] = vh[u].y; w[6] = vh[u].z; w[7] = vh[u].w;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = i < ncol ? w[i] : 0u;
+        vh[u] = make_uint4(w[4], w[5], w[6], w[7]);
+      } else {
+        if constexpr (IN == kInBf16Any) {
+          const uint32_t sh = (off[u] & 2u) * 8u;
+          w[0] = __builtin_amdgcn_alignbit(w[1], w[0], sh);
+          w[1] = __builtin_amdgcn_alignbit(w[2], w[1], sh);
+          w[2] = __builtin_amdgcn_alignbit(w[3], w[2], sh);
+          w[3] = __builtin_amdgcn_alignbit(tail[u], w[3], sh);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] &= 2 * i + 2 <= ncol ? 0xFFFFFFFFu : 2 * i + 1 == ncol ? 0xFFFFu : 0u;
+      }
+      v[u] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      v[u] = ch_ok ? ldg_stream(x + (r0 + rr + 32 * u) * cchunks + (c0 >> 3) + ch) : make_uint4(0, 0, 0, 0);
+  }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int row = rr + 32 * u;
+    const bool row_in = !RAGGED || r0 + row < rows;
     if (do_rows) {
       float sc;
-      if constexpr (IO) {
+      if constexpr (F32) {
+        const float f[8] = {__uint_as_float(v[u].x), __uint_as_float(v[u].y), __uint_as_float(v[u].z),
+                            __uint_as_float(v[u].w), __uint_as_float(vh[u].x), __uint_as_float(vh[u].y),
+                            __uint_as_float(vh[u].z), __uint_as_float(vh[u].w)};
+        sc = block_scale(row16_max_u32(absmax8(f)));
+        if (row_in) q[(r0 + row) * cchunks + (c0 >> 3) + ch] = quant8<false>(f, sc);
+      } else if constexpr (IO) {
         sc = __uint_as_float(v[u].x);
         q[(r0 + row) * cchunks + (c0 >> 3) + ch] = make_uint2(v[u].x ^ v[u].z, v[u].y ^ v[u].w);
       } else {
@@ -151,19 +224,29 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
         f[0] = bf16lo(v[u].x); f[1] = bf16hi(v[u].x); f[2] = bf16lo(v[u].y); f[3] = bf16hi(v[u].y);
         f[4] = bf16lo(v[u].z); f[5] = bf16hi(v[u].z); f[6] = bf16lo(v[u].w); f[7] = bf16hi(v[u].w);
         sc = block_scale_bf16(row16_max_u32(absmax8(f)));
-        q[(r0 + row) * cchunks + (c0 >> 3) + ch] = quant8<true>(f, sc);
+        if (row_in) q[(r0 + row) * cchunks + (c0 >> 3) + ch] = quant8<true>(f, sc);
       }
       if (kScales && ch == 0) {
         if (skm) sgather[0][row] = sc;
-        else s[(r0 + row) * (cols >> 7) + tx] = sc;
+        else if (row_in) s[(r0 + row) * (cchunks >> 4) + tx] = sc;
       }
     }
-    if (do_cols) *reinterpret_cast<uint4*>(&tile[row * 68 + ((ch * 4) ^ (4 * ((row >> 3) & 3)))]) = v[u];
+    if (do_cols) {
+      if constexpr (F32) {
+        uint2* p = reinterpret_cast<uint2*>(&tile[row * kF32Pitch + ch * 8]);
+        p[0] = make_uint2(v[u].x, v[u].y);
+        p[1] = make_uint2(v[u].z, v[u].w);
+        p[2] = make_uint2(vh[u].x, vh[u].y);
+        p[3] = make_uint2(vh[u].z, vh[u].w);
+      } else {
+        *reinterpret_cast<uint4*>(&tile[row * 68 + ((ch * 4) ^ (4 * ((row >> 3) & 3)))]) = v[u];
+      }
+    }
   }
   const bool rows_gathered = kScales && do_rows && skm;
   if (!do_cols && !rows_gathered) return;
   __syncthreads();
-  if (rows_gathered && tid < 128) s[(int64_t)tx * rows + r0 + tid] = sgather[0][tid];
+  if (rows_gathered && tid < 128 && (!RAGGED || r0 + tid < rows)) s[(int64_t)tx * rows + r0 + tid] = sgather[0][tid];
   if (!do_cols) return;
 
   // columns: the 8 lanes tid >> 3 own the column pair 2c, 2c + 1 (one 32-bit
@@ -174,7 +257,7 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
   auto put_scale = [&](float sc, int n) {
     if (kScales && j == 0 && (!GUARD || c0 + n < cols)) {
       if (skm) sgather[1][n] = sc;
-      else st[(c0 + n) * (rows >> 7) + ty] = sc;
+      else st[(c0 + n) * (rpitch >> 7) + ty] = sc;
     }
   };
   // word g = 8t + j of column n: chunk (g >> 2) = 2t + (j >> 2), word j & 3 of it
@@ -199,9 +282,15 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const uint32_t w = tile[(32 * t + 4 * j + r) * 68 + cpw];
-        f0[t * 4 + r] = __uint_as_float(w << 16);
-        f1[t * 4 + r] = __uint_as_float(w & 0xFFFF0000u);
+        if constexpr (F32) {
+          const uint2 w = *reinterpret_cast<const uint2*>(&tile[(32 * t + 4 * j + r) * kF32Pitch + 2 * cp]);
+          f0[t * 4 + r] = __uint_as_float(w.x);
+          f1[t * 4 + r] = __uint_as_float(w.y);
+        } else {
+          const uint32_t w = tile[(32 * t + 4 * j + r) * 68 + cpw];
+          f0[t * 4 + r] = __uint_as_float(w << 16);
+          f1[t * 4 + r] = __uint_as_float(w & 0xFFFF0000u);
+        }
       }
     uint32_t m0 = 0, m1 = 0;
 #pragma unroll
@@ -209,8 +298,9 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
       m0 = max(m0, __float_as_uint(f0[i]) & 0x7FFFFFFFu);
       m1 = max(m1, __float_as_uint(f1[i]) & 0x7FFFFFFFu);
     }
-    const float sc0 = block_scale_bf16(oct_max_u32(m0));
-    const float sc1 = block_scale_bf16(oct_max_u32(m1));
+    const uint32_t a0 = oct_max_u32(m0), a1 = oct_max_u32(m1);
+    const float sc0 = F32 ? block_scale(a0) : block_scale_bf16(a0);
+    const float sc1 = F32 ? block_scale(a1) : block_scale_bf16(a1);
     __syncthreads();   // every lane has read its columns: the tile becomes tq
     auto col_words = [&](const float (&f)[16], float sc, int n) {
       Divider d(sc);
@@ -218,7 +308,8 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
       for (int t = 0; t < 4; ++t) {
         uint32_t w;
         if (d.fast) {
-          w = e4m3x4(d.div(f[4 * t]), d.div(f[4 * t + 1]), d.div(f[4 * t + 2]), d.div(f[4 * t + 3]));
+          w = F32 ? e4m3x4(f[4 * t] / sc, f[4 * t + 1] / sc, f[4 * t + 2] / sc, f[4 * t + 3] / sc)
+                  : e4m3x4(d.div(f[4 * t]), d.div(f[4 * t + 1]), d.div(f[4 * t + 2]), d.div(f[4 * t + 3]));
         } else {
           w = e4m3_nonfinite_scale(f[4 * t], sc) | (e4m3_nonfinite_scale(f[4 * t + 1], sc) << 8) |
               (e4m3_nonfinite_scale(f[4 * t + 2], sc) << 16) |
@@ -243,7 +334,7 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
     const int n = (tid >> 3) + 64 * p, k = tid & 7;
     if (GUARD && c0 + n >= cols) continue;
     const uint4 val = *reinterpret_cast<const uint4*>(&tq[dual_tq_at(n, k)]);
-    *(reinterpret_cast<uint4*>(qt + (c0 + n) * rows + r0) + k) = val;
+    *(reinterpret_cast<uint4*>(qt + (c0 + n) * rpitch + r0) + k) = val;
   }
   if (kScales && skm && tid >= 128 && tid < 256 && (!GUARD || c0 + tid - 128 < cols))
     st[(int64_t)ty * cols + c0 + tid - 128] = sgather[1][tid - 128];
@@ -256,7 +347,7 @@ constexpr int64_t kDualMaxTiles = int64_t(1) << 23;   // slots fit one 1-D grid 
 
 inline int dual_job(DualJob& j, const char* who, const void* x, int64_t rows, int64_t cols, uint8_t* q,
                     float* s, uint8_t* q_t, float* s_t, bool xcd_ok, bool skm) {
-  const int64_t gx = (cols + 127) / 128, gy = rows / 128;
+  const int64_t gx = (cols + 127) / 128, gy = (rows + 127) / 128;
   if (gx * gy > kDualMaxTiles) {
     char msg[160];
     snprintf(msg, sizeof msg, "%s: (rows / 128) x (cols / 128) must be <= %lld tiles", who,
@@ -275,6 +366,8 @@ inline int dual_job(DualJob& j, const char* who, const void* x, int64_t rows, in
   j.xcd_blocks = xcd_ok && gx % 32 == 0 && gy % 16 == 0 && (gx * gy / 8) % 512 == 0;
   j.skm = skm ? 1 : 0;
   j.part = 0;
+  j.rp = gy * 128;
+  j.cp = gx * 128;
   return TG_OK;
 }
 

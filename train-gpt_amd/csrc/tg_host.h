@@ -68,6 +68,27 @@ int launch_quant_rows_cols(const void* a, int64_t M, int64_t K, uint8_t* qa, flo
 int launch_quant_dual_pair(const void* x0, int64_t rows0, int64_t cols0, uint8_t* q0, float* s0,
                            uint8_t* qt0, float* st0, const void* x1, int64_t rows1, int64_t cols1,
                            uint8_t* q1, float* s1, uint8_t* qt1, float* st1, hipStream_t st, bool skm = false);
+// One tensor of a quantization launch: x (rows, cols) bf16 or f32, any extents
+// and any alignment of its element; what lies past x is zero padding up to
+// whole 128-wide blocks.  Rows along cols: q (rows, round128(cols)) and s, for
+// parts 0 and 1; x.T along rows: qt (cols, round128(rows)) and st, for parts 0
+// and 2.
+struct QuantTensor {
+  const void* x;
+  int x_dtype;
+  int64_t rows, cols;
+  int part;
+  uint8_t* q;
+  float* s;
+  uint8_t* qt;
+  float* st;
+};
+constexpr int64_t kQuantMaxCols = int64_t(1) << 26;   // four rows of f32 stay below 2^31 bytes
+int launch_quant_tensors(const QuantTensor* t, int n, bool skm, hipStream_t st);
+
+// c_dtype of launch_gemm_fp8 besides TG_DTYPE_*: the bf16 result widened to f32
+// (fp8.py:95-96's cast of a bf16 gradient to an f32 operand's dtype).
+constexpr int kOutF32OfBf16 = 0x100;
 int launch_gemm_fp8(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, const float* b_s,
                     int b_scale_bn, void* c, int c_dtype, int64_t M, int64_t N, int64_t K,
                     hipStream_t st, bool skm = false);

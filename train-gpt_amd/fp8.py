@@ -17,12 +17,14 @@ Backward modes (``BACKWARD_MODE``):
     GEMMs of the un-quantized operands.
 
 Residuals.  In "fp8" mode with bf16 operands whose M and N divide by
-block_k, the forward quantizes a and b once each in both directions
-(tg_quantize_dual: a along K and a.T along M; b.T along K and b along N) and
-keeps the FP8 forms the backward needs (a.T, b) instead of a and b.  The
+block_k, the forward quantizes a and b once each in both directions (a along
+K and a.T along M; b.T along K and b along N) and keeps the FP8 forms the
+backward needs (a.T, b; one buffer, tg_linear_fwd) instead of a and b.  The
 bytes are those the backward would compute from a and b, so the gradients
 are the same bits; each operand is read once instead of twice and the saved
-residuals take ~half the memory.
+residuals take ~half the memory.  Other operands (a ragged token count or
+width, f32) are saved themselves, as in the reference, and quantized by the
+backward (tg_linear_bwd).
 
 Additive entry points (no reference counterpart): ``quantize_fp8`` (row or
 transposed), ``quantize_weight`` (pre-quantized weight format) and
@@ -217,18 +219,6 @@ def _quantize_dual_pair_km(x0: torch.Tensor, x1: torch.Tensor, block_k: int):
     return outs
 
 
-def _scaled_matmul_km(a_q, a_s_km, b_q, b_s_km):
-    """scaled_matmul on K-block-major scales (tg_gemm_fp8_nt_km), bf16 out; the
-    same bits as scaled_matmul on the transposed scales."""
-    M, K = a_q.shape
-    N = b_q.shape[0]
-    c = torch.empty((M, N), dtype=torch.bfloat16, device=a_q.device)
-    _L.check(_L.lib().tg_gemm_fp8_nt_km(_L.ptr(a_q), _L.ptr(a_s_km), _L.ptr(b_q), _L.ptr(b_s_km), 1,
-                                        _L.ptr(c), _L.TG_DTYPE_BF16, M, N, K, DEFAULT_BLOCK_K,
-                                        _L.stream_of(a_q)))
-    return c
-
-
 def scaled_matmul(a_q, a_s, b_q, b_s, b_scale_bn: int = 1, out_dtype=torch.bfloat16):
     """The scaled GEMM of fp8.py:70-76 on already-quantized operands ("NT"):
     a_q (M, K), b_q (N, K) e4m3fn; a_s (M, K/bk), b_s (N or ceil(N/128), K/bk)
@@ -259,11 +249,12 @@ def _fp8_forward(a: torch.Tensor, b: torch.Tensor, block_k: int) -> torch.Tensor
     leading, K, N = _validate(a, b, block_k)
     _L.require_gpu(a, b)
     _check_block_k(block_k)
-    a_2d = a.reshape(-1, K)
+    a_2d = a.reshape(-1, K).contiguous()
+    b_c = b.contiguous()
     M = a_2d.shape[0]
+    if block_k == TUNED_BLOCK_K and a.dtype in _KERNEL_DTYPES and b.dtype in _KERNEL_DTYPES:
+        return _linear_fwd(a_2d, b_c, 0)[0].reshape(*leading, N)
     if a.dtype == torch.bfloat16 and b.dtype == torch.bfloat16:
-        a_2d = a_2d.contiguous()
-        b_c = b.contiguous()
         out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
         ws_bytes = _L.lib().tg_block_scaled_matmul_workspace(M, N, K, block_k)
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=a.device)
@@ -271,9 +262,62 @@ def _fp8_forward(a: torch.Tensor, b: torch.Tensor, block_k: int) -> torch.Tensor
                                                  block_k, _L.ptr(ws), ws_bytes, _L.stream_of(a_2d)))
         return out.reshape(*leading, N)
     a_q, a_s = quantize_fp8(a_2d, block_k)                         # fp8.py:66
-    b_q, b_s = quantize_fp8(b, block_k, transpose=True)            # fp8.py:68
+    b_q, b_s = quantize_fp8(b_c, block_k, transpose=True)          # fp8.py:68
     out = scaled_matmul(a_q.view(torch.uint8), a_s, b_q.view(torch.uint8), b_s)   # fp8.py:70-78
     return out.reshape(*leading, N)
+
+
+_KERNEL_DTYPES = (torch.bfloat16, torch.float32)
+
+
+def _linear_fwd(a_2d, b, keep):
+    """tg_linear_fwd on contiguous a (M, K) and b (K, N), bf16 or f32: out (M, N)
+    bf16 and, with keep (_L.TG_KEEP_*), the buffer of the backward's FP8 operands."""
+    M, K = a_2d.shape
+    N = b.shape[1]
+    L, dev, u8 = _L.lib(), a_2d.device, torch.uint8
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    kept = torch.empty(L.tg_linear_kept_bytes(M, N, K, keep), dtype=u8, device=dev) if keep else None
+    ws_bytes = L.tg_linear_fwd_workspace(M, N, K)
+    ws = torch.empty(ws_bytes, dtype=u8, device=dev)
+    _L.check(L.tg_linear_fwd(_L.ptr(a_2d), _L.dtype_code(a_2d), _L.ptr(b), _L.dtype_code(b), _L.ptr(out), M, N, K,
+                             keep, _L.ptr(kept) if keep else None, _L.ptr(ws), ws_bytes, _L.stream_of(a_2d)))
+    return out, kept
+
+
+def _linear_bwd_kept(kept, keep, g_2d, K, da_dtype, db_dtype):
+    """(da or None, db or None) from a forward's kept operands and contiguous g (M, N)."""
+    M, N = g_2d.shape
+    L, dev = _L.lib(), g_2d.device
+    da = torch.empty((M, K), dtype=da_dtype, device=dev) if keep & _L.TG_KEEP_B else None
+    db = torch.empty((K, N), dtype=db_dtype, device=dev) if keep & _L.TG_KEEP_A else None
+    ws_bytes = L.tg_linear_bwd_kept_workspace(M, N)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    _L.check(L.tg_linear_bwd_kept(
+        _L.ptr(kept), keep, _L.ptr(g_2d), _L.dtype_code(g_2d),
+        _L.ptr(da) if da is not None else None, _L.dtype_code(da) if da is not None else 0,
+        _L.ptr(db) if db is not None else None, _L.dtype_code(db) if db is not None else 0, M, N, K,
+        _L.ptr(ws), ws_bytes, _L.stream_of(g_2d)))
+    return da, db
+
+
+def _linear_bwd(a_2d, b, g_2d):
+    """(da, db) in a's and b's dtypes from contiguous bf16 or f32 operands, any M and N."""
+    M, K = a_2d.shape
+    N = b.shape[1]
+    L, dev = _L.lib(), a_2d.device
+    da, db = torch.empty_like(a_2d), torch.empty_like(b)
+    ws_bytes = L.tg_linear_bwd_workspace(M, N, K)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    _L.check(L.tg_linear_bwd(_L.ptr(a_2d), _L.dtype_code(a_2d), _L.ptr(b), _L.dtype_code(b), _L.ptr(g_2d),
+                             _L.dtype_code(g_2d), _L.ptr(da), _L.ptr(db), M, N, K, _L.ptr(ws), ws_bytes,
+                             _L.stream_of(a_2d)))
+    return da, db
+
+
+def _kernel_dtype(x):
+    """x itself when the kernels take its dtype, else its f32 values."""
+    return x if x.dtype in _KERNEL_DTYPES else x.to(torch.float32)
 
 
 def _fp8_forward_with_residuals(a, b, block_k):
@@ -310,6 +354,10 @@ def _fp8_backward(block_k, residuals, g):
         # empty contraction or empty result: the reference's dots give zeros
         return (torch.zeros(a.shape, dtype=a.dtype, device=a.device),
                 torch.zeros(b.shape, dtype=b.dtype, device=b.device))
+    if block_k == TUNED_BLOCK_K:
+        da, db = _linear_bwd(_kernel_dtype(a_2d).contiguous(), _kernel_dtype(b).contiguous(),
+                             _kernel_dtype(g_2d).contiguous())
+        return da.reshape(*leading, K).to(a.dtype), db.to(b.dtype)
     Mp, Np = -(-M // block_k) * block_k, -(-N // block_k) * block_k
     if (Mp, Np) != (M, N):
         a_p = a_2d.new_zeros((Mp, K))
@@ -332,11 +380,8 @@ def _fp8_backward(block_k, residuals, g):
             _L.ptr(ws), ws_bytes, _L.stream_of(a_2d)))
     else:
         u8 = torch.uint8
-        if g_2d.dtype == bf and block_k == TUNED_BLOCK_K:
-            qg, sg, qgt, sgt = quantize_fp8_dual(g_2d, block_k)    # g along N and g.T along M
-        else:
-            qg, sg = quantize_fp8(g_2d, block_k)                   # g along N
-            qgt, sgt = quantize_fp8(g_2d, block_k, transpose=True)  # g.T along M
+        qg, sg = quantize_fp8(g_2d, block_k)                       # g along N
+        qgt, sgt = quantize_fp8(g_2d, block_k, transpose=True)     # g.T along M
         qb, sb = quantize_fp8(b, block_k)                          # b along N
         da = scaled_matmul(qg.view(u8), sg, qb.view(u8), sb)
         qat, sat = quantize_fp8(a_2d, block_k, transpose=True)     # a.T along M
@@ -366,77 +411,6 @@ def _bf16_backward(a, b, g):
     return da.reshape(*leading, K).to(a.dtype), db.to(b.dtype)
 
 
-def _fp8_forward_quantized_residuals(a, b, block_k, need_da, need_db):
-    """_fp8_forward with the FP8 operands of the backward kept as residuals.
-
-    a (..., K), b (K, N) bf16, M and N multiples of block_k.  Returns (out,
-    (a.T bytes, a.T scales) or None, (b bytes, b scales) or None): a.T along M
-    for db = fwd(a.T, g), b along N for da = fwd(g, b.T) -- the operands
-    _fp8_backward would quantize from a and b (fp8.py:66,68 on those inputs).
-    When both are kept, their scales are K-block-major and each tuple carries a
-    third element "km" (the layout tg_gemm_fp8_nt_km reads); the bytes and the
-    scale values are the same either way.
-    """
-    leading, K, N = _validate(a, b, block_k)
-    a_2d = a.reshape(-1, K)
-    if need_db and need_da:
-        # a along K + a.T along M, and b along N + b.T along K: one launch, the
-        # scales K-block-major (the residuals' scales too; the backward reads
-        # them with the same GEMM), so the returned residuals are tagged "km"
-        (qa, sa, qat, sat), (qb, sb, qbt, sbt) = _quantize_dual_pair_km(a_2d.contiguous(), b.contiguous(),
-                                                                         block_k)
-        out = _scaled_matmul_km(qa, sa, qbt, sbt)                   # fp8.py:70-78
-        e4 = torch.float8_e4m3fn
-        return out.reshape(*leading, N), (qat.view(e4), sat, "km"), (qb.view(e4), sb, "km")
-    if need_db:
-        qa, sa, qat, sat = quantize_fp8_dual(a_2d, block_k)    # a along K, a.T along M
-        res_a = (qat, sat)
-    else:
-        (qa, sa), res_a = quantize_fp8(a_2d, block_k), None
-    if need_da:
-        qb, sb, qbt, sbt = quantize_fp8_dual(b, block_k)       # b along N, b.T along K
-        res_b = (qb, sb)
-    else:
-        (qbt, sbt), res_b = quantize_fp8(b, block_k, transpose=True), None
-    u8 = torch.uint8
-    out = scaled_matmul(qa.view(u8), sa, qbt.view(u8), sbt)     # fp8.py:70-78
-    return out.reshape(*leading, N), res_a, res_b
-
-
-def _fp8_backward_quantized(block_k, res_a, res_b, g, a_shape, a_dtype, b_dtype):
-    """BACKWARD_MODE "fp8" gradients from the kept FP8 residuals (same bits as
-    _fp8_backward on the bf16 operands)."""
-    N = g.shape[-1]
-    g_2d = g.reshape(-1, N)
-    u8 = torch.uint8
-    km = res_a is not None and len(res_a) == 3
-    if km and g_2d.dtype == torch.bfloat16:
-        # K-block-major scales throughout: g along N and g.T along M from one read
-        qg, sg, qgt, sgt = _quantize_dual_km(g_2d.contiguous(), block_k)
-        (qat, sat, _), (qb, sb, _) = res_a, res_b
-        da = _scaled_matmul_km(qg, sg, qb.view(u8), sb).reshape(a_shape).to(a_dtype)
-        db = _scaled_matmul_km(qat.view(u8), sat, qgt, sgt).to(b_dtype)
-        return da, db
-    if km:
-        # a non-bf16 gradient: its scales come in the reference layout, so the
-        # residuals' scales are transposed back to it
-        res_a = (res_a[0], res_a[1].t().contiguous())
-        res_b = (res_b[0], res_b[1].t().contiguous())
-    if g_2d.dtype == torch.bfloat16 and res_a is not None and res_b is not None:
-        qg, sg, qgt, sgt = quantize_fp8_dual(g_2d, block_k)      # g along N and g.T along M
-    else:
-        qg, sg = quantize_fp8(g_2d, block_k) if res_b is not None else (None, None)
-        qgt, sgt = quantize_fp8(g_2d, block_k, transpose=True) if res_a is not None else (None, None)
-    da = db = None
-    if res_b is not None:
-        qb, sb = res_b
-        da = scaled_matmul(qg.view(u8), sg, qb.view(u8), sb).reshape(a_shape).to(a_dtype)
-    if res_a is not None:
-        qat, sat = res_a
-        db = scaled_matmul(qat.view(u8), sat, qgt.view(u8), sgt).to(b_dtype)
-    return da, db
-
-
 class _BlockScaledMatmul(torch.autograd.Function):
     """custom_vjp of fp8.py:30-36,101 as a torch autograd Function."""
 
@@ -451,14 +425,14 @@ class _BlockScaledMatmul(torch.autograd.Function):
             _check_block_k(block_k)
             M = a.numel() // K if K else 0
             if block_k == TUNED_BLOCK_K and M > 0 and N > 0 and M % block_k == 0 and N % block_k == 0:
-                out, res_a, res_b = _fp8_forward_quantized_residuals(a, b, block_k, need_da,
-                                                                     need_db)
+                # the FP8 operands of the backward (fp8.py:66,68 on g's partners): a.T along
+                # M for db = fwd(a.T, g), b along N for da = fwd(g, b.T)
+                ctx.keep = (_L.TG_KEEP_B if need_da else 0) | (_L.TG_KEEP_A if need_db else 0)
+                out, kept = _linear_fwd(a.reshape(-1, K).contiguous(), b.contiguous(), ctx.keep)
                 ctx.quantized = True
-                ctx.has_a, ctx.has_b = res_a is not None, res_b is not None
-                ctx.km = res_a is not None and len(res_a) == 3      # K-block-major residual scales
-                ctx.save_for_backward(*(res_a[:2] if res_a else ()), *(res_b[:2] if res_b else ()))
+                ctx.save_for_backward(kept)
                 ctx.a_shape, ctx.a_dtype, ctx.b_dtype = a.shape, a.dtype, b.dtype
-                return out
+                return out.reshape(*leading, N)
         out, (ra, rb) = _fp8_forward_with_residuals(a, b, block_k)
         ctx.save_for_backward(ra, rb)
         return out
@@ -469,13 +443,10 @@ class _BlockScaledMatmul(torch.autograd.Function):
             if BACKWARD_MODE != "fp8":
                 raise RuntimeError("BACKWARD_MODE changed between forward and backward: this "
                                    "graph kept FP8 residuals for the 'fp8' backward")
-            saved = list(ctx.saved_tensors)
-            tag = ("km",) if ctx.km else ()
-            res_a = (saved.pop(0), saved.pop(0), *tag) if ctx.has_a else None
-            res_b = (saved.pop(0), saved.pop(0), *tag) if ctx.has_b else None
-            da, db = _fp8_backward_quantized(ctx.block_k, res_a, res_b, g, ctx.a_shape,
-                                             ctx.a_dtype, ctx.b_dtype)
-            return da, db, None
+            (kept,) = ctx.saved_tensors
+            g_2d = _kernel_dtype(g.reshape(-1, g.shape[-1])).contiguous()
+            da, db = _linear_bwd_kept(kept, ctx.keep, g_2d, ctx.a_shape[-1], ctx.a_dtype, ctx.b_dtype)
+            return da.reshape(ctx.a_shape) if da is not None else None, db, None
         a, b = ctx.saved_tensors
         da, db = _fp8_backward(ctx.block_k, (a, b), g)
         return da, db, None
