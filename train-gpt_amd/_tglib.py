@@ -117,9 +117,11 @@ def ptr(t: torch.Tensor):
     return ctypes.c_void_p(t.data_ptr())
 
 
-def stream_of(t: torch.Tensor):
-    """The current torch stream of t's device, as the C ABI's void* stream."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def stream_of(t: torch.Tensor) -> int:
+    """The current torch stream of t's device, as the C ABI's void* stream: the
+    raw handle, without the Stream object torch.cuda.current_stream builds
+    around it (2.2 us a call, 0.1 without)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def require_gpu(*ts: torch.Tensor) -> None:

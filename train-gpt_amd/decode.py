@@ -181,7 +181,7 @@ def decode_embed(embed: torch.Tensor, pos: torch.Tensor, tok: torch.Tensor, t: t
     tk = tok.to(device=embed.device, dtype=torch.int64).contiguous()
     e, p = embed.contiguous(), pos.contiguous()
     out = torch.empty((tk.shape[0], e.shape[1]), dtype=torch.bfloat16, device=e.device)
-    _L.check(_L.lib().tg_decode_embed(_L.ptr(e), _L.ptr(p), _L.ptr(tk), _L.ptr(t), _L.ptr(out), tk.shape[0],
+    _L.check(_L.lib().tg_decode_embed(e.data_ptr(), p.data_ptr(), tk.data_ptr(), t.data_ptr(), out.data_ptr(), tk.shape[0],
                                       e.shape[0], p.shape[0], e.shape[1], _L.stream_of(e)))
     return out
 
@@ -194,7 +194,7 @@ def logit_cap(logits: torch.Tensor, cap: float) -> torch.Tensor:
     _L.require_gpu(logits)
     x = logits.contiguous()
     out = torch.empty(x.shape, dtype=torch.float32, device=x.device)
-    _L.check(_L.lib().tg_logit_cap(_L.ptr(x), _L.ptr(out), x.numel(), float(cap), _L.stream_of(x)))
+    _L.check(_L.lib().tg_logit_cap(x.data_ptr(), out.data_ptr(), x.numel(), float(cap), _L.stream_of(x)))
     return out
 
 
@@ -216,8 +216,8 @@ def decode_attention(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Te
     o_s = torch.empty((B, n_heads), dtype=torch.float32, device=qkv.device)
     o = torch.empty((B, n_heads * Dh), dtype=torch.bfloat16, device=qkv.device) if want_bf16 else None
     _L.check(_L.lib().tg_decode_attention(
-        _L.ptr(qkv), _L.ptr(k_cache), _L.ptr(v_cache), _L.ptr(t), _L.ptr(o_q), _L.ptr(o_s),
-        _L.ptr(o) if o is not None else None, B, n_heads, S, Dh, 1.0 / math.sqrt(Dh),
+        qkv.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), t.data_ptr(), o_q.data_ptr(), o_s.data_ptr(),
+        o.data_ptr() if o is not None else None, B, n_heads, S, Dh, 1.0 / math.sqrt(Dh),
         _L.stream_of(qkv)))
     return o_q.view(torch.float8_e4m3fn), o_s, o
 

@@ -101,12 +101,11 @@ def quantize_fp8(x: torch.Tensor, block_k: int = DEFAULT_BLOCK_K, transpose: boo
     if x.dtype not in (torch.bfloat16, torch.float32):
         x = x.to(torch.float32)
     x2 = x.reshape(-1, K).contiguous()
-    R = x2.shape[0]
-    q = torch.empty((R, K), dtype=torch.uint8, device=x.device)
-    s = torch.empty((R, K // block_k), dtype=torch.float32, device=x.device)
-    _L.check(_L.lib().tg_quantize_rows(_L.ptr(x2), _L.dtype_code(x2), R, K, block_k,
-                                       _L.ptr(q), _L.ptr(s), _L.stream_of(x2)))
-    return q.view(torch.float8_e4m3fn).reshape(*lead, K), s.reshape(*lead, K // block_k)
+    q = torch.empty((*lead, K), dtype=torch.float8_e4m3fn, device=x.device)
+    s = torch.empty((*lead, K // block_k), dtype=torch.float32, device=x.device)
+    _L.check(_L.lib().tg_quantize_rows(x2.data_ptr(), _L.dtype_code(x2), x2.shape[0], K, block_k,
+                                       q.data_ptr(), s.data_ptr(), _L.stream_of(x2)))
+    return q, s
 
 
 def quantize_relu2(x: torch.Tensor, block_k: int = DEFAULT_BLOCK_K):
@@ -120,12 +119,11 @@ def quantize_relu2(x: torch.Tensor, block_k: int = DEFAULT_BLOCK_K):
     if K % block_k:
         raise ValueError(f"K={K} not divisible by block_k={block_k}")
     x2 = x.reshape(-1, K).contiguous()
-    R = x2.shape[0]
-    q = torch.empty((R, K), dtype=torch.uint8, device=x.device)
-    s = torch.empty((R, K // block_k), dtype=torch.float32, device=x.device)
-    _L.check(_L.lib().tg_quantize_rows_relu2(_L.ptr(x2), R, K, block_k, _L.ptr(q), _L.ptr(s),
+    q = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
+    s = torch.empty((*x.shape[:-1], K // block_k), dtype=torch.float32, device=x.device)
+    _L.check(_L.lib().tg_quantize_rows_relu2(x2.data_ptr(), x2.shape[0], K, block_k, q.data_ptr(), s.data_ptr(),
                                              _L.stream_of(x2)))
-    return q.view(torch.float8_e4m3fn).reshape(x.shape), s.reshape(*x.shape[:-1], K // block_k)
+    return q, s
 
 
 def _validate(a: torch.Tensor, b: torch.Tensor, block_k: int):
@@ -238,8 +236,8 @@ def scaled_matmul(a_q, a_s, b_q, b_s, b_scale_bn: int = 1, out_dtype=torch.bfloa
     code = _L.TG_DTYPE_F32 if out_dtype == torch.float32 else _L.TG_DTYPE_BF16
     a_q, b_q = a_q.contiguous(), b_q.contiguous()
     a_s, b_s = a_s.contiguous().float(), b_s.contiguous().float()
-    _L.check(_L.lib().tg_gemm_fp8_nt(_L.ptr(a_q), _L.ptr(a_s), _L.ptr(b_q), _L.ptr(b_s),
-                                     b_scale_bn, _L.ptr(c), code, M, N, K, block_k,
+    _L.check(_L.lib().tg_gemm_fp8_nt(a_q.data_ptr(), a_s.data_ptr(), b_q.data_ptr(), b_s.data_ptr(),
+                                     b_scale_bn, c.data_ptr(), code, M, N, K, block_k,
                                      _L.stream_of(a_q)))
     return c
 
@@ -280,8 +278,9 @@ def _linear_fwd(a_2d, b, keep):
     kept = torch.empty(L.tg_linear_kept_bytes(M, N, K, keep), dtype=u8, device=dev) if keep else None
     ws_bytes = L.tg_linear_fwd_workspace(M, N, K)
     ws = torch.empty(ws_bytes, dtype=u8, device=dev)
-    _L.check(L.tg_linear_fwd(_L.ptr(a_2d), _L.dtype_code(a_2d), _L.ptr(b), _L.dtype_code(b), _L.ptr(out), M, N, K,
-                             keep, _L.ptr(kept) if keep else None, _L.ptr(ws), ws_bytes, _L.stream_of(a_2d)))
+    _L.check(L.tg_linear_fwd(a_2d.data_ptr(), _L.dtype_code(a_2d), b.data_ptr(), _L.dtype_code(b), out.data_ptr(),
+                             M, N, K, keep, kept.data_ptr() if keep else None, ws.data_ptr(), ws_bytes,
+                             _L.stream_of(a_2d)))
     return out, kept
 
 
@@ -289,15 +288,18 @@ def _linear_bwd_kept(kept, keep, g_2d, K, da_dtype, db_dtype):
     """(da or None, db or None) from a forward's kept operands and contiguous g (M, N)."""
     M, N = g_2d.shape
     L, dev = _L.lib(), g_2d.device
-    da = torch.empty((M, K), dtype=da_dtype, device=dev) if keep & _L.TG_KEEP_B else None
-    db = torch.empty((K, N), dtype=db_dtype, device=dev) if keep & _L.TG_KEEP_A else None
+    da = db = pa = pb = None
+    ca = cb = 0
+    if keep & _L.TG_KEEP_B:
+        da = torch.empty((M, K), dtype=da_dtype, device=dev)
+        pa, ca = da.data_ptr(), _L.dtype_code(da)
+    if keep & _L.TG_KEEP_A:
+        db = torch.empty((K, N), dtype=db_dtype, device=dev)
+        pb, cb = db.data_ptr(), _L.dtype_code(db)
     ws_bytes = L.tg_linear_bwd_kept_workspace(M, N)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    _L.check(L.tg_linear_bwd_kept(
-        _L.ptr(kept), keep, _L.ptr(g_2d), _L.dtype_code(g_2d),
-        _L.ptr(da) if da is not None else None, _L.dtype_code(da) if da is not None else 0,
-        _L.ptr(db) if db is not None else None, _L.dtype_code(db) if db is not None else 0, M, N, K,
-        _L.ptr(ws), ws_bytes, _L.stream_of(g_2d)))
+    _L.check(L.tg_linear_bwd_kept(kept.data_ptr(), keep, g_2d.data_ptr(), _L.dtype_code(g_2d), pa, ca, pb, cb,
+                                  M, N, K, ws.data_ptr(), ws_bytes, _L.stream_of(g_2d)))
     return da, db
 
 
@@ -309,8 +311,8 @@ def _linear_bwd(a_2d, b, g_2d):
     da, db = torch.empty_like(a_2d), torch.empty_like(b)
     ws_bytes = L.tg_linear_bwd_workspace(M, N, K)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    _L.check(L.tg_linear_bwd(_L.ptr(a_2d), _L.dtype_code(a_2d), _L.ptr(b), _L.dtype_code(b), _L.ptr(g_2d),
-                             _L.dtype_code(g_2d), _L.ptr(da), _L.ptr(db), M, N, K, _L.ptr(ws), ws_bytes,
+    _L.check(L.tg_linear_bwd(a_2d.data_ptr(), _L.dtype_code(a_2d), b.data_ptr(), _L.dtype_code(b), g_2d.data_ptr(),
+                             _L.dtype_code(g_2d), da.data_ptr(), db.data_ptr(), M, N, K, ws.data_ptr(), ws_bytes,
                              _L.stream_of(a_2d)))
     return da, db
 
@@ -404,8 +406,8 @@ def _bf16_backward(a, b, g):
     ws_bytes = _L.lib().tg_block_scaled_matmul_bwd_bf16_workspace(M, N, K)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=a.device)
     _L.check(_L.lib().tg_block_scaled_matmul_bwd_bf16(
-        _L.ptr(a_2d), _L.dtype_code(a_2d), _L.ptr(b_c), _L.dtype_code(b_c), _L.ptr(g_2d),
-        _L.dtype_code(g_2d), _L.ptr(da), _L.ptr(db), M, N, K, _L.ptr(ws), ws_bytes,
+        a_2d.data_ptr(), _L.dtype_code(a_2d), b_c.data_ptr(), _L.dtype_code(b_c), g_2d.data_ptr(),
+        _L.dtype_code(g_2d), da.data_ptr(), db.data_ptr(), M, N, K, ws.data_ptr(), ws_bytes,
         _L.stream_of(a_2d)))
     # fp8.py:95-96: .astype(a.dtype) / .astype(b.dtype) of the bf16 results (exact widening)
     return da.reshape(*leading, K).to(a.dtype), db.to(b.dtype)
@@ -610,8 +612,7 @@ class QuantizedWeight:
         if 0 < M <= 64:
             return fp8_gemv(x, self.q, self.scales, self.bn, self.block_k, exact=exact)
         a_q, a_s = quantize_fp8(x.reshape(-1, K), self.block_k)
-        out = scaled_matmul(a_q.view(torch.uint8), a_s, self.q.view(torch.uint8), self.scales,
-                            b_scale_bn=self.bn)
+        out = scaled_matmul(a_q, a_s, self.q, self.scales, b_scale_bn=self.bn)
         return out.reshape(*lead, self.shape[1])
 
     def matmul_prequant(self, x_q: torch.Tensor, x_s: torch.Tensor, exact: bool = False) -> torch.Tensor:
@@ -621,14 +622,13 @@ class QuantizedWeight:
         M, K = x_q.shape
         if K != self.shape[0]:
             raise ValueError(f"contracted-dim mismatch: a K={K}, b K={self.shape[0]}")
-        xq = x_q.view(torch.uint8).contiguous()
+        xq = x_q.contiguous()
         xs = x_s.contiguous().float()
         if 0 < M <= 64:
             out = torch.empty((M, self.shape[1]), dtype=torch.bfloat16, device=x_q.device)
-            _gemv_prequant(xq, xs, self.q.view(torch.uint8), self.scales, self.bn, out, self.block_k,
-                           exact)
+            _gemv_prequant(xq, xs, self.q, self.scales, self.bn, out, self.block_k, exact)
             return out
-        return scaled_matmul(xq, xs, self.q.view(torch.uint8), self.scales, b_scale_bn=self.bn)
+        return scaled_matmul(xq, xs, self.q, self.scales, b_scale_bn=self.bn)
 
     def matmul_rms_norm(self, x: torch.Tensor, gamma: torch.Tensor, eps: float,
                         delta: torch.Tensor = None, xout: torch.Tensor = None) -> torch.Tensor:
@@ -652,11 +652,12 @@ class QuantizedWeight:
         _L.require_gpu(x, self.q)
         x = x.contiguous()
         d = delta.contiguous() if delta is not None else None
+        gamma = gamma.contiguous()
         out = torch.empty((x.shape[0], N), dtype=torch.bfloat16, device=x.device)
         _L.check(_L.lib().tg_rms_norm_fp8_gemv(
-            _L.ptr(x), _L.ptr(d) if d is not None else None, _L.ptr(gamma.contiguous()), float(eps),
-            _L.ptr(xout) if d is not None else None, _L.ptr(self.q.view(torch.uint8)), _L.ptr(self.scales),
-            self.bn, _L.ptr(out), x.shape[0], N, K, _L.stream_of(x)))
+            x.data_ptr(), d.data_ptr() if d is not None else None, gamma.data_ptr(), float(eps),
+            xout.data_ptr() if d is not None else None, self.q.data_ptr(), self.scales.data_ptr(),
+            self.bn, out.data_ptr(), x.shape[0], N, K, _L.stream_of(x)))
         return out
 
     def matmul_relu2(self, u: torch.Tensor) -> torch.Tensor:
@@ -669,8 +670,8 @@ class QuantizedWeight:
         _L.require_gpu(u, self.q)
         u = u.contiguous()
         out = torch.empty((u.shape[0], N), dtype=torch.bfloat16, device=u.device)
-        _L.check(_L.lib().tg_relu2_fp8_gemv(_L.ptr(u), _L.ptr(self.q.view(torch.uint8)), _L.ptr(self.scales),
-                                            self.bn, _L.ptr(out), u.shape[0], N, K, _L.stream_of(u)))
+        _L.check(_L.lib().tg_relu2_fp8_gemv(u.data_ptr(), self.q.data_ptr(), self.scales.data_ptr(),
+                                            self.bn, out.data_ptr(), u.shape[0], N, K, _L.stream_of(u)))
         return out
 
     def _check_resid(self, x, resid, out, who):
@@ -696,11 +697,11 @@ class QuantizedWeight:
             raise ValueError(f"matmul_prequant_add: 1-2 rows with K <= {ROWDOT_MAX_K}")
         out = self._check_resid(x_q, resid, out, "matmul_prequant_add")
         _L.require_gpu(x_q, self.q)
-        xq = x_q.view(torch.uint8).contiguous()
+        xq = x_q.contiguous()
         xs = x_s.contiguous().float()
         _L.check(_L.lib().tg_gemv_fp8_rowdot_add(
-            _L.ptr(xq), _L.ptr(xs), _L.ptr(self.q.view(torch.uint8)), _L.ptr(self.scales), self.bn,
-            _L.ptr(resid), _L.ptr(out), M, self.shape[1], K, self.block_k, _L.stream_of(xq)))
+            xq.data_ptr(), xs.data_ptr(), self.q.data_ptr(), self.scales.data_ptr(), self.bn,
+            resid.data_ptr(), out.data_ptr(), M, self.shape[1], K, self.block_k, _L.stream_of(xq)))
         return out
 
     def matmul_relu2_add(self, u: torch.Tensor, resid: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
@@ -714,8 +715,8 @@ class QuantizedWeight:
         out = self._check_resid(u, resid, out, "matmul_relu2_add")
         _L.require_gpu(u, self.q)
         u = u.contiguous()
-        _L.check(_L.lib().tg_relu2_fp8_gemv_add(_L.ptr(u), _L.ptr(self.q.view(torch.uint8)), _L.ptr(self.scales),
-                                                self.bn, _L.ptr(resid), _L.ptr(out), u.shape[0], N, K,
+        _L.check(_L.lib().tg_relu2_fp8_gemv_add(u.data_ptr(), self.q.data_ptr(), self.scales.data_ptr(),
+                                                self.bn, resid.data_ptr(), out.data_ptr(), u.shape[0], N, K,
                                                 _L.stream_of(u)))
         return out
 
@@ -750,15 +751,18 @@ ROWDOT_MAX_K = 16384
 
 
 def _gemv_prequant(xq, xs, wq, ws, bn, out, block_k, exact):
-    """out (M, N) = GEMV of quantized rows xq (M, K) u8, xs on W (wq (N, K) u8, ws).
+    """out (M, N) = GEMV of quantized rows xq (M, K) one byte, xs on W (wq (N, K), ws).
     1-2 rows take tg_gemv_fp8_rowdot (VALU dot products) unless exact, which
     keeps tg_gemv_fp8 (the GEMM's MFMA block arithmetic, bit for bit)."""
-    M, K = xq.shape
-    N = wq.shape[0]
+    _gemv_call(xq.data_ptr(), xs.data_ptr(), wq, ws, bn, out, xq.shape[0], block_k, exact)
+
+
+def _gemv_call(xq_ptr, xs_ptr, wq, ws, bn, out, M, block_k, exact):
+    N, K = wq.shape
     fn = (_L.lib().tg_gemv_fp8_rowdot if (M <= 2 and K <= ROWDOT_MAX_K and not exact)
           else _L.lib().tg_gemv_fp8)
-    _L.check(fn(_L.ptr(xq), _L.ptr(xs), _L.ptr(wq), _L.ptr(ws), bn, _L.ptr(out), M, N, K, block_k,
-                _L.stream_of(xq)))
+    _L.check(fn(xq_ptr, xs_ptr, wq.data_ptr(), ws.data_ptr(), bn, out.data_ptr(), M, N, K, block_k,
+                _L.stream_of(out)))
 
 
 def fp8_gemv(x: torch.Tensor, w_q: torch.Tensor, w_s: torch.Tensor, w_scale_bn: int = 1,
@@ -772,9 +776,18 @@ def fp8_gemv(x: torch.Tensor, w_q: torch.Tensor, w_s: torch.Tensor, w_scale_bn: 
     N = w_q.shape[0]
     if w_q.shape[1] != K:
         raise ValueError(f"contracted-dim mismatch: x K={K}, w K={w_q.shape[1]}")
-    x_q, x_s = quantize_fp8(x.reshape(-1, K), block_k)
-    M = x_q.shape[0]
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    _gemv_prequant(x_q.view(torch.uint8), x_s, w_q.view(torch.uint8).contiguous(), w_s.contiguous(),
-                   w_scale_bn, out, block_k, exact)
-    return out.reshape(*lead, N)
+    if K % block_k:
+        raise ValueError(f"K={K} not divisible by block_k={block_k}")
+    if x.dtype not in _KERNEL_DTYPES:
+        x = x.to(torch.float32)
+    x2 = x.reshape(-1, K).contiguous()
+    M = x2.shape[0]
+    # the quantized rows, then their scales, in one scratch buffer
+    so = (M * K + 255) // 256 * 256
+    xq = torch.empty(so + M * (K // block_k) * 4, dtype=torch.uint8, device=x.device)
+    qp = xq.data_ptr()
+    out = torch.empty((*lead, N), dtype=torch.bfloat16, device=x.device)
+    _L.check(_L.lib().tg_quantize_rows(x2.data_ptr(), _L.dtype_code(x2), M, K, block_k, qp, qp + so,
+                                       _L.stream_of(x2)))
+    _gemv_call(qp, qp + so, w_q.contiguous(), w_s.contiguous(), w_scale_bn, out, M, block_k, exact)
+    return out

@@ -50,11 +50,11 @@ def _out_dtype(x: torch.Tensor, scale: torch.Tensor):
 def _rms_norm_pure(x: torch.Tensor, scale: torch.Tensor, eps: float) -> torch.Tensor:
     """kernels.py:30-33 on the GPU: x (..., D), scale (D,), bf16, f16 or f32 -> (..., D) in the promoted dtype."""
     x2, g, D = _prep(x, scale, bf16_only=False)
-    y = torch.empty(x2.shape, dtype=_out_dtype(x, scale), device=x.device)
+    y = torch.empty(x.shape, dtype=_out_dtype(x, scale), device=x.device)
     # bf16 x and scale with D % 8 == 0 (D <= 16384) take the fast kernel inside
-    _L.check(_L.lib().tg_rms_norm_ex(_L.ptr(x2), _L.norm_dtype_code(x2), _L.ptr(g), _L.norm_dtype_code(g),
-                                     _L.ptr(y), x2.shape[0], D, float(eps), _L.stream_of(x2)))
-    return y.reshape(x.shape)
+    _L.check(_L.lib().tg_rms_norm_ex(x2.data_ptr(), _L.norm_dtype_code(x2), g.data_ptr(), _L.norm_dtype_code(g),
+                                     y.data_ptr(), x2.shape[0], D, float(eps), _L.stream_of(x2)))
+    return y
 
 
 def rms_norm_fp8(x: torch.Tensor, scale: torch.Tensor, eps: float, block_k: int = 128):
@@ -84,15 +84,13 @@ def add_rms_norm_fp8(x: torch.Tensor, delta: torch.Tensor, scale: torch.Tensor, 
     d2 = delta.reshape(-1, D).contiguous()
     R = x2.shape[0]
     xo = x2 if inplace else torch.empty_like(x2)
-    y = torch.empty_like(x2) if want_y else None
-    q = torch.empty((R, D), dtype=torch.uint8, device=x.device)
-    s = torch.empty((R, D // block_k), dtype=torch.float32, device=x.device)
-    _L.check(_L.lib().tg_add_rms_norm_fp8(_L.ptr(x2), _L.ptr(d2), _L.ptr(g), _L.ptr(xo),
-                                          _L.ptr(y) if y is not None else None, _L.ptr(q), _L.ptr(s),
+    y = torch.empty(x.shape, dtype=x.dtype, device=x.device) if want_y else None
+    q = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
+    s = torch.empty((*x.shape[:-1], D // block_k), dtype=torch.float32, device=x.device)
+    _L.check(_L.lib().tg_add_rms_norm_fp8(x2.data_ptr(), d2.data_ptr(), g.data_ptr(), xo.data_ptr(),
+                                          y.data_ptr() if y is not None else None, q.data_ptr(), s.data_ptr(),
                                           R, D, float(eps), block_k, _L.stream_of(x2)))
-    lead = x.shape[:-1]
-    return (xo.reshape(x.shape), q.view(torch.float8_e4m3fn).reshape(x.shape),
-            s.reshape(*lead, D // block_k), y.reshape(x.shape) if y is not None else None)
+    return xo.reshape(x.shape), q, s, y
 
 
 def _rms_norm_fp8_fwd(x: torch.Tensor, scale: torch.Tensor, eps: float, block_k: int):
@@ -100,14 +98,12 @@ def _rms_norm_fp8_fwd(x: torch.Tensor, scale: torch.Tensor, eps: float, block_k:
     if D % block_k:
         raise ValueError(f"K={D} not divisible by block_k={block_k}")
     R = x2.shape[0]
-    y = torch.empty_like(x2)
-    q = torch.empty((R, D), dtype=torch.uint8, device=x.device)
-    s = torch.empty((R, D // block_k), dtype=torch.float32, device=x.device)
-    _L.check(_L.lib().tg_rms_norm_fp8(_L.ptr(x2), _L.ptr(g), _L.ptr(y), _L.ptr(q), _L.ptr(s), R, D,
+    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    q = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
+    s = torch.empty((*x.shape[:-1], D // block_k), dtype=torch.float32, device=x.device)
+    _L.check(_L.lib().tg_rms_norm_fp8(x2.data_ptr(), g.data_ptr(), y.data_ptr(), q.data_ptr(), s.data_ptr(), R, D,
                                       float(eps), block_k, _L.stream_of(x2)))
-    lead = x.shape[:-1]
-    return (y.reshape(x.shape), q.view(torch.float8_e4m3fn).reshape(x.shape),
-            s.reshape(*lead, D // block_k))
+    return y, q, s
 
 
 def _rms_norm_bwd(x: torch.Tensor, scale: torch.Tensor, eps: float, g: torch.Tensor):
@@ -117,15 +113,15 @@ def _rms_norm_bwd(x: torch.Tensor, scale: torch.Tensor, eps: float, g: torch.Ten
         g = g.to(torch.float32)
     g2 = g.reshape(-1, D).contiguous()
     R = x2.shape[0]
-    dx = torch.empty_like(x2)
+    dx = torch.empty(x.shape, dtype=x.dtype, device=x.device)
     dscale = torch.empty((D,), dtype=scale.dtype, device=x.device)
     ws_bytes = _L.lib().tg_rms_norm_bwd_workspace(R, D)
     ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=x.device)
     # all-bf16 operands with D % 8 == 0 take tg_rms_norm_bwd's kernels inside
     _L.check(_L.lib().tg_rms_norm_bwd_ex(
-        _L.ptr(x2), _L.norm_dtype_code(x2), _L.ptr(sc), _L.norm_dtype_code(sc), _L.ptr(g2), _L.norm_dtype_code(g2),
-        _L.ptr(dx), _L.ptr(dscale), R, D, float(eps), _L.ptr(ws), ws_bytes, _L.stream_of(x2)))
-    return dx.reshape(x.shape), dscale
+        x2.data_ptr(), _L.norm_dtype_code(x2), sc.data_ptr(), _L.norm_dtype_code(sc), g2.data_ptr(), _L.norm_dtype_code(g2),
+        dx.data_ptr(), dscale.data_ptr(), R, D, float(eps), ws.data_ptr(), ws_bytes, _L.stream_of(x2)))
+    return dx, dscale
 
 
 class _RMSNormFP8(torch.autograd.Function):

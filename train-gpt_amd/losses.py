@@ -27,8 +27,8 @@ class _CappedXent(torch.autograd.Function):
         R = l2.shape[0]
         row_loss = torch.empty(R, dtype=torch.float32, device=logits.device)
         row_lse = torch.empty(R, dtype=torch.float32, device=logits.device)
-        _L.check(_L.lib().tg_logit_cap_xent_fwd(_L.ptr(l2), _L.ptr(t2), R, V, float(cap),
-                                                _L.ptr(row_loss), _L.ptr(row_lse),
+        _L.check(_L.lib().tg_logit_cap_xent_fwd(l2.data_ptr(), t2.data_ptr(), R, V, float(cap),
+                                                row_loss.data_ptr(), row_lse.data_ptr(),
                                                 _L.stream_of(l2)))
         if loss_mask is None:
             loss, w = row_loss.mean(), None                                 # losses.py:12
@@ -47,9 +47,9 @@ class _CappedXent(torch.autograd.Function):
         g1 = g.reshape(1).to(torch.float32).contiguous()
         dl = torch.empty_like(l2)
         g_scale = 1.0 if w is not None else 1.0 / max(R, 1)
-        _L.check(_L.lib().tg_logit_cap_xent_bwd(_L.ptr(l2), _L.ptr(t2), _L.ptr(row_lse), _L.ptr(g1),
-                                                g_scale, _L.ptr(w) if w is not None else None,
-                                                R, V, ctx.cap, _L.ptr(dl), _L.stream_of(l2)))
+        _L.check(_L.lib().tg_logit_cap_xent_bwd(l2.data_ptr(), t2.data_ptr(), row_lse.data_ptr(), g1.data_ptr(),
+                                                g_scale, w.data_ptr() if w is not None else None,
+                                                R, V, ctx.cap, dl.data_ptr(), _L.stream_of(l2)))
         return dl.reshape(ctx.shape), None, None, None
 
 
@@ -89,6 +89,6 @@ def capped_cross_entropy_rows(logits: torch.Tensor, target_ids: torch.Tensor, lo
     R = l2.shape[0]
     nll = torch.empty(R, dtype=torch.float32, device=logits.device)
     lse = torch.empty(R, dtype=torch.float32, device=logits.device)
-    _L.check(_L.lib().tg_logit_cap_xent_fwd(_L.ptr(l2), _L.ptr(t2), R, V, float(logit_cap),
-                                            _L.ptr(nll), _L.ptr(lse), _L.stream_of(l2)))
+    _L.check(_L.lib().tg_logit_cap_xent_fwd(l2.data_ptr(), t2.data_ptr(), R, V, float(logit_cap),
+                                            nll.data_ptr(), lse.data_ptr(), _L.stream_of(l2)))
     return nll.reshape(target_ids.shape), lse.reshape(target_ids.shape)
