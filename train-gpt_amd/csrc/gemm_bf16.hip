@@ -143,14 +143,18 @@ __device__ __forceinline__ uint4 tn_frag(const uint8_t* l, const Q4Ctx& c, uint3
                     ((uint32_t)(uint16_t)hi[2]) | ((uint32_t)(uint16_t)hi[3] << 16));
 }
 
-// s_waitcnt vmcnt(16) as the builtin (gfx9 encoding: vmcnt bits 15:14 = 1,
-// expcnt and lgkmcnt not waited), which the compiler's own wait insertion
-// takes into account; an inline-asm wait is opaque to it.
-constexpr int kWaitVm16 = (1 << 14) | (0xF << 8) | (0x7 << 4);
+// s_waitcnt vmcnt(16) lgkmcnt(0), and lgkmcnt(0) alone, as the builtin (gfx9
+// encoding: vmcnt bits 3:0 and 15:14, expcnt not waited), which the compiler's
+// own wait insertion takes into account; an inline-asm wait is opaque to it.
+// lgkmcnt: a wave's reads of slice ks - 1 have left LDS before a loader, past
+// the barrier, refills that stage (the refills past the last slice return their
+// zeros at once, without a trip to memory).
+constexpr int kWaitVm16 = (1 << 14) | (0x7 << 4);
+constexpr int kWaitLds = (3 << 14) | (0x7 << 4) | 0xF;
 
 template <int S, bool LOADER, bool TN>
 __device__ __forceinline__ void q4_step(const Q4Ctx& c, int ks, v4f (&acc)[4][8]) {
-  if (LOADER) __builtin_amdgcn_s_waitcnt(kWaitVm16);
+  __builtin_amdgcn_s_waitcnt(LOADER ? kWaitVm16 : kWaitLds);
   __builtin_amdgcn_s_barrier();
   constexpr int kRefill = (S + 3) & 3;   // the stage slice ks - 1 occupied
   q4_issue<LOADER, TN>(c, q4_a<kRefill>(), q4_b<kRefill>(), ks + 3);
