@@ -4,9 +4,10 @@
 //   c[m, n] = bf16( sum_kb sa[m, kb] * sb[n, kb] * sum_{k in kb} qa[m, k] * qb[n, k] )
 // with e4m3fn operands and one fp32 scale per 128-wide K block.
 //
-// Two kernels: gemm_fp8_nt_256_kernel (256 x 256 tiles on 32 x 32 x 64
-// MFMAs, persistent; used once a launch has >= 128 tiles, see its own
-// comment) and gemm_fp8_nt_kernel below (128 x 128 tiles) for smaller shapes.
+// Three kernels, one set of output bits: gemm_fp8_nt_256_kernel (256 x 256 tiles
+// on 32 x 32 x 64 MFMAs, persistent; used where its tiles fill the chip),
+// gemm_fp8_lat_kernel (32- to 128-row tiles, gemm_tile_of chooses) and, for
+// operands past 32-bit buffer offsets, gemm_fp8_nt_kernel below (128 x 128 tiles).
 //
 // Design of the 128 x 128 kernel (gfx950, wave64):
 //   * v_mfma_f32_16x16x128_f8f6f4: one MFMA consumes exactly one 128-wide
@@ -186,16 +187,17 @@ __global__ __launch_bounds__(256, 2) void gemm_fp8_nt_kernel(
 template <int V> using IntC = std::integral_constant<int, V>;
 
 // ---------------------------------------------------------------------------
-// Short-K kernel for launches of fewer than 128 tiles of 256 x 256 (C1's
-// 2048 x 3072 x 768 and the decode prefill's GEMMs).  With a few K blocks per
+// Short-K kernel for launches that the 256 x 256 tiles fill badly (C1's
+// 2048 x 3072 x 768, the decode prefill's GEMMs; gemm_tile_of chooses).  With a few K blocks per
 // tile (6 at K = 768) the time a block's bytes take to arrive, not the MFMAs,
 // is what one block in flight leaves exposed; here NST stages of one K block
 // each ring through LDS, so NST - 1 blocks are in flight while one is computed.
-//   * Workgroup tile 128 x BN (BN = 32 * TN), 2 x WN waves, wave tile
-//     64 x BN / WN on v_mfma_f32_16x16x128_f8f6f4: the same fragments, MFMA
+//   * Workgroup tile BM x BN (32 TM x 32 TN), 2 x WN waves, wave tile
+//     16 TM x BN / WN on v_mfma_f32_16x16x128_f8f6f4: the same fragments, MFMA
 //     operand order and promotion as gemm_fp8_nt_kernel, so the same bits.
+//     OCC: workgroups that fit a CU together, each with its share of the LDS.
 //   * Copies: HBM -> LDS with buffer_load ... lds (no VGPR staging).  A stage
-//     is 128 + BN rows of 128 B plus the block's scales; the W waves split the
+//     is BM + BN rows of 128 B plus the block's scales; the W waves split the
 //     A rows and the B rows evenly, 8 rows (1 KiB) per instruction, and the
 //     64-float scale copies (padded to a multiple of W with copies that read
 //     nothing).  16-byte chunk c of row r sits at c ^ g256_swz(r): the 16 rows
@@ -212,19 +214,20 @@ template <int V> using IntC = std::integral_constant<int, V>;
 //     LDS region and stores whole 16-byte pieces of rows; otherwise element
 //     stores.
 // ---------------------------------------------------------------------------
-template <int TN, int WN> struct LatCfg {
-  static constexpr int TM = 4, BM = 128, BN = 32 * TN, W = 2 * WN;
-  static constexpr int TNW = 2 * TN / WN;                     // 16-column tiles per wave
-  static constexpr int APW = 16 / W, BPW = 4 * TN / W;        // 1 KiB copies per wave: A, B
-  static constexpr int SAC = BM / 64, SBC = (BN + 63) / 64;   // 64-float scale copies of A / B
-  static constexpr int SCW = (SAC + SBC + W - 1) / W;         // scale copies per wave (padded)
-  static constexpr int SREG = W * SCW * 64;                   // scale floats per stage
-  static constexpr int STAGE = (BM + BN) * 128 + SREG * 4;    // bytes per stage
-  static constexpr int NST = 163840 / STAGE > 6 ? 6 : 163840 / STAGE;
-  static constexpr int IPW = APW + BPW + SCW;                 // copy instructions per wave per block
-  static constexpr int RP = 32 * TNW + 16;                    // epilogue row pitch (bytes)
-  static constexpr int RPS = (W + NST - 1) / NST;             // epilogue regions per stage
-  static_assert(16 % W == 0 && (4 * TN) % W == 0 && (2 * TN) % WN == 0, "even split over the waves");
+template <int TM_, int TN, int WN, int OCC> struct LatCfg {
+  static constexpr int TM = TM_, BM = 32 * TM, BN = 32 * TN, W = 2 * WN;
+  static constexpr int TNW = 2 * TN / WN;                          // 16-column tiles per wave
+  static constexpr int APW = BM / 8 / W, BPW = 4 * TN / W;         // 1 KiB copies per wave: A, B
+  static constexpr int SAC = (BM + 63) / 64, SBC = (BN + 63) / 64; // 64-float scale copies of A / B
+  static constexpr int SCW = (SAC + SBC + W - 1) / W;              // scale copies per wave (padded)
+  static constexpr int SREG = W * SCW * 64;                        // scale floats per stage
+  static constexpr int STAGE = (BM + BN) * 128 + SREG * 4;         // bytes per stage
+  static constexpr int FIT = 163840 / OCC / STAGE;                 // stages that leave OCC workgroups per CU
+  static constexpr int NST = FIT > 6 ? 6 : FIT;
+  static constexpr int IPW = APW + BPW + SCW;                      // copy instructions per wave per block
+  static constexpr int RP = 32 * TNW + 16;                         // epilogue row pitch (bytes)
+  static constexpr int RPS = (W + NST - 1) / NST;                  // epilogue regions per stage
+  static_assert((BM / 8) % W == 0 && (4 * TN) % W == 0 && (2 * TN) % WN == 0, "even split over the waves");
   static_assert(APW <= 4 && BPW <= 6 && SCW <= 2, "within LatLoad's arrays");
 };
 
@@ -287,9 +290,13 @@ __device__ __forceinline__ void lat_step(const LatLoad& ld, const LatFrag& f,
                                          int kb_refill) {
   constexpr int TM = Cfg::TM, TNW = Cfg::TNW;
   constexpr int kWait = (Cfg::NST - 2) * Cfg::IPW;
-  // s_waitcnt vmcnt(kWait) in the gfx9 encoding (vmcnt low bits 3:0, high
-  // bits 15:14; expcnt and lgkmcnt not waited)
-  constexpr int kWaitImm = (kWait & 15) | ((kWait >> 4) << 14) | (0x7 << 4) | (0xF << 8);
+  // s_waitcnt vmcnt(kWait) lgkmcnt(0) in the gfx9 encoding (vmcnt low bits 3:0,
+  // high bits 15:14; expcnt not waited).  lgkmcnt: this wave's reads of block
+  // kb - 1 have left LDS before another wave, past the barrier, refills that
+  // stage.  A refill past the last block returns its zeros without a trip to
+  // memory, fast enough to overtake a read that the compiler left in flight
+  // across the barrier (seen as wrong sums with three workgroups on a CU).
+  constexpr int kWaitImm = (kWait & 15) | ((kWait >> 4) << 14) | (0x7 << 4);
   __builtin_amdgcn_s_waitcnt(kWaitImm);
   __builtin_amdgcn_s_barrier();
   lat_issue<Cfg>(ld, refill, kb_refill);
@@ -333,17 +340,20 @@ __device__ __forceinline__ uint8_t* lat_pick(uint8_t* s0, uint8_t* s1, uint8_t* 
 // each element then copied out for the promotion; this file is built with
 // -amdgpu-mfma-vgpr-form, which keeps them in VGPRs and changes no other
 // kernel here.)
-template <int TN, int WN, int BNS, bool OUT_F32, bool SKM>
-__global__ __launch_bounds__(128 * WN, 1) void gemm_fp8_lat_kernel(
+// out: kLatBf16, kLatF32, or kLatF32Of16 (the bf16 result widened).
+constexpr int kLatBf16 = 0, kLatF32 = 1, kLatF32Of16 = 2;
+template <int TM_, int TN, int WN, int OCC, int BNS, bool SKM>
+__global__ __launch_bounds__(128 * WN, OCC * WN / 2 > 1 ? OCC * WN / 2 : 1) void gemm_fp8_lat_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ SA, const uint8_t* __restrict__ B,
     const float* __restrict__ SB, void* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
-    int vec_out, int round16) {
-  using Cfg = LatCfg<TN, WN>;
+    int vec_out, int out) {
+  using Cfg = LatCfg<TM_, TN, WN, OCC>;
   constexpr int TM = Cfg::TM, BM = Cfg::BM, BN = Cfg::BN, NST = Cfg::NST, STAGE = Cfg::STAGE;
   constexpr int TNW = Cfg::TNW, W = Cfg::W;
   static_assert(NST >= 3, "at least two blocks in flight");
   static_assert((NST - 2) * Cfg::IPW <= 63, "vmcnt immediate");
-  static_assert(Cfg::RPS * 64 * Cfg::RP <= STAGE, "epilogue regions fit the stages");
+  static_assert(Cfg::RPS * 16 * TM * Cfg::RP <= STAGE, "epilogue regions fit the stages");
+  static_assert(2 * TM * Cfg::TNW * 16 % 64 == 0, "whole waves of 16-byte pieces");
   __shared__ __attribute__((aligned(16))) uint8_t st0[STAGE];
   __shared__ __attribute__((aligned(16))) uint8_t st1[STAGE];
   __shared__ __attribute__((aligned(16))) uint8_t st2[STAGE];
@@ -453,15 +463,17 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_fp8_lat_kernel(
 #undef TG_LAT_STEP
 
   // ---- epilogue: lane holds rows 4 * fg + r, column fr of each 16 x 16 tile ----
+  // every copy has landed (the last ones read zero): none may outlive the
+  // workgroup's LDS
+  __builtin_amdgcn_s_waitcnt(0x0070 | 0x0F00);      // vmcnt(0)
   const int mw = m0 + wm * 16 * TM, nw = n0 + wn * 16 * TNW;
-  if (!OUT_F32 && vec_out) {
-    // every copy has landed (the last ones read zero) and every wave is done
-    // with the stages before they hold results
-    __builtin_amdgcn_s_waitcnt(0x0070 | 0x0F00);    // vmcnt(0)
+  if (out == kLatBf16 && vec_out) {
+    // every wave is done with the stages before they hold results
+    __builtin_amdgcn_s_waitcnt(0xC07F);             // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     const int so = wave % NST;
     uint8_t* wb = (so == 0 ? st0 : so == 1 ? st1 : so == 2 ? st2 : so == 3 ? st3 : so == 4 ? st4 : st5) +
-                  (wave / NST) * 64 * Cfg::RP;
+                  (wave / NST) * 16 * TM * Cfg::RP;
     lds_u8* wl = (lds_u8*)wb;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -474,7 +486,7 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_fp8_lat_kernel(
     // a wave reads back only what it wrote; LDS completes a wave's accesses in order
     constexpr int CPR = 2 * TNW;                    // 16-byte pieces per row
 #pragma unroll
-    for (int u = 0; u < CPR; ++u) {
+    for (int u = 0; u < CPR * 16 * TM / 64; ++u) {
       const int idx = lane + 64 * u, row = idx / CPR, ch = idx % CPR;
       const u32x4_t v = lat_ld16(wl + row * Cfg::RP + ch * 16);
       const int m = mw + row, n = nw + ch * 8;
@@ -492,8 +504,9 @@ __global__ __launch_bounds__(128 * WN, 1) void gemm_fp8_lat_kernel(
       for (int r = 0; r < 4; ++r) {
         const int m = mw + i * 16 + 4 * fg + r;
         if (m < M && n < N) {
-          if (OUT_F32)
-            reinterpret_cast<float*>(C)[(int64_t)m * N + n] = round16 ? round_bf16(acc[i][j][r]) : acc[i][j][r];
+          if (out != kLatBf16)
+            reinterpret_cast<float*>(C)[(int64_t)m * N + n] =
+                out == kLatF32Of16 ? round_bf16(acc[i][j][r]) : acc[i][j][r];
           else
             reinterpret_cast<__bf16*>(C)[(int64_t)m * N + n] = (__bf16)acc[i][j][r];
         }
@@ -1078,54 +1091,74 @@ static int launch_gemm_cfg(const uint8_t* a_q, const float* a_s, const uint8_t* 
   return check_launch("gemm_fp8_nt");
 }
 
-#ifndef TG_LAT_WN
-#define TG_LAT_WN 4
-#endif
-template <int TN, bool SKM>
+template <int TM, int TN, int WN, int OCC, bool SKM>
 static int launch_gemm_lat(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, const float* b_s,
                            int b_scale_bn, void* c, bool f32, int M, int N, int K, int r16, hipStream_t st) {
-  constexpr int BM = 128, BN = 32 * TN, WN = TG_LAT_WN;
-  if constexpr ((2 * TN) % WN != 0) {
-    return einval("gemm_fp8_lat: tile width not split over the waves");
-  } else {
+  constexpr int BM = 32 * TM, BN = 32 * TN;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const int vec = !f32 && N % 8 == 0 && aligned(c, 16);
-  const dim3 grid((unsigned)(tiles_m * tiles_n));
-#define TG_LAT(BNS, F32)                                                                                    \
-  hipLaunchKernelGGL((gemm_fp8_lat_kernel<TN, WN, BNS, F32, SKM>), grid, dim3(128 * WN), 0, st, a_q, a_s, b_q, \
-                     b_s, c, M, N, K, tiles_m, tiles_n, vec, r16)
-  if (b_scale_bn == 1) {
-    if (f32) TG_LAT(1, true); else TG_LAT(1, false);
-  } else {
-    if (f32) TG_LAT(128, true); else TG_LAT(128, false);
-  }
-#undef TG_LAT
+  const int vec = N % 8 == 0 && aligned(c, 16);
+  const int out = r16 ? kLatF32Of16 : f32 ? kLatF32 : kLatBf16;
+  const dim3 grid((unsigned)(tiles_m * tiles_n)), block(128 * WN);
+  if (b_scale_bn == 1)
+    hipLaunchKernelGGL((gemm_fp8_lat_kernel<TM, TN, WN, OCC, 1, SKM>), grid, block, 0, st, a_q, a_s, b_q, b_s, c, M,
+                       N, K, tiles_m, tiles_n, vec, out);
+  else
+    hipLaunchKernelGGL((gemm_fp8_lat_kernel<TM, TN, WN, OCC, 128, SKM>), grid, block, 0, st, a_q, a_s, b_q, b_s, c,
+                       M, N, K, tiles_m, tiles_n, vec, out);
   return check_launch("gemm_fp8_lat");
-  }
 }
 
-// Build-time choice of the short-K kernel (0: the VGPR-staged 128-row kernel
-// for every launch below 128 tiles of 256).
-#ifndef TG_GEMM_LAT
-#define TG_GEMM_LAT 1
-#endif
-static bool lat_kernel_enabled() { return TG_GEMM_LAT != 0; }
+// The kernels that give one GEMM's bits, and what each costs.  A tile's time is
+// a fixed part (first round trip, epilogue, launch) plus a part per K block,
+// measured on 256 CUs at 18 and 72 blocks; `two` are the times of a CU's two
+// resident workgroups together, for the shapes that leave room for two.  The
+// 64-row and 32-row tiles of four waves hide one workgroup's round trips and
+// barriers behind the other's MFMAs; the 128-row tiles of eight waves read
+// fewer bytes per product, and the 256 x 256 persistent kernel fewest.
+// us, before (128-row tiles of 64 to 192 columns) -> now: 512 x 2304 x 9216 36.0
+// -> 29.9, 512 x 6912 x 2304 18.0 -> 16.4, 128 x 2304 x 9216 34.9 -> 16.7, 768 x
+// 3072 x 2048 15.9 -> 12.9, 2048 x 2304 x 2304 22.5 -> 20.8, 3000 x 2304 x 9216
+// (4096 x 4352 x 4096) 108 -> 95 (113 -> 104).
+struct GemmTile {
+  int bm, bn, occ;
+  float f1, b1, f2, b2;   // us: fixed and per K block, one and two workgroups on a CU
+};
+constexpr GemmTile kGemmTiles[] = {
+    {256, 256, 1, 6.5f, 0.f, 0.f, 0.f},      // 0: gemm_fp8_nt_256_kernel (per block below)
+    {128, 256, 1, 7.5f, 1.22f, 0.f, 0.f},    // 1: lat <4, 8, 4, 1>
+    {128, 192, 1, 6.9f, 0.90f, 0.f, 0.f},    // 2: lat <4, 6, 4, 1>
+    {64, 128, 2, 3.8f, 0.446f, 4.3f, 0.634f},  // 3: lat <2, 4, 2, 2>
+    {64, 96, 2, 3.8f, 0.365f, 4.1f, 0.541f},   // 4: lat <2, 3, 2, 2>
+    {64, 64, 2, 3.6f, 0.267f, 3.9f, 0.459f},   // 5: lat <2, 2, 2, 2>
+    {32, 64, 2, 3.4f, 0.185f, 4.0f, 0.290f},   // 6: lat <1, 2, 2, 2>
+};
 
-// The short-K kernel's tile width: 192, 128, 96 or 64 columns, whichever
-// leaves the busiest CU the least work, counted as workgroups per CU (one
-// fits a CU) times (columns + 48), the 48 standing for a tile's fixed cost
-// (pipeline fill, epilogue).  C1's 2048 x 3072: 256 tiles of 192, one per CU.
-static int lat_tile_n(int m, int n) {
+// The tile with the least modelled time.  Successive workgroups of a CU overlap
+// a launch's and a round trip's ~2 us.  The 256 kernel's block takes
+// 1.4 us on few CUs and 1.95 on all of them (the board's power), and output rows
+// that are not 16-byte aligned cost its tile 29 us more in 2-byte stores (512 x
+// 50257 against 50256 x 2304; a wider store beside the kept one takes registers
+// that the K loop needs: 5% to 4x slower).
+static int gemm_tile_of(int64_t m, int64_t n, int64_t nkb) {
   const int64_t cus = device_cus() > 0 ? device_cus() : 1;
-  int best = 6;
-  int64_t best_cost = -1;
-  for (int tn : {6, 4, 3, 2}) {
-    if ((2 * tn) % TG_LAT_WN) continue;               // the wave split needs whole 16-column tiles
-    const int64_t tiles = (int64_t)((m + 127) / 128) * ((n + 32 * tn - 1) / (32 * tn));
-    const int64_t cost = (tiles + cus - 1) / cus * (32 * tn + 48);
-    if (best_cost < 0 || cost < best_cost) {
-      best = tn;
-      best_cost = cost;
+  int best = 0;
+  double cost = 1e300;
+  for (int i = 0; i < (int)(sizeof(kGemmTiles) / sizeof(kGemmTiles[0])); ++i) {
+    const GemmTile& t = kGemmTiles[i];
+    const int64_t wgs = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+    const double r = (double)((wgs + cus - 1) / cus);
+    double c;
+    if (i == 0) {
+      const double fill = (double)wgs / (r * (double)cus), block = 1.4 + 0.55 * fill * fill;
+      c = r * (t.f1 + (n % 8 ? 29.0 : 0.0) + block * (double)nkb);
+    } else {
+      const double one = t.f1 + t.b1 * (double)nkb - 2.0, two = t.f2 + t.b2 * (double)nkb - 2.0;
+      const int64_t ri = (int64_t)r;
+      c = 2.0 + (t.occ == 2 ? (double)(ri / 2) * two + (double)(ri % 2) * one : r * one);
+    }
+    if (c < cost) {
+      cost = c;
+      best = i;
     }
   }
   return best;
@@ -1134,16 +1167,19 @@ static int lat_tile_n(int m, int n) {
 template <bool SKM>
 static int launch_gemm_fp8_layout(const uint8_t* a_q, const float* a_s, const uint8_t* b_q,
                                   const float* b_s, int b_scale_bn, void* c, bool f32, int m, int n,
-                                  int k, int r16, bool big, bool lat, hipStream_t st) {
-  if (lat) {
-    switch (lat_tile_n(m, n)) {
-      case 6: return launch_gemm_lat<6, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st);
-      case 4: return launch_gemm_lat<4, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st);
-      case 3: return launch_gemm_lat<3, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st);
-      default: return launch_gemm_lat<2, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st);
+                                  int k, int r16, bool fits32, hipStream_t st) {
+  if (fits32) {
+#define TG_LAT(...) launch_gemm_lat<__VA_ARGS__, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st)
+    switch (gemm_tile_of(m, n, k / 128)) {
+      case 1: return TG_LAT(4, 8, 4, 1);
+      case 2: return TG_LAT(4, 6, 4, 1);
+      case 3: return TG_LAT(2, 4, 2, 2);
+      case 4: return TG_LAT(2, 3, 2, 2);
+      case 5: return TG_LAT(2, 2, 2, 2);
+      case 6: return TG_LAT(1, 2, 2, 2);
+      default: break;
     }
-  }
-  if (big) {
+#undef TG_LAT
     if (b_scale_bn == 1)
       return f32 ? launch_gemm_256<1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
                  : launch_gemm_256<1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
@@ -1179,13 +1215,10 @@ int launch_gemm_fp8(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, co
   const int m = (int)M, n = (int)N, k = (int)K;
   const int r16 = c_dtype == kOutF32OfBf16;   // f32 output holding the bf16 result
   const bool f32 = c_dtype == TG_DTYPE_F32 || r16;
-  // 256 x 256 tiles once they fill the chip (>= 128 workgroups), else 128 x 128
+  // the tuned kernels take 32-bit buffer offsets; larger operands the VGPR-staged one
   const bool fits32 = (uint64_t)M * (uint64_t)K < (1ull << 31) && (uint64_t)N * (uint64_t)K < (1ull << 31);
-  const bool big = fits32 && ((M + 255) / 256) * ((N + 255) / 256) >= 128;
-  // below that, the short-K ring kernel (32-bit buffer offsets, as the 256 kernel)
-  const bool lat = fits32 && !big && lat_kernel_enabled();
-  return skm ? launch_gemm_fp8_layout<true>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, big, lat, st)
-             : launch_gemm_fp8_layout<false>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, big, lat, st);
+  return skm ? launch_gemm_fp8_layout<true>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, fits32, st)
+             : launch_gemm_fp8_layout<false>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, fits32, st);
 }
 
 // ---------------------------------------------------------------------------
