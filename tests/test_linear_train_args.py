@@ -1,5 +1,5 @@
-"""Argument checks of include/tg_fp8_train.h's entry points (no GPU): the header
-and the ctypes table agree, and bad calls are answered before any launch."""
+"""Argument checks of the entry points of include/tg_fp8_train.h and tg_fp8_prefill.h (no GPU): the headers
+and the ctypes tables agree, and bad calls are answered before any launch."""
 import re
 import os
 
@@ -10,9 +10,10 @@ BIG = 1 << 40
 
 
 def test_header_and_signatures_agree():
-    text = open(os.path.join(os.path.dirname(L.HEADER_PATH), "tg_fp8_train.h")).read()
-    names = set(re.findall(r"\b(tg_[a-z0-9_]+)\s*\(", re.sub(r"/\*.*?\*/", "", text, flags=re.S)))
-    assert names == set(L.TRAIN_SIGNATURES)
+    for header, table in (("tg_fp8_train.h", L.TRAIN_SIGNATURES), ("tg_fp8_prefill.h", L.PREFILL_SIGNATURES)):
+        text = open(os.path.join(os.path.dirname(L.HEADER_PATH), header)).read()
+        names = set(re.findall(r"\b(tg_[a-z0-9_]+)\s*\(", re.sub(r"/\*.*?\*/", "", text, flags=re.S)))
+        assert names == set(table)
 
 
 def _einval(rc, what):
@@ -34,3 +35,12 @@ def test_bad_calls():
     _einval(lib.tg_linear_bwd(N, 0, N, 0, N, 3, 256, 256, 4, 4, 128, N, BIG, N), "bf16 or f32")
     _einval(lib.tg_linear_bwd(256, 0, 256, 0, 256, 0, 256, 256, 4, 4, 128, 256, 0, N), "workspace too small")
     assert lib.tg_linear_bwd(N, 0, N, 0, N, 0, N, N, 4, 4, 128, N, 0, N) == L.TG_OK
+
+
+def test_prefill_kv_bad_calls():
+    lib = L.lib()
+    _einval(lib.tg_prefill_kv(N, N, N, 1, 4, 2, 8, 128, N), "null pointer")
+    _einval(lib.tg_prefill_kv(N, N, N, 1, 9, 2, 8, 128, N), "more rows")
+    _einval(lib.tg_prefill_kv(N, N, N, 1, 4, 2, 8, 100, N), "multiple of 8")
+    _einval(lib.tg_prefill_kv(N, N, N, -1, 4, 2, 8, 128, N), "bad shape")
+    assert lib.tg_prefill_kv(N, N, N, 0, 4, 2, 8, 128, N) == L.TG_OK

@@ -83,6 +83,11 @@ TRAIN_SIGNATURES = {
     "tg_linear_bwd": (_int, [_vp, _int, _vp, _int, _vp, _int, _vp, _vp, _i64, _i64, _i64, _vp, _sz, _vp]),
 }
 
+# include/tg_fp8_prefill.h: the decoder's prefill
+PREFILL_SIGNATURES = {
+    "tg_prefill_kv": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp]),
+}
+
 _lib = None
 
 
@@ -95,7 +100,7 @@ def lib():
                 f"{LIB_PATH} is missing: build it with `python train-gpt_amd/build.py` "
                 "(the FP8 hot path has no non-HIP implementation)")
         L = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in (*SIGNATURES.items(), *TRAIN_SIGNATURES.items()):
+        for name, (res, args) in (*SIGNATURES.items(), *TRAIN_SIGNATURES.items(), *PREFILL_SIGNATURES.items()):
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args

@@ -293,25 +293,30 @@ class FP8Decoder:
         self.length = 0
         self._graph = None
 
-    # -- one transformer block over the prompt rows x (B, T, d), positions 0 .. T-1 --
-    def _block(self, li: int, x: torch.Tensor) -> torch.Tensor:
+    # -- one transformer block over the prompt rows, positions 0 .. T-1 --
+    def _block(self, li: int, x: torch.Tensor, h_q: torch.Tensor, h_s: torch.Tensor, B: int):
+        """Layer li on the residual rows x (B T, d), which it adds its attention
+        term to in place, given norm1's FP8 rows of x.  Returns the MLP's term,
+        which the caller adds together with the next norm: both residual adds
+        (model.py:75-76) run inside the norm kernel after them, and relu^2 inside
+        the quantizer of w_down's input, with the bits of the separate ops."""
         cfg, lp = self.cfg, self.layers[li]
-        B, T, d = x.shape
+        T = x.shape[0] // B
         H, Dh = cfg.n_heads, cfg.head_dim
-        h, h_q, h_s = kernels.rms_norm_fp8(x, lp["norm1"], cfg.rms_eps)
-        qkv = lp["wqkv"].matmul_prequant(h_q.reshape(B * T, d), h_s.reshape(B * T, -1),
-                                       exact=self.exact_gemv)
+        qkv = lp["wqkv"].matmul_prequant(h_q, h_s, exact=self.exact_gemv)
         q, k, v = qkv.reshape(B, T, 3, H, Dh).permute(2, 0, 3, 1, 4).unbind(0)   # each (B, H, T, Dh)
-        self.k_cache[li, :B, :, :T] = k
-        self.v_cache[li, :B, :, :T] = v
+        kc, vc = self.k_cache[li], self.v_cache[li]
+        if Dh % 8 == 0:
+            _L.check(_L.lib().tg_prefill_kv(qkv.data_ptr(), kc.data_ptr(), vc.data_ptr(), B, T, H, kc.shape[2], Dh,
+                                            _L.stream_of(qkv)))
+        else:
+            kc[:B, :, :T] = k
+            vc[:B, :, :T] = v
         o = _attention(q, k, v, causal=True)                           # model.py:67
-        o = o.transpose(1, 2).reshape(B * T, H * Dh)
-        x = x + lp["wo"].matmul(o, exact=self.exact_gemv).reshape(B, T, d)   # model.py:68, 75
-        h2, h2_q, h2_s = kernels.rms_norm_fp8(x, lp["norm2"], cfg.rms_eps)
-        u = lp["w_up"].matmul_prequant(h2_q.reshape(B * T, d), h2_s.reshape(B * T, -1),
-                                        exact=self.exact_gemv)
-        u = F.relu(u).square()                                         # model.py:72 (bf16)
-        return x + lp["w_down"].matmul(u, exact=self.exact_gemv).reshape(B, T, d)   # model.py:76
+        a = lp["wo"].matmul(o.transpose(1, 2).reshape(B * T, H * Dh), exact=self.exact_gemv)     # model.py:68
+        _, h2_q, h2_s, _ = kernels.add_rms_norm_fp8(x, a, lp["norm2"], cfg.rms_eps, inplace=True)   # model.py:75
+        u = lp["w_up"].matmul_prequant(h2_q, h2_s, exact=self.exact_gemv)
+        return lp["w_down"].matmul_prequant(*fp8.quantize_relu2(u), exact=self.exact_gemv)           # model.py:71-73
 
     def _head(self, x: torch.Tensor) -> torch.Tensor:
         """Final norm -> FP8 unembedding -> logit cap (model.py:93-97); f32 (rows, V)."""
@@ -330,9 +335,18 @@ class FP8Decoder:
             raise ValueError(f"batch {B} exceeds max_batch={self.max_batch}")
         if not 1 <= T <= self.cfg.seq_len:
             raise ValueError(f"prompt length {T} must be in [1, seq_len={self.cfg.seq_len}]")
-        x = self.embed[ids] + self.pos[:T]                              # model.py:83
-        for li in range(self.cfg.n_layers):
-            x = self._block(li, x)
+        cfg = self.cfg
+        x = (self.embed[ids] + self.pos[:T]).reshape(B * T, cfg.d_model)   # model.py:83
+        if cfg.n_layers:
+            _, h_q, h_s = kernels.rms_norm_fp8(x, self.layers[0]["norm1"], cfg.rms_eps)
+        for li in range(cfg.n_layers):
+            m = self._block(li, x, h_q, h_s, B)
+            if li + 1 < cfg.n_layers:
+                # x = x + m (model.py:76) with the next layer's norm1
+                _, h_q, h_s, _ = kernels.add_rms_norm_fp8(x, m, self.layers[li + 1]["norm1"], cfg.rms_eps, inplace=True)
+            else:
+                x = x + m
+        x = x.reshape(B, T, cfg.d_model)
         self.length = T
         if all_logits:
             return self._head(x).reshape(B, T, -1)
