@@ -87,3 +87,22 @@ def test_decode_attention_rejects_bad_arguments(dev):
         decode.decode_attention(qkv, kc, vc, tt, 3)
     with pytest.raises(ValueError, match="one-element int64"):
         decode.decode_attention(qkv, kc, vc, tt.int(), 2)
+
+
+# a key raises the running maximum at every step, never after the first, or ties
+# it; t on both sides of a whole group of 64 keys and of a pair of groups
+@pytest.mark.parametrize("order", ["rising", "falling", "equal"])
+@pytest.mark.parametrize("t", [63, 64, 65, 128, 191, 700])
+def test_decode_attention_running_maximum(dev, order, t):
+    B, H, S = 1, 2, 768
+    qkv, kc, vc = _inputs(dev, B, H, S, seed=t)
+    q = qkv.reshape(B, 3, H, 128)[:, 0]
+    j = torch.arange(S, device=dev)[None, None, :, None]
+    step = {"rising": j, "falling": S - j, "equal": torch.full_like(j, S // 2)}[order].float() * (2.0 / S)
+    kc.copy_((q[:, :, None].float() * step).to(torch.bfloat16))
+    ref = _reference(qkv, kc, vc, t, H)
+    tt = torch.tensor([t], dtype=torch.long, device=dev)
+    _, _, o = decode.decode_attention(qkv, kc, vc, tt, H, want_bf16=True)
+    got = o.float().cpu().numpy().astype(np.float64)
+    tol = np.abs(ref) * 2.0 ** -6 + 1e-4 * np.max(np.abs(ref))   # as above
+    assert np.all(np.abs(got - ref) <= tol)

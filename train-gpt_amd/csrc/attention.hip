@@ -26,7 +26,7 @@ namespace tg {
 
 constexpr int kAttnDh = 128;
 constexpr int kAttnWaves = 4;
-constexpr int kAttnUnroll = 4;        // key groups in flight per wave
+constexpr int kAttnUnroll = 4;        // key slices per group
 
 __device__ __forceinline__ float row16_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));   // [1,0,3,2]
@@ -56,8 +56,60 @@ __device__ __forceinline__ void kv_load(KvGroup& G, const __amdgpu_buffer_rsrc_t
   }
 }
 
-// online-softmax update of a lane row with the keys of group G; keys past t
-// are skipped, key t is the new (k, v) from the projection output
+__device__ __forceinline__ float kv_score(const uint4& k, const float (&qf)[8], float scale) {
+  float d = qf[0] * bf16lo(k.x);
+  d = __builtin_fmaf(qf[1], bf16hi(k.x), d);
+  d = __builtin_fmaf(qf[2], bf16lo(k.y), d);
+  d = __builtin_fmaf(qf[3], bf16hi(k.y), d);
+  d = __builtin_fmaf(qf[4], bf16lo(k.z), d);
+  d = __builtin_fmaf(qf[5], bf16hi(k.z), d);
+  d = __builtin_fmaf(qf[6], bf16lo(k.w), d);
+  d = __builtin_fmaf(qf[7], bf16hi(k.w), d);
+  return row16_sum(d) * scale;
+}
+
+__device__ __forceinline__ void kv_accum(const uint4& v, float p, float (&acc)[8]) {
+  acc[0] = __builtin_fmaf(p, bf16lo(v.x), acc[0]);
+  acc[1] = __builtin_fmaf(p, bf16hi(v.x), acc[1]);
+  acc[2] = __builtin_fmaf(p, bf16lo(v.y), acc[2]);
+  acc[3] = __builtin_fmaf(p, bf16hi(v.y), acc[3]);
+  acc[4] = __builtin_fmaf(p, bf16lo(v.z), acc[4]);
+  acc[5] = __builtin_fmaf(p, bf16hi(v.z), acc[5]);
+  acc[6] = __builtin_fmaf(p, bf16lo(v.w), acc[6]);
+  acc[7] = __builtin_fmaf(p, bf16hi(v.w), acc[7]);
+}
+
+// The state (m, l, acc) rescaled to a maximum mn >= m.
+__device__ __forceinline__ void kv_rescale(float mn, float& m, float& l, float (&acc)[8]) {
+  const float corr = __expf(m - mn);
+  l *= corr;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] *= corr;
+  m = mn;
+}
+
+// Online-softmax update of a lane row with the keys of group G, all of them
+// before t: no key selection, and the rescaling (11 of 55 operations a key) only
+// when a key of the wave raises its row's maximum, a handful of times over a
+// context.  With an unchanged maximum the factor is exactly 1, so the bits are
+// the same.  Keys are taken one by one, each waiting for its own loads only (the
+// group's four scores first: 19.4 -> 21.8 us), and four groups in flight instead
+// of two gain nothing (20.1 us): a CU's stream of misses is the bound.  18 heads,
+// one sequence: t = 700 11.6 -> 10.2 us, t = 1900 24.0 -> 19.4 us.
+__device__ __forceinline__ void kv_step_full(const KvGroup& G, const float (&qf)[8], float scale, float& m, float& l,
+                                             float (&acc)[8]) {
+#pragma unroll
+  for (int u = 0; u < kAttnUnroll; ++u) {
+    const float sc = kv_score(G.k[u], qf, scale);
+    if (__any(sc > m)) kv_rescale(sc > m ? sc : m, m, l, acc);
+    const float p = __expf(sc - m);
+    l += p;
+    kv_accum(G.v[u], p, acc);
+  }
+}
+
+// The same for a group that holds key t or ends past it: keys past t are
+// skipped, key t is the new (k, v) from the projection output.
 __device__ __forceinline__ void kv_step(const KvGroup& G, int64_t i0, int64_t t, int wave, int kr,
                                         const float (&qf)[8], const uint4& knew, const uint4& vnew, float scale,
                                         float& m, float& l, float (&acc)[8]) {
@@ -65,28 +117,12 @@ __device__ __forceinline__ void kv_step(const KvGroup& G, int64_t i0, int64_t t,
   for (int u = 0; u < kAttnUnroll; ++u) {
     const int64_t j = (i0 + u) * (4 * kAttnWaves) + 4 * wave + kr;
     const uint4 k = j < t ? G.k[u] : knew, v = j < t ? G.v[u] : vnew;
-    float d = qf[0] * bf16lo(k.x);
-    d = __builtin_fmaf(qf[1], bf16hi(k.x), d);
-    d = __builtin_fmaf(qf[2], bf16lo(k.y), d);
-    d = __builtin_fmaf(qf[3], bf16hi(k.y), d);
-    d = __builtin_fmaf(qf[4], bf16lo(k.z), d);
-    d = __builtin_fmaf(qf[5], bf16hi(k.z), d);
-    d = __builtin_fmaf(qf[6], bf16lo(k.w), d);
-    d = __builtin_fmaf(qf[7], bf16hi(k.w), d);
-    const float sc = row16_sum(d) * scale;
+    const float sc = kv_score(k, qf, scale);
     if (j <= t) {                                        // uniform over the 16-lane row
-      const float mn = sc > m ? sc : m;
-      const float corr = __expf(m - mn), p = __expf(sc - mn);
-      l = l * corr + p;
-      acc[0] = __builtin_fmaf(p, bf16lo(v.x), acc[0] * corr);
-      acc[1] = __builtin_fmaf(p, bf16hi(v.x), acc[1] * corr);
-      acc[2] = __builtin_fmaf(p, bf16lo(v.y), acc[2] * corr);
-      acc[3] = __builtin_fmaf(p, bf16hi(v.y), acc[3] * corr);
-      acc[4] = __builtin_fmaf(p, bf16lo(v.z), acc[4] * corr);
-      acc[5] = __builtin_fmaf(p, bf16hi(v.z), acc[5] * corr);
-      acc[6] = __builtin_fmaf(p, bf16lo(v.w), acc[6] * corr);
-      acc[7] = __builtin_fmaf(p, bf16hi(v.w), acc[7] * corr);
-      m = mn;
+      kv_rescale(sc > m ? sc : m, m, l, acc);
+      const float p = __expf(sc - m);
+      l += p;
+      kv_accum(v, p, acc);
     }
   }
 }
@@ -130,22 +166,30 @@ __global__ __launch_bounds__(kAttnWaves * 64) void decode_attention_kernel(
 
   // online softmax over keys j = 16 i + 4 wave + kr (i = 0, 1, ...), j <= t;
   // two key groups in flight: the next group's loads go out before the
-  // current group's arithmetic (whole pairs in the loop, no exit inside it)
+  // current group's arithmetic (whole rounds in the loops, no exit inside)
   float m = -__builtin_inff(), l = 0.0f, acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-  const int64_t nk = t + 1;
-  const int64_t ngroups = (nk + 4 * kAttnWaves - 1) / (4 * kAttnWaves);
-  const int64_t nit = (ngroups + kAttnUnroll - 1) / kAttnUnroll;   // >= 1
-  int64_t i0 = 0;
-  for (int64_t p = 0; p + 1 < nit; p += 2) {
-    kv_load(B, rk, rv, i0 + kAttnUnroll, wave, kr, dl);
-    kv_step(A, i0, t, wave, kr, qf, knew, vnew, scale, m, l, acc);
-    kv_load(A, rk, rv, i0 + 2 * kAttnUnroll, wave, kr, dl);
-    kv_step(B, i0 + kAttnUnroll, t, wave, kr, qf, knew, vnew, scale, m, l, acc);
-    i0 += 2 * kAttnUnroll;
+  const int64_t nfull = t / (4 * kAttnWaves * kAttnUnroll);        // groups of keys before t
+  auto load = [&](KvGroup& G, int64_t g) { kv_load(G, rk, rv, g * kAttnUnroll, wave, kr, dl); };
+  auto full = [&](const KvGroup& G) { kv_step_full(G, qf, scale, m, l, acc); };
+  auto last = [&](const KvGroup& G) {                              // group nfull: key t and past it
+    kv_step(G, nfull * kAttnUnroll, t, wave, kr, qf, knew, vnew, scale, m, l, acc);
+  };
+  int64_t p = 0;
+  for (; p + 2 <= nfull; p += 2) {
+    load(B, p + 1);
+    full(A);
+    load(A, p + 2);
+    full(B);
   }
-  if (nit & 1) kv_step(A, i0, t, wave, kr, qf, knew, vnew, scale, m, l, acc);
+  if (p < nfull) {
+    load(B, p + 1);
+    full(A);
+    last(B);
+  } else {
+    last(A);
+  }
 
   // merge the 16 partial states (4 key rows x 4 waves) in a fixed order
   __shared__ float sm[16], sl[16];
@@ -233,7 +277,7 @@ __global__ __launch_bounds__(256) void decode_embed_kernel(const uint16_t* __res
 // k and v of a prompt's projection rows (B T, 3 H Dh) into the caches
 // (B, H, S, Dh) at positions 0 .. T - 1: one 16-byte piece per thread, read in
 // row order, written as whole rows of a head.  512 rows of 18 heads of 128: 9.4 MB
-// each way in one launch of 5 us (two strided copies took 5.7 us each).
+// each way in one launch of 4.4 us (two strided copies took 5.7 us each).
 __global__ __launch_bounds__(256) void prefill_kv_kernel(const uint4* __restrict__ qkv, uint4* __restrict__ kc,
                                                          uint4* __restrict__ vc, int64_t n, int T, int H, int64_t S,
                                                          int dc) {

@@ -6,7 +6,7 @@
 // operands whose contraction is padded to whole blocks, so nothing is copied to
 // a padded tensor first (3000 x 2304 x 9216, forward and backward: three fills,
 // three copies and two slices, 72 us, and five quantizer launches, 48 us, are
-// two launches of 58 us).  f32 operands go through the same tiles.
+// two launches of 56 us).  f32 operands go through the same tiles.
 #include "tg_device.h"
 #include "tg_host.h"
 #include "../../include/tg_fp8_train.h"
