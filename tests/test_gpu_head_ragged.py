@@ -52,6 +52,21 @@ def test_gemm_bf16_ragged_rows_of_c(dev, M, N, off):
     assert bool((buf[:8 + off] == 9.0).all()) and bool((buf[8 + off + M * N:] == 9.0).all())
 
 
+# 192-wide tiles (few of them) at their edges, and 256-wide ones (a whole round);
+# 2, 6 and 10 slices of the four-stage ring
+@pytest.mark.parametrize("M,N,K", [(1, 192, 64), (255, 191, 64), (256, 200, 192), (257, 193, 192), (130, 384, 320),
+                                   (300, 576, 64), (4096, 4096, 64), (4090, 4089, 64)])
+def test_gemm_bf16_tile_widths(dev, M, N, K):
+    """Exact integer products, every value of C written and nothing past it."""
+    a = ((np.arange(M)[:, None] * 3 + np.arange(K)) % 5 - 2).astype(np.float32)
+    b = ((np.arange(N)[:, None] * 5 + 2 * np.arange(K)) % 7 - 3).astype(np.float32)
+    ta, tb = to_dev(ob.f32_to_bf16(a), dev), to_dev(ob.f32_to_bf16(b), dev)
+    buf = torch.full((M * N + 64,), 0.5, dtype=torch.bfloat16, device=dev)
+    L.check(L.lib().tg_gemm_bf16_nt(L.ptr(ta), L.ptr(tb), L.ptr(buf), M, N, K, L.stream_of(ta)))
+    assert np.array_equal(bf16_bits(buf[:M * N].reshape(M, N)), ob.f32_to_bf16((a @ b.T).astype(np.float32)))
+    assert bool((buf[M * N:] == 0.5).all())
+
+
 # dX contracts N, dW contracts M: each splits where its 256 x 256 tiles are few
 # and the contraction long (down to 16 slices of 32 per split, a last split shorter)
 @pytest.mark.parametrize("M,K,N", [(33, 256, 5001), (2049, 128, 72), (700, 384, 1025), (4100, 256, 264),

@@ -11,7 +11,11 @@
 //   * v_mfma_f32_16x16x32_bf16, accumulating in place: no per-block scales,
 //     so the K loop is MFMA work only.
 //   * Workgroup tile 256 x 256, 8 waves as 4 (M) x 2 (N), wave tile 64 x 128
-//     = 4 x 8 MFMA tiles, 128 fp32 accumulators per lane.
+//     = 4 x 8 MFMA tiles, 128 fp32 accumulators per lane; 256 x 192 (wave tile
+//     64 x 96) where 256-wide tiles would leave more CUs idle (q4_split_of).
+//     Four waves of 128 x 128 read a third less LDS per product but are no
+//     faster (0.59 against 0.58 us per slice): one wave per SIMD has nothing
+//     to run at a wait, and 256 accumulators fill the accumulation registers.
 //   * Operands travel HBM -> LDS by buffer_load ... lds through a ring of four
 //     K32 stages (one barrier per stage), issued by one wave per SIMD.
 //   * dW contracts over the token axis, which is the row axis of both a and
@@ -34,18 +38,19 @@ __device__ __forceinline__ v4f mfma_bf16_16x16x32(const uint4& a, const uint4& b
 
 // ---------------------------------------------------------------------------
 // Four-stage pipeline.  A stage is one K32 slice of the workgroup tile: 256
-// rows x 64 B of A and of B, 32 KiB; four stages ring through 128 KiB of LDS,
-// so three slices (96 KiB per CU) are in flight while one is computed.  (With
+// rows x 64 B of A and of B (192 of B for the narrow tile), 32 KiB; four stages
+// ring through 128 KiB of LDS, so three slices (96 KiB per CU) are in flight
+// while one is computed.  (With
 // two stages of K64, one 64 KiB step in flight, the copy stream was capped by
 // the ~1.4 us round trip to L2 / Infinity Cache at ~45 B/ns per CU; the MFMAs
 // consume a K64 step in ~0.9 us.)
-//   step s: loader waves wait for their copies of slice s (vmcnt(16): the 16
-//           DMA instructions of slices s+1 and s+2 stay outstanding); barrier
+//   step s: loader waves wait for their copies of slice s (vmcnt(16), narrow
+//           14: the copies of slices s+1 and s+2 stay outstanding); barrier
 //           (slice s complete, slice s-1 read by every wave); the loader waves
 //           issue slice s+3 into slice s-1's stage; every wave computes s.
-// Loads: waves 0-3 (one per SIMD) issue all copies, 8 per slice (rows
-// 64w .. 64w+63 of A and of B), so the other wave of each SIMD never stalls at
-// a DMA issue; loader and compute waves run separate copies of the loop.  The
+// Loads: waves 0-3 (one per SIMD) issue all copies, 8 (narrow: 7) per slice
+// (a quarter of the rows of A and of B), so the other wave of each SIMD never
+// stalls at a DMA issue; loader and compute waves run separate copies of the loop.  The
 // copies are issued unconditionally: past the last slice the offset is out of
 // range and the loads read zero, which keeps the vmcnt arithmetic exact.  The
 // main loop runs whole rounds of four slices with no exit inside (with exits,
@@ -96,9 +101,9 @@ struct Q4Ctx {
 __device__ __forceinline__ uint32_t tn_swz(uint32_t r) { return ((r & 3u) | (((r >> 3) & 1u) << 2)) << 1; }
 
 // slice ks into the stage at (la, lb).  NT: loader wave w fills rows
-// 64w .. 64w+63 of A and of B, 16 rows per instruction; TN: contraction rows
-// 8w .. 8w+7, 2 rows per instruction.
-template <bool LOADER, bool TN>
+// 64w .. 64w+63 of A and its quarter of B's 32 NJ rows, 16 rows per instruction;
+// TN: contraction rows 8w .. 8w+7, 2 rows per instruction.
+template <bool LOADER, bool TN, int NJ>
 __device__ __forceinline__ void q4_issue(const Q4Ctx& c, uint8_t* la, uint8_t* lb, int ks) {
   if (!LOADER) return;
   if constexpr (TN) {
@@ -116,8 +121,9 @@ __device__ __forceinline__ void q4_issue(const Q4Ctx& c, uint8_t* la, uint8_t* l
     for (int p = 0; p < 4; ++p) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(c.ra, la + c.wave * 4096 + p * 1024, 16, c.voa,
                                                so + p * c.row16, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(c.rb, lb + c.wave * 4096 + p * 1024, 16, c.vob,
-                                               so + p * c.row16, 0, 0);
+      if (p < NJ / 2)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(c.rb, lb + c.wave * (NJ * 512) + p * 1024, 16, c.vob,
+                                                 so + p * c.row16, 0, 0);
     }
   }
 }
@@ -143,21 +149,22 @@ __device__ __forceinline__ uint4 tn_frag(const uint8_t* l, const Q4Ctx& c, uint3
                     ((uint32_t)(uint16_t)hi[2]) | ((uint32_t)(uint16_t)hi[3] << 16));
 }
 
-// s_waitcnt vmcnt(16) lgkmcnt(0), and lgkmcnt(0) alone, as the builtin (gfx9
+// s_waitcnt vmcnt(n) lgkmcnt(0), and lgkmcnt(0) alone, as the builtin (gfx9
 // encoding: vmcnt bits 3:0 and 15:14, expcnt not waited), which the compiler's
 // own wait insertion takes into account; an inline-asm wait is opaque to it.
 // lgkmcnt: a wave's reads of slice ks - 1 have left LDS before a loader, past
 // the barrier, refills that stage (the refills past the last slice return their
 // zeros at once, without a trip to memory).
-constexpr int kWaitVm16 = (1 << 14) | (0x7 << 4);
+constexpr int wait_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (0x7 << 4); }
 constexpr int kWaitLds = (3 << 14) | (0x7 << 4) | 0xF;
 
-template <int S, bool LOADER, bool TN>
-__device__ __forceinline__ void q4_step(const Q4Ctx& c, int ks, v4f (&acc)[4][8]) {
-  __builtin_amdgcn_s_waitcnt(LOADER ? kWaitVm16 : kWaitLds);
+template <int S, bool LOADER, bool TN, int NJ>
+__device__ __forceinline__ void q4_step(const Q4Ctx& c, int ks, v4f (&acc)[4][NJ]) {
+  constexpr int kCopies = 4 + NJ / 2;    // a loader wave's per slice
+  __builtin_amdgcn_s_waitcnt(LOADER ? wait_vm(2 * kCopies) : kWaitLds);
   __builtin_amdgcn_s_barrier();
   constexpr int kRefill = (S + 3) & 3;   // the stage slice ks - 1 occupied
-  q4_issue<LOADER, TN>(c, q4_a<kRefill>(), q4_b<kRefill>(), ks + 3);
+  q4_issue<LOADER, TN, NJ>(c, q4_a<kRefill>(), q4_b<kRefill>(), ks + 3);
   const uint8_t* la = q4_a<S>();
   const uint8_t* lb = q4_b<S>();
   uint4 af[4];
@@ -166,58 +173,59 @@ __device__ __forceinline__ void q4_step(const Q4Ctx& c, int ks, v4f (&acc)[4][8]
     af[i] = TN ? tn_frag(la, c, c.tca, i) : *reinterpret_cast<const uint4*>(la + c.fa + i * 1024);
   uint4 bn = TN ? tn_frag(lb, c, c.tcb, 0) : *reinterpret_cast<const uint4*>(lb + c.fb);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < NJ; ++j) {
     const uint4 bf = bn;
-    if (j + 1 < 8)
+    if (j + 1 < NJ)
       bn = TN ? tn_frag(lb, c, c.tcb, j + 1) : *reinterpret_cast<const uint4*>(lb + c.fb + (j + 1) * 1024);
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i][j] = mfma_bf16_16x16x32(bf, af[i], acc[i][j]);
   }
 }
 
-template <bool LOADER, bool TN>
-__device__ __forceinline__ void q4_main_loop(const Q4Ctx& c, v4f (&acc)[4][8]) {
-  q4_issue<LOADER, TN>(c, q4_a0, q4_b0, 0);
-  q4_issue<LOADER, TN>(c, q4_a1, q4_b1, 1);
-  q4_issue<LOADER, TN>(c, q4_a2, q4_b2, 2);
+template <bool LOADER, bool TN, int NJ>
+__device__ __forceinline__ void q4_main_loop(const Q4Ctx& c, v4f (&acc)[4][NJ]) {
+  q4_issue<LOADER, TN, NJ>(c, q4_a0, q4_b0, 0);
+  q4_issue<LOADER, TN, NJ>(c, q4_a1, q4_b1, 1);
+  q4_issue<LOADER, TN, NJ>(c, q4_a2, q4_b2, 2);
   int ks = 0;
   for (; ks + 4 <= c.nks; ks += 4) {
-    q4_step<0, LOADER, TN>(c, ks, acc);
-    q4_step<1, LOADER, TN>(c, ks + 1, acc);
-    q4_step<2, LOADER, TN>(c, ks + 2, acc);
-    q4_step<3, LOADER, TN>(c, ks + 3, acc);
+    q4_step<0, LOADER, TN, NJ>(c, ks, acc);
+    q4_step<1, LOADER, TN, NJ>(c, ks + 1, acc);
+    q4_step<2, LOADER, TN, NJ>(c, ks + 2, acc);
+    q4_step<3, LOADER, TN, NJ>(c, ks + 3, acc);
   }
   if (ks < c.nks) {
-    q4_step<0, LOADER, TN>(c, ks, acc);
+    q4_step<0, LOADER, TN, NJ>(c, ks, acc);
     if (ks + 1 < c.nks) {
-      q4_step<1, LOADER, TN>(c, ks + 1, acc);
-      if (ks + 2 < c.nks) q4_step<2, LOADER, TN>(c, ks + 2, acc);
+      q4_step<1, LOADER, TN, NJ>(c, ks + 1, acc);
+      if (ks + 2 < c.nks) q4_step<2, LOADER, TN, NJ>(c, ks + 2, acc);
     }
   }
 }
 
-// R rows of 128 bf16 from LDS (256-byte rows, chunk c of row r at
-// c ^ (r & 15)), rows r0 .. r0 + R - 1, to C rows mw + r, columns nw .. nw + 127,
-// by one wave.  Rows of N % 8 == 0 go out as 16-byte pieces, 16 lanes per row.
-// Other rows start at any even address: one row per instruction as 64
-// consecutive 4-byte words from its first 4-byte boundary, and a single value
+// R rows of W = 16 NJ bf16 from LDS (256-byte rows, chunk c of row r at
+// c ^ (r & 15)) to C rows mw + r, columns nw .. nw + W - 1, by one wave; r0 is
+// the first row.  Rows of N % 8 == 0 go out as 16-byte pieces, W / 8 lanes per
+// row.  Other rows start at any even address: one row per instruction as up to
+// 64 consecutive 4-byte words from its first 4-byte boundary, and a single value
 // at either end where one is left over (2-byte stores of whole pieces touched
 // every line eight times).
-template <int R, int PITCH>
+template <int R, int NJ>
 __device__ __forceinline__ void q4_store_rows(const uint8_t* l, __bf16* __restrict__ C, int M, int N, int mw, int nw,
                                               int lane, int r0) {
+  constexpr int PITCH = 256, kRow = 2 * NJ;   // 16-byte pieces per row
   if (N % 8 == 0) {
-    const int k = lane & 15;
 #pragma unroll
-    for (int q = 0; q < R / 4; ++q) {
-      const int r = r0 + q * 4 + (lane >> 4);
+    for (int q = 0; q < R * kRow / 64; ++q) {
+      const int o = q * 64 + lane;
+      const int r = r0 + o / kRow, k = o % kRow;
       const int m = mw + r, n = nw + k * 8;
       const uint4 v = *reinterpret_cast<const uint4*>(l + r * PITCH + ((k ^ (r & 15)) * 16));
       if (m < M && n < N) *reinterpret_cast<uint4*>(C + (int64_t)m * N + n) = v;
     }
     return;
   }
-  const int cnt = min(128, N - nw);
+  const int cnt = min(16 * NJ, N - nw);
   if (cnt <= 0) return;
   auto at = [&](int r, int e) {
     return *reinterpret_cast<const uint16_t*>(l + r * PITCH + (((e >> 3) ^ (r & 15)) * 16) + (e & 7) * 2);
@@ -236,11 +244,11 @@ __device__ __forceinline__ void q4_store_rows(const uint8_t* l, __bf16* __restri
   }
 }
 
-// Epilogue of the 256 x 256 bf16 kernels: lane (fr, fg) holds row i * 16 + fr
-// and columns j * 16 + 4 fg .. +3 of the wave tile; stage it in this wave's
-// 16 KiB (256-byte rows, chunk c of row r at c ^ (r & 15)), then 16 lanes
-// store each row's 256 bytes.
-__device__ __forceinline__ void q4_store_tile(const v4f (&acc)[4][8], __bf16* __restrict__ C, int M, int N, int m0,
+// Epilogue: lane (fr, fg) holds row i * 16 + fr and columns j * 16 + 4 fg .. +3
+// of the wave tile; stage it in this wave's 16 KiB (256-byte rows, chunk c of
+// row r at c ^ (r & 15)), then store whole rows.
+template <int NJ>
+__device__ __forceinline__ void q4_store_tile(const v4f (&acc)[4][NJ], __bf16* __restrict__ C, int M, int N, int m0,
                                               int n0, int wm, int wn, int wave, int lane) {
   const int fr = lane & 15, fg = lane >> 4;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -250,7 +258,7 @@ __device__ __forceinline__ void q4_store_tile(const v4f (&acc)[4][8], __bf16* __
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       const int r = i * 16 + fr;
       const int chunk = (j * 2 + (fg >> 1)) ^ (r & 15);
       const v4f v = acc[i][j];
@@ -258,57 +266,59 @@ __device__ __forceinline__ void q4_store_tile(const v4f (&acc)[4][8], __bf16* __
           make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  q4_store_rows<64, 256>(wbuf, C, M, N, m0 + wm * 64, n0 + wn * 128, lane, 0);
+  q4_store_rows<64, NJ>(wbuf, C, M, N, m0 + wm * 64, n0 + wn * (16 * NJ), lane, 0);
 }
 
 // Split-K: the workgroup's f32 tile in register order, one contiguous 8 KiB
 // per (i, j), for q4_reduce_kernel.  The copies issued past the last slice
 // still write LDS, so they are waited for before the wave ends.
-__device__ __forceinline__ void q4_store_part(const v4f (&acc)[4][8], float* __restrict__ part) {
-  float4* p = reinterpret_cast<float4*>(part) + (size_t)blockIdx.x * (32 * 512) + threadIdx.x;
+template <int NJ>
+__device__ __forceinline__ void q4_store_part(const v4f (&acc)[4][NJ], float* __restrict__ part) {
+  float4* p = reinterpret_cast<float4*>(part) + (size_t)blockIdx.x * (4 * NJ * 512) + threadIdx.x;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      p[(i * 8 + j) * 512] = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+    for (int j = 0; j < NJ; ++j)
+      p[(i * NJ + j) * 512] = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // Sum of the splits' partial tiles in split order, rounded once to bf16.  One
-// workgroup per 64 x 128 wave tile (8 per 256 x 256 tile): wave i sums the
+// workgroup per wave tile (8 per workgroup tile): wave i sums the
 // fragments of rows 16 i .. +15 as the GEMM's lanes held them, and the bf16
-// rows leave through LDS as whole 256-byte pieces.
+// rows leave through LDS as whole pieces.
+template <int NJ>
 __global__ __launch_bounds__(256) void q4_reduce_kernel(const float4* __restrict__ part, __bf16* __restrict__ C,
                                                         int M, int N, int tiles_m, int tiles_n, int nsplit) {
   __shared__ __attribute__((aligned(16))) uint8_t rows[64 * 256];
   const int tile = blockIdx.x >> 3, w = blockIdx.x & 7;
   int tmi, tni;
   tile_of(tile, tiles_m, tiles_n, tmi, tni);
-  const int mw = tmi * 256 + (w >> 1) * 64, nw = tni * 256 + (w & 1) * 128;
+  const int mw = tmi * 256 + (w >> 1) * 64, nw = tni * (32 * NJ) + (w & 1) * (16 * NJ);
   if (mw >= M || nw >= N) return;
   const int lane = threadIdx.x & 63, i = threadIdx.x >> 6, fr = lane & 15, fg = lane >> 4;
   const size_t ntiles = (size_t)tiles_m * tiles_n;
-  const float4* p = part + ((size_t)tile * 32 + i * 8) * 512 + w * 64 + lane;
-  float4 t[8];
+  const float4* p = part + ((size_t)tile * (4 * NJ) + i * NJ) * 512 + w * 64 + lane;
+  float4 t[NJ];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) t[j] = p[j * 512];
+  for (int j = 0; j < NJ; ++j) t[j] = p[j * 512];
   for (int s = 1; s < nsplit; ++s) {
-    p += ntiles * (32 * 512);
-    float4 v[8];
+    p += ntiles * (4 * NJ * 512);
+    float4 v[NJ];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = p[j * 512];
+    for (int j = 0; j < NJ; ++j) v[j] = p[j * 512];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       t[j].x += v[j].x; t[j].y += v[j].y; t[j].z += v[j].z; t[j].w += v[j].w;
     }
   }
   const int r = i * 16 + fr;
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
+  for (int j = 0; j < NJ; ++j)
     *reinterpret_cast<uint2*>(rows + r * 256 + (((j * 2 + (fg >> 1)) ^ (r & 15)) * 16) + (fg & 1) * 8) =
         make_uint2(pack_bf16x2(t[j].x, t[j].y), pack_bf16x2(t[j].z, t[j].w));
   __syncthreads();
-  q4_store_rows<16, 256>(rows, C, M, N, mw, nw, lane, 16 * i);
+  q4_store_rows<16, NJ>(rows, C, M, N, mw, nw, lane, 16 * i);
 }
 
 // The K slices of this workgroup's split: first slice and count (per slices
@@ -321,6 +331,7 @@ __device__ __forceinline__ int q4_split(int nks, int tiles_m, int tiles_n, int n
   return (int)blockIdx.x - sp * ntiles;
 }
 
+template <int NJ>
 __global__ __launch_bounds__(512, 1) void gemm_bf16_nt_q4_kernel(const __bf16* __restrict__ A,
                                                                  const __bf16* __restrict__ B,
                                                                  __bf16* __restrict__ C, int M, int N,
@@ -335,31 +346,31 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_nt_q4_kernel(const __bf16* _
   const int wm = c.wave >> 1, wn = c.wave & 1;
   int tmi, tni;
   tile_of(slot, tiles_m, tiles_n, tmi, tni);
-  const int m0 = tmi * 256, n0 = tni * 256;
+  const int m0 = tmi * 256, n0 = tni * (32 * NJ);
   const uint32_t rowb = 2u * (uint32_t)K;
   c.ra = make_rsrc(A, (uint32_t)M * rowb);
   c.rb = make_rsrc(B, (uint32_t)N * rowb);
   c.row16 = 16u * rowb;
   // DMA lane L lands at byte 16 L of its 1 KiB slot: row slot + L / 4,
   // physical chunk L % 4, which holds logical chunk (L % 4) ^ ((L >> 3) & 3)
-  const int lrow = c.wave * 64 + (lane >> 2);   // loader waves 0-3
+  const int lrow = lane >> 2;   // loader waves 0-3
   const uint32_t lch = (uint32_t)((lane & 3) ^ ((lane >> 3) & 3)) * 16u;
-  c.voa = (uint32_t)(m0 + lrow) * rowb + lch + (uint32_t)ks0 * 64u;
-  c.vob = (uint32_t)(n0 + lrow) * rowb + lch + (uint32_t)ks0 * 64u;
+  c.voa = (uint32_t)(m0 + c.wave * 64 + lrow) * rowb + lch + (uint32_t)ks0 * 64u;
+  c.vob = (uint32_t)(n0 + c.wave * (8 * NJ) + lrow) * rowb + lch + (uint32_t)ks0 * 64u;
   // fragment: lane (fr, fg) reads logical chunk fg (k 8fg .. 8fg+7) of row
   // (wave tile row) + 16 t + fr, at physical chunk fg ^ ((fr >> 1) & 3)
   const uint32_t ch = (uint32_t)(fg ^ ((fr >> 1) & 3)) * 16u;
   c.fa = (uint32_t)(wm * 64 + fr) * 64u + ch;
-  c.fb = (uint32_t)(wn * 128 + fr) * 64u + ch;
+  c.fb = (uint32_t)(wn * (16 * NJ) + fr) * 64u + ch;
 
-  v4f acc[4][8];
+  v4f acc[4][NJ];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NJ; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  if (c.wave < 4) q4_main_loop<true, false>(c, acc);
-  else q4_main_loop<false, false>(c, acc);
+  if (c.wave < 4) q4_main_loop<true, false, NJ>(c, acc);
+  else q4_main_loop<false, false, NJ>(c, acc);
 
   if (nsplit > 1) q4_store_part(acc, part);
   else q4_store_tile(acc, C, M, N, m0, n0, wm, wn, c.wave, lane);
@@ -422,8 +433,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_tn_q4_kernel(const __bf16* _
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  if (c.wave < 4) q4_main_loop<true, true>(c, acc);
-  else q4_main_loop<false, true>(c, acc);
+  if (c.wave < 4) q4_main_loop<true, true, 8>(c, acc);
+  else q4_main_loop<false, true, 8>(c, acc);
 
   if (nsplit > 1) q4_store_part(acc, part);
   else q4_store_tile(acc, C, M, N, m0, n0, wm, wn, c.wave, lane);
@@ -673,43 +684,58 @@ int launch_fill_zero_bf16(void* p, int64_t n, hipStream_t st) {
   return check_launch("fill_zero_bf16");
 }
 
-// Split of a contraction of nks 32-wide slices over workgroups, for outputs
-// whose 256 x 256 tiles leave CUs idle (a head's dX at 2048 x 2304: 72 tiles
-// on 256 CUs) or fill a last round badly.
+// Tile width, and the split of a contraction of nks 32-wide slices over
+// workgroups, for outputs whose 256 x 256 tiles leave CUs idle (a head's dX at
+// 2048 x 2304: 72 tiles on 256 CUs) or fill a last round badly.
 struct Q4Split {
   int n, per;   // splits, slices per split
+  int nj;       // tile width / 32: 8 (256 columns) or 6 (192, NT operands only)
 };
-// The split with the least modelled time, in slices (~0.5 us each): rounds of
-// 256 workgroups times a split's slices plus 8 for its first round trip and
-// its tile's store, and for n > 1 the partial tiles written and read back
-// (8 bytes per output and split at ~5 TB/s) and the reduction's launch.
-// Measured: dX 2048 x 2304 over 50304, three splits on 216 CUs, 1219 us on 72
-// CUs -> 479 + 12 (reduction); dX 4096 x 2304 over 6912 (144 tiles, 176 us)
-// stays whole: three splits would move 226 MB of partial tiles.  A function of the shape alone: the workspace size and the launch agree on
+// The choice with the least modelled time, in slices of the 256-wide tile
+// (~0.5 us each; one of the 192-wide tile, three quarters of the matrix work but
+// ten twelfths of the fragment reads, takes 0.84 of it): rounds of 256 workgroups
+// times a split's slices plus 8 for its first round trip and its tile's store,
+// and for n > 1 the partial tiles written and read back (8 bytes per output and
+// split at ~5 TB/s) and the reduction's launch.  Measured:
+//   4096 x 2304 over 6912   144 tiles 142 us, 192 narrow ones 122; three splits
+//                           would move 226 MB of partial tiles
+//   512 x 768 over 3072     63 -> 54 us
+//   4096 x 4096 over 4096   256 tiles 109 us, 352 narrow ones 152
+//   2048 x 50304 over 2304  1576 tiles 466 us, 2096 narrow ones 492
+//   2048 x 2304 over 50304  72 tiles 1219 us, three splits of them 479 + 12
+//                           (reduction)
+// A function of the shape alone: the workspace size and the launch agree on
 // every device, and the split (so the sum's order) is the same on every call.
-static Q4Split q4_split_of(int64_t M, int64_t N, int64_t Kc) {
-  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), nks = (Kc + 31) / 32;
-  Q4Split best{1, (int)nks};
+// The width does not change a result: every output sums its slices in order.
+static int64_t q4_tiles(int64_t M, int64_t N, int nj) { return ((M + 255) / 256) * ((N + 32 * nj - 1) / (32 * nj)); }
+static Q4Split q4_split_of(int64_t M, int64_t N, int64_t Kc, bool tn, int max_split) {
+  const int64_t nks = (Kc + 31) / 32;
+  Q4Split best{1, (int)nks, 8};
   double cost = 1e300;
-  for (int64_t n = 1; n <= 16; ++n) {
-    const int64_t per = (nks + n - 1) / n;
-    if (n > 1 && (per < 16 || (nks + per - 1) / per != n)) continue;
-    const double c = (double)((tiles * n + 255) / 256) * (double)(per + 8) +
-                     (n > 1 ? 6.0 + (double)(tiles * n) * (65536.0 * 8.0 / 2.5e6) : 0.0);
-    if (c < cost * 0.97) {
-      cost = c;
-      best = Q4Split{(int)n, (int)per};
+  for (int nj = 8; nj >= (tn ? 8 : 6); nj -= 2) {
+    const int64_t tiles = q4_tiles(M, N, nj);
+    const double rel = nj == 8 ? 1.0 : 0.84;   // a slice's time
+    for (int64_t n = 1; n <= max_split; ++n) {
+      const int64_t per = (nks + n - 1) / n;
+      if (n > 1 && (per < 16 || (nks + per - 1) / per != n)) continue;
+      const double c = (double)((tiles * n + 255) / 256) * ((double)per * rel + 8) +
+                       (n > 1 ? 6.0 + (double)(tiles * n) * (8192.0 * nj * 8.0 / 2.5e6) : 0.0);
+      if (c < cost * 0.97) {
+        cost = c;
+        best = Q4Split{(int)n, (int)per, nj};
+      }
     }
   }
   return best;
 }
 static size_t q4_part_bytes(const Q4Split& sp, int64_t M, int64_t N) {
-  return sp.n > 1 ? (size_t)sp.n * (size_t)(((M + 255) / 256) * ((N + 255) / 256)) * 65536 * 4 : 0;
+  return sp.n > 1 ? (size_t)sp.n * (size_t)q4_tiles(M, N, sp.nj) * (size_t)(8192 * sp.nj) * 4 : 0;
 }
 
+template <int NJ>
 static int launch_q4_reduce(const float* part, __bf16* c, int64_t M, int64_t N, int tiles_m, int tiles_n, int n,
                             hipStream_t st) {
-  hipLaunchKernelGGL(q4_reduce_kernel, dim3((unsigned)(tiles_m * tiles_n * 8)), dim3(256), 0, st,
+  hipLaunchKernelGGL(q4_reduce_kernel<NJ>, dim3((unsigned)(tiles_m * tiles_n * 8)), dim3(256), 0, st,
                      reinterpret_cast<const float4*>(part), c, (int)M, (int)N, tiles_m, tiles_n, n);
   return check_launch("gemm_bf16_reduce");
 }
@@ -722,18 +748,24 @@ int launch_gemm_bf16_tn(const __bf16* a, int64_t lda, const __bf16* b, int64_t l
   const int tiles_m = (int)((M + 255) / 256), tiles_n = (int)((N + 255) / 256);
   hipLaunchKernelGGL(gemm_bf16_tn_q4_kernel, dim3((unsigned)(tiles_m * tiles_n * sp.n)), dim3(512), 0, st, a, b, c,
                      (int)M, (int)N, (int)Kc, (int)lda, (int)ldb, tiles_m, tiles_n, sp.n, sp.per, part);
-  TG_TRY(check_launch("gemm_bf16_tn_256"));
-  return sp.n > 1 ? launch_q4_reduce(part, c, M, N, tiles_m, tiles_n, sp.n, st) : TG_OK;
+  TG_TRY(check_launch("gemm_bf16_tn"));
+  return sp.n > 1 ? launch_q4_reduce<8>(part, c, M, N, tiles_m, tiles_n, sp.n, st) : TG_OK;
+}
+
+template <int NJ>
+static int launch_q4_nt(const __bf16* a, const __bf16* b, __bf16* c, int64_t M, int64_t N, int64_t K,
+                        const Q4Split& sp, float* part, hipStream_t st) {
+  const int tiles_m = (int)((M + 255) / 256), tiles_n = (int)((N + 32 * NJ - 1) / (32 * NJ));
+  hipLaunchKernelGGL(gemm_bf16_nt_q4_kernel<NJ>, dim3((unsigned)(tiles_m * tiles_n * sp.n)), dim3(512), 0, st,
+                     a, b, c, (int)M, (int)N, (int)K, tiles_m, tiles_n, sp.n, sp.per, part);
+  TG_TRY(check_launch("gemm_bf16_nt"));
+  return sp.n > 1 ? launch_q4_reduce<NJ>(part, c, M, N, tiles_m, tiles_n, sp.n, st) : TG_OK;
 }
 
 int launch_gemm_bf16(const __bf16* a, const __bf16* b, __bf16* c, int64_t M, int64_t N, int64_t K,
                      const Q4Split& sp, float* part, hipStream_t st) {
   if (M == 0 || N == 0) return TG_OK;
-  const int tiles_m = (int)((M + 255) / 256), tiles_n = (int)((N + 255) / 256);
-  hipLaunchKernelGGL(gemm_bf16_nt_q4_kernel, dim3((unsigned)(tiles_m * tiles_n * sp.n)), dim3(512), 0, st,
-                     a, b, c, (int)M, (int)N, (int)K, tiles_m, tiles_n, sp.n, sp.per, part);
-  TG_TRY(check_launch("gemm_bf16_nt_256"));
-  return sp.n > 1 ? launch_q4_reduce(part, c, M, N, tiles_m, tiles_n, sp.n, st) : TG_OK;
+  return sp.nj == 8 ? launch_q4_nt<8>(a, b, c, M, N, K, sp, part, st) : launch_q4_nt<6>(a, b, c, M, N, K, sp, part, st);
 }
 
 }  // namespace tg
@@ -760,7 +792,7 @@ extern "C" int tg_gemm_bf16_nt(const void* a, const void* b, void* c, int64_t M,
   if (!a || !b || !c) return einval("gemm_bf16_nt: null pointer");
   if (!aligned(a, 16) || !aligned(b, 16)) return einval("gemm_bf16_nt: operands must be 16-byte aligned");
   return launch_gemm_bf16(reinterpret_cast<const __bf16*>(a), reinterpret_cast<const __bf16*>(b),
-                          reinterpret_cast<__bf16*>(c), M, N, K, Q4Split{1, (int)(K / 32)}, nullptr,
+                          reinterpret_cast<__bf16*>(c), M, N, K, q4_split_of(M, N, K, false, 1), nullptr,
                           as_stream(stream));
 }
 
@@ -779,8 +811,8 @@ extern "C" int tg_pack_bf16(const void* x, int x_dtype, int64_t rows, int64_t co
 extern "C" size_t tg_block_scaled_matmul_bwd_bf16_workspace(int64_t M, int64_t N, int64_t K) {
   if (M < 0 || N < 0 || K < 0) return 0;
   const size_t np = (size_t)round64(N), mp = (size_t)round64(M);
-  const size_t px = q4_part_bytes(q4_split_of(M, K, (int64_t)np), M, K);
-  const size_t pw = q4_part_bytes(q4_split_of(K, N, M), K, N);
+  const size_t px = q4_part_bytes(q4_split_of(M, K, (int64_t)np, false, 16), M, K);
+  const size_t pw = q4_part_bytes(q4_split_of(K, N, M, true, 16), K, N);
   return align256((size_t)M * np * 2) + align256((size_t)K * np * 2) +   // g, b packed along N
          align256((size_t)K * mp * 2) + align256((size_t)N * mp * 2) +   // a.T, g.T packed along M
          (px > pw ? px : pw);                                            // split-K partial tiles of dX, then of dW
@@ -814,7 +846,7 @@ extern "C" int tg_block_scaled_matmul_bwd_bf16(const void* a, int a_dtype, const
   __bf16* at = reinterpret_cast<__bf16*>(p);   p += align256((size_t)K * mp * 2);
   __bf16* gt = reinterpret_cast<__bf16*>(p);   p += align256((size_t)N * mp * 2);
   float* part = reinterpret_cast<float*>(p);
-  const Q4Split spx = q4_split_of(M, K, np), spw = q4_split_of(K, N, M);
+  const Q4Split spx = q4_split_of(M, K, np, false, 16), spw = q4_split_of(K, N, M, true, 16);
   // dX operands: used in place when already bf16, 64-aligned along N and 16-byte aligned
   const __bf16* gx = reinterpret_cast<const __bf16*>(g);
   const __bf16* bx = reinterpret_cast<const __bf16*>(b);
