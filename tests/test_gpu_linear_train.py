@@ -112,3 +112,25 @@ def test_quantize_cols_f32_same_bits_as_rows_of_the_transpose(dev, cols):
     q, s = fp8.quantize_fp8(x, transpose=True)
     rq, rs = fp8.quantize_fp8(x.t().contiguous())
     assert torch.equal(q.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(s, rs)
+
+
+@pytest.mark.parametrize("off", [1, 2, 8])
+def test_frozen_input_takes_weights_and_gradients_at_any_element(dev, off):
+    """Only dW wanted: b and g may start at any element of a flat buffer."""
+    M, K, N = 128, 256, 384
+    a, b, g = _inputs(dev, M, K, N, BF, BF)
+
+    def at(x):
+        flat = torch.empty(x.numel() + off, dtype=x.dtype, device=dev)
+        flat[off:].copy_(x.reshape(-1))
+        return flat[off:].view(x.shape)
+
+    grads = []
+    for bb, gg in ((b, g), (at(b), at(g))):
+        w = bb.detach().requires_grad_()
+        y = fp8.block_scaled_matmul(a, w)
+        y.backward(gg)
+        grads.append((y.detach(), w.grad))
+    assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])
+    # beside f32 activations too
+    assert torch.equal(fp8._fp8_forward(a.float(), at(b), 128), fp8._fp8_forward(a.float(), b, 128))

@@ -37,6 +37,17 @@ def test_bad_calls():
     assert lib.tg_linear_bwd(N, 0, N, 0, N, 0, N, N, 4, 4, 128, N, 0, N) == L.TG_OK
 
 
+def test_operand_alignment():
+    """b at an odd element is refused beside a bf16 a, except where only a.T is kept; g, except where only dW is
+    asked for."""
+    lib = L.lib()
+    fwd = lambda ac, b, bc, keep: lib.tg_linear_fwd(256, ac, b, bc, 256, 128, 128, 128, keep, 256, 256, BIG, N)
+    for ac, b, bc, keep in ((0, 258, 0, 0), (0, 258, 0, 2), (0, 258, 0, 3), (1, 257, 0, 0), (0, 257, 0, 1)):
+        _einval(fwd(ac, b, bc, keep), "16-byte")
+    _einval(lib.tg_linear_bwd_kept(256, 3, 258, 0, 256, 0, 256, 0, 128, 128, 128, 256, BIG, N), "16-byte")
+    _einval(lib.tg_linear_bwd_kept(256, 1, 257, 0, N, 0, 256, 0, 128, 128, 128, 256, BIG, N), "16-byte")
+
+
 def test_prefill_kv_bad_calls():
     lib = L.lib()
     _einval(lib.tg_prefill_kv(N, N, N, 1, 4, 2, 8, 128, N), "null pointer")

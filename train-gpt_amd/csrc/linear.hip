@@ -60,7 +60,9 @@ extern "C" int tg_linear_fwd(const void* a, int a_dtype, const void* b, int b_dt
   if (M == 0 || N == 0) return TG_OK;
   if (!a || !b || !out || !workspace || (keep && !kept)) return einval("linear_fwd: null pointer");
   if (workspace_bytes < tg_linear_fwd_workspace(M, N, K)) return einval("linear_fwd: workspace too small");
-  if (!aligned(a, 16) || !aligned(b, b_dtype == TG_DTYPE_F32 ? 4 : 16) || !aligned(workspace, 256) ||
+  // b by itself along K (beside an f32 a, or where a.T alone is kept) may start at any element
+  const bool b_any = b_dtype == TG_DTYPE_F32 || a_dtype == TG_DTYPE_F32 || keep == TG_KEEP_A;
+  if (!aligned(a, 16) || !(b_any ? aligned_as(b, b_dtype) : aligned(b, 16)) || !aligned(workspace, 256) ||
       !aligned(kept, 256))
     return einval("linear_fwd: a and b must be 16-byte and the buffers 256-byte aligned");
   hipStream_t st = as_stream(stream);
@@ -96,7 +98,8 @@ extern "C" int tg_linear_bwd_kept(const void* kept, int keep, const void* g, int
   if (M == 0 || N == 0 || (!da && !db)) return TG_OK;
   if (!kept || !g || !workspace) return einval("linear_bwd_kept: null pointer");
   if (workspace_bytes < tg_linear_bwd_kept_workspace(M, N)) return einval("linear_bwd_kept: workspace too small");
-  if (!aligned(g, 16) || !aligned(workspace, 256) || !aligned(kept, 256))
+  // g.T alone (dW) may be read from any element
+  if (!(da ? aligned(g, 16) : aligned_as(g, g_dtype)) || !aligned(workspace, 256) || !aligned(kept, 256))
     return einval("linear_bwd_kept: g must be 16-byte and the buffers 256-byte aligned");
   hipStream_t st = as_stream(stream);
   uint8_t* p = reinterpret_cast<uint8_t*>(workspace);
