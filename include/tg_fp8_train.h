@@ -30,15 +30,19 @@ int tg_linear_fwd(const void* a, int a_dtype, const void* b, int b_dtype, void* 
 
 size_t tg_linear_bwd_kept_workspace(int64_t M, int64_t N);
 
-/* da (M, K) and db (K, N), either of them null, from a forward's kept operands.
- * A gradient of dtype f32 holds the bf16 result (fp8.py:95-96). */
+/* da (M, K) and db (K, N) from a forward's kept operands.  A null one is not
+ * wanted.  A gradient of dtype f32 holds the bf16 result (fp8.py:95-96).  With
+ * M == 0 or N == 0 nothing but the gradients is touched: the wanted one that
+ * sums over the empty extent (db with M == 0, da with N == 0) is written as
+ * zeros. */
 int tg_linear_bwd_kept(const void* kept, int keep, const void* g, int g_dtype, void* da, int da_dtype, void* db,
                        int db_dtype, int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes,
                        void* stream);
 
 size_t tg_linear_bwd_workspace(int64_t M, int64_t N, int64_t K);
 
-/* The same from a (M, K), b (K, N) and g (M, N); da has a's dtype, db b's. */
+/* The same from a (M, K), b (K, N) and g (M, N), empty extents included; da has
+ * a's dtype, db b's. */
 int tg_linear_bwd(const void* a, int a_dtype, const void* b, int b_dtype, const void* g, int g_dtype, void* da,
                   void* db, int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes,
                   void* stream);

@@ -51,6 +51,25 @@ def test_fp8_backward_empty_needs_the_gradient_it_writes(dev):
     assert rc == L.TG_EINVAL and L.lib().tg_last_error().endswith(b"null pointer")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N", [(0, 384), (128, 0), (0, 0)])
+def test_linear_backward_empty_extent_zero_fills_the_wanted_gradients(dev, M, N, dtype):
+    """tg_linear_bwd and tg_linear_bwd_kept: db over M = 0 and da over N = 0 are zeros, a null gradient is not
+    wanted, and what lies past a gradient stays."""
+    K, lib = 256, L.lib()
+    code = L.TG_DTYPE_F32 if dtype == torch.float32 else L.TG_DTYPE_BF16
+    calls = (lambda da, db, st: lib.tg_linear_bwd(NUL, code, NUL, code, NUL, 0, da, db, M, N, K, NUL, 0, st),
+             lambda da, db, st: lib.tg_linear_bwd_kept(NUL, L.TG_KEEP_A | L.TG_KEEP_B, NUL, 0, da, code, db, code, M, N,
+                                                       K, NUL, 0, st))
+    for call in calls:
+        for want_a, want_b in ((True, True), (True, False), (False, True), (False, False)):
+            da, db = (torch.full((n + 64,), 3.0, dtype=dtype, device=dev) for n in (M * K, K * N))
+            L.check(call(L.ptr(da) if want_a else NUL, L.ptr(db) if want_b else NUL, L.stream_of(da)))
+            torch.cuda.synchronize()
+            for d, n, want in ((da, M * K, want_a), (db, K * N, want_b)):
+                assert torch.all(d[:n] == (0.0 if want else 3.0)) and torch.all(d[n:] == 3.0)
+
+
 @pytest.mark.parametrize("dim", [256, 2048, 6144])   # the row kernel's widths and the general one
 def test_norm_backward_zero_rows_gives_zero_dscale(dev, dim):
     scale = torch.ones(dim, dtype=torch.bfloat16, device=dev)

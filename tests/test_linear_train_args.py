@@ -37,6 +37,22 @@ def test_bad_calls():
     assert lib.tg_linear_bwd(N, 0, N, 0, N, 0, N, N, 4, 4, 128, N, 0, N) == L.TG_OK
 
 
+def test_negative_extents_and_empty_problems():
+    """Negative extents are refused before the pointers are looked at; an empty problem without a wanted gradient
+    is a no-op (test_gpu_empty_extents.py has the wanted ones)."""
+    lib = L.lib()
+    for m, n in ((-128, 128), (128, -128)):
+        _einval(lib.tg_linear_fwd(N, 0, N, 0, N, m, n, 128, 0, N, N, BIG, N), "bad GEMM shape")
+        _einval(lib.tg_linear_bwd_kept(N, 3, N, 0, 256, 0, 256, 0, m, n, 128, N, BIG, N), "bad GEMM shape")
+        _einval(lib.tg_linear_bwd(N, 0, N, 0, N, 0, 256, 256, m, n, 128, N, BIG, N), "bad GEMM shape")
+    for m, n in ((0, 128), (128, 0), (0, 0)):
+        assert lib.tg_linear_fwd(N, 0, N, 0, N, m, n, 128, 0, N, N, 0, N) == L.TG_OK
+        assert lib.tg_linear_bwd_kept(N, 3, N, 0, N, 0, N, 0, m, n, 128, N, 0, N) == L.TG_OK
+        assert lib.tg_linear_bwd(N, 0, N, 0, N, 0, N, N, m, n, 128, N, 0, N) == L.TG_OK
+    # the gradient of an operand that was not kept stays refused
+    _einval(lib.tg_linear_bwd_kept(N, 1, N, 0, 256, 0, N, 0, 128, 0, 128, N, 0, N), "not kept")
+
+
 def test_operand_alignment():
     """b at an odd element is refused beside a bf16 a, except where only a.T is kept; g, except where only dW is
     asked for."""

@@ -36,6 +36,15 @@ static bool valid_dtype(int d) { return d == TG_DTYPE_BF16 || d == TG_DTYPE_F32;
 static bool aligned_as(const void* p, int dtype) { return aligned(p, dtype == TG_DTYPE_F32 ? 4 : 2); }
 static int grad_dtype(int d) { return d == TG_DTYPE_F32 ? kOutF32OfBf16 : TG_DTYPE_BF16; }
 
+// The wanted gradients of an empty M or N, where nothing is summed: zeros.
+static int zero_grad(void* d, int dtype, int64_t n, hipStream_t st) {
+  return d ? launch_fill_zero_bf16(d, dtype == TG_DTYPE_F32 ? 2 * n : n, st) : TG_OK;
+}
+static int zero_grads(void* da, int da_dtype, void* db, int db_dtype, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+  TG_TRY(zero_grad(da, da_dtype, M * K, st));
+  return zero_grad(db, db_dtype, K * N, st);
+}
+
 }  // namespace tg
 
 using namespace tg;
@@ -95,7 +104,8 @@ extern "C" int tg_linear_bwd_kept(const void* kept, int keep, const void* g, int
   if (M % 128 || N % 128) return einval("linear_bwd_kept: M and N must be multiples of 128");
   if ((db && !(keep & TG_KEEP_A)) || (da && !(keep & TG_KEEP_B)))
     return einval("linear_bwd_kept: the operand of a wanted gradient was not kept");
-  if (M == 0 || N == 0 || (!da && !db)) return TG_OK;
+  if (M == 0 || N == 0) return zero_grads(da, da_dtype, db, db_dtype, M, N, K, as_stream(stream));
+  if (!da && !db) return TG_OK;
   if (!kept || !g || !workspace) return einval("linear_bwd_kept: null pointer");
   if (workspace_bytes < tg_linear_bwd_kept_workspace(M, N)) return einval("linear_bwd_kept: workspace too small");
   // g.T alone (dW) may be read from any element
@@ -127,7 +137,8 @@ extern "C" int tg_linear_bwd(const void* a, int a_dtype, const void* b, int b_dt
   TG_TRY(check_gemm_args("linear_bwd", M, N, K, 128, 1));
   if (!valid_dtype(a_dtype) || !valid_dtype(b_dtype) || !valid_dtype(g_dtype))
     return einval("linear_bwd: operands must be bf16 or f32");
-  if (M == 0 || N == 0 || (!da && !db)) return TG_OK;
+  if (M == 0 || N == 0) return zero_grads(da, a_dtype, db, b_dtype, M, N, K, as_stream(stream));
+  if (!da && !db) return TG_OK;
   if (!a || !b || !g || !workspace) return einval("linear_bwd: null pointer");
   if (workspace_bytes < tg_linear_bwd_workspace(M, N, K)) return einval("linear_bwd: workspace too small");
   if (!aligned_as(a, a_dtype) || !aligned_as(b, b_dtype) || !aligned_as(g, g_dtype) || !aligned(workspace, 256))
