@@ -134,3 +134,36 @@ def test_frozen_input_takes_weights_and_gradients_at_any_element(dev, off):
     assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])
     # beside f32 activations too
     assert torch.equal(fp8._fp8_forward(a.float(), at(b), 128), fp8._fp8_forward(a.float(), b, 128))
+
+
+# rows of more columns than the ragged kernels' 32-bit offsets reach (2^26), and a column of so many rows (2^29) that
+# its tiles pass a 1-D grid: element loads, the bytes of the separate quantizers
+def test_quantize_cols_of_very_wide_unaligned_rows(dev):
+    cols = (1 << 26) + 3
+    x = torch.empty((128, cols), dtype=BF, device=dev).normal_(generator=torch.Generator(device=dev).manual_seed(5))
+    q, s = fp8.quantize_fp8(x, transpose=True)
+    for c in (0, (1 << 25) + 61, cols - 1024):
+        rq, rs = fp8.quantize_fp8(x[:, c:c + 1024].t().contiguous())
+        assert torch.equal(q[c:c + 1024].view(torch.uint8), rq.view(torch.uint8)) and torch.equal(s[c:c + 1024], rs)
+
+
+def test_quantize_cols_of_one_very_long_f32_column(dev):
+    x = torch.empty(((1 << 29) + 128, 1), device=dev).normal_(generator=torch.Generator(device=dev).manual_seed(6))
+    q, s = fp8.quantize_fp8(x, transpose=True)
+    rq, rs = fp8.quantize_fp8(x.reshape(1, -1))
+    assert torch.equal(q.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(s, rs)
+
+
+def test_linear_over_a_very_long_contraction(dev):
+    """K past 2^26 in f32, one token and one output: y, da and db against the row quantizers and the GEMM."""
+    K = (1 << 26) + 128
+    gen = torch.Generator(device=dev).manual_seed(7)
+    a, b = (torch.empty(s, device=dev).normal_(generator=gen).requires_grad_() for s in ((1, K), (K, 1)))
+    y = fp8.block_scaled_matmul(a, b)
+    qa, qb = fp8.quantize_fp8(a.detach()), fp8.quantize_fp8(b.detach().reshape(1, K))
+    assert torch.equal(y, fp8.scaled_matmul(qa[0], qa[1], qb[0], qb[1]))
+    da, db = torch.autograd.grad(y, (a, b), torch.full((1, 1), 0.5, dtype=BF, device=dev))
+    # one value to a block: its code is 448, its scale |value| / 448, so the products are the values themselves
+    for got, v in ((da, b), (db, a)):
+        want = 0.5 * v.detach().reshape(got.shape)
+        assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs()).all())

@@ -140,18 +140,20 @@ int launch_quant_cols(const void* x, int64_t rows, int64_t cols, uint8_t* q_t, f
 // The launch for tensors of any extents: all bf16 ones together (up to three,
 // as the backward's g, b and a), read the way the least aligned of them needs,
 // and all f32 ones together.  Whole-tile bf16 tensors take the plain kernel
-// when they are at most two.
+// when they are at most two.  Rows of more than kQuantMaxCols columns (the
+// ragged kernels' 32-bit offsets) and grids past half of kDualMaxTiles (one
+// column of 2^30 rows) are read element by element.
 int launch_quant_tensors(const QuantTensor* t, int n, bool skm, hipStream_t st) {
   for (int f32 = 0; f32 < 2; ++f32) {
     DualJobs jobs{};
     int cnt = 0, in = f32 ? kInF32 : kInVec;
-    int64_t total = 0;
+    int64_t total = 0, widest = 0;
     for (int i = 0; i < n; ++i) {
       if ((t[i].x_dtype == TG_DTYPE_F32) != (f32 != 0) || t[i].rows == 0 || t[i].cols == 0) continue;
       if (cnt == 3) return einval("quantize: at most three tensors of a type");
-      if (t[i].cols > kQuantMaxCols) return einval("quantize: rows too wide");
       TG_TRY(dual_job(jobs.job[cnt], "quantize", t[i].x, t[i].rows, t[i].cols, t[i].q, t[i].s, t[i].qt, t[i].st,
-                      total % 8 == 0, skm));
+                      total % 8 == 0, skm, 0x7FFFFFFF));
+      widest = t[i].cols > widest ? t[i].cols : widest;
       jobs.job[cnt].part = t[i].part;
       if (!f32) {
         const bool whole = t[i].rows % 128 == 0 && t[i].cols % 128 == 0 && aligned(t[i].x, 16);
@@ -166,9 +168,20 @@ int launch_quant_tensors(const QuantTensor* t, int n, bool skm, hipStream_t st) 
       ++cnt;
     }
     if (cnt == 0) continue;
-    if (total > kDualMaxTiles) return einval("quantize: too many 128 x 128 tiles");
     if (cnt == 3 && in == kInVec) in = kInBf16;
-    const dim3 grid((unsigned)total), block(kDualThreads);
+    const bool wide = in != kInVec && (widest > kQuantMaxCols || total > kDualMaxTiles / 2);
+    if (total > (wide ? 0x7FFF0000 : kDualMaxTiles)) return einval("quantize: too many 128 x 128 tiles");
+    jobs.nall = (int)total;
+    const dim3 block(kDualThreads);
+    if (wide) {
+      constexpr int64_t kRow = int64_t(1) << 16;   // workgroups per row of the 2-D grid
+      const dim3 grid2((unsigned)(total < kRow ? total : kRow), (unsigned)((total + kRow - 1) / kRow));
+      if (f32) hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInF32Wide>), grid2, block, 0, st, jobs);
+      else hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInBf16Wide>), grid2, block, 0, st, jobs);
+      TG_TRY(check_launch("quant_tensors"));
+      continue;
+    }
+    const dim3 grid((unsigned)total);
     if (in == kInVec) hipLaunchKernelGGL((quant_dual_kernel<true, false>), grid, block, 0, st, jobs);
     else if (in == kInBf16)
       hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInBf16>), grid, block, 0, st, jobs);

@@ -40,6 +40,8 @@
 // bf16 rows at any even address (an odd width); kInF32: f32 rows, whose scale
 // and quotient are IEEE divides and whose raw tile takes 65 KiB of LDS (row
 // pitch 130 words: the column reads, two values at a time, touch all 64 banks).
+// kInBf16Wide, kInF32Wide: the same tensors past 32-bit offsets or a 1-D grid
+// (rows of more than kQuantMaxCols columns, more than kDualMaxTiles / 2 tiles), by element loads.
 //
 // Scales.  With K-block-major scales (skm) a tile's 128 row scales are 512
 // contiguous bytes (s[tx * rows + r0 ..]) and so are its 128 column scales
@@ -91,9 +93,10 @@ struct DualJob {
 struct DualJobs {
   DualJob job[3];
   int nblk0, nblk1;   // tiles of jobs 0 and 1; the grid's others are job 2's (job 1's with nblk1 = 0)
+  int nall;           // tiles of all jobs (read by the wide forms, whose 2-D grid may overhang)
 };
 
-constexpr int kInVec = 0, kInBf16 = 1, kInBf16Any = 2, kInF32 = 3;
+constexpr int kInVec = 0, kInBf16 = 1, kInBf16Any = 2, kInF32 = 3, kInBf16Wide = 4, kInF32Wide = 5;
 
 constexpr int kDualThreads = 512;
 
@@ -115,7 +118,8 @@ __device__ __forceinline__ uint32_t oct_max_u32(uint32_t v) {
 // the scale stores.
 template <bool ROWS, bool GUARD, bool IO = false, bool IO_SCALES = true, int IN = kInVec>
 __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs) {
-  constexpr bool F32 = IN == kInF32, RAGGED = IN != kInVec;
+  constexpr bool F32 = IN == kInF32 || IN == kInF32Wide, RAGGED = IN != kInVec;
+  constexpr bool WIDE = IN == kInBf16Wide || IN == kInF32Wide;
   static_assert(!RAGGED || (GUARD && !IO), "ragged tiles are guarded");
   constexpr int kF32Pitch = 130;
   // the raw tile (row pitch 272 B); once every column is in registers the
@@ -125,8 +129,10 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
   uint32_t* tq = tile;
   constexpr bool kScales = !IO || IO_SCALES;
   const int tid = threadIdx.x;
-  const bool second = (int)blockIdx.x >= jobs.nblk0;
-  const bool third = RAGGED && jobs.nblk1 > 0 && (int)blockIdx.x >= jobs.nblk0 + jobs.nblk1;
+  const int blk = WIDE ? (int)(blockIdx.y * gridDim.x + blockIdx.x) : (int)blockIdx.x;
+  if (WIDE && blk >= jobs.nall) return;
+  const bool second = blk >= jobs.nblk0;
+  const bool third = RAGGED && jobs.nblk1 > 0 && blk >= jobs.nblk0 + jobs.nblk1;
   const DualJob& J = third ? jobs.job[2] : second ? jobs.job[1] : jobs.job[0];
   const uint4* __restrict__ x = J.x;
   const int64_t rows = J.rows, cols = J.cols;
@@ -135,7 +141,7 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
   uint8_t* __restrict__ qt = J.qt;
   float* __restrict__ st = J.st;
   const bool skm = J.skm != 0;
-  const int slot = (int)blockIdx.x - (second ? jobs.nblk0 : 0) - (third ? jobs.nblk1 : 0);
+  const int slot = blk - (second ? jobs.nblk0 : 0) - (third ? jobs.nblk1 : 0);
   int tx = slot % J.gx, ty = slot / J.gx;
   if (J.xcd_blocks) {
     // slot % 8 is the XCD: the host sets xcd_blocks only on a job that
@@ -154,7 +160,25 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
   // the job's parts (workgroup-uniform)
   const bool do_rows = ROWS && J.part != 2, do_cols = J.part != 1;
   uint4 v[4], vh[F32 ? 4 : 1];   // F32: v[u], vh[u] the lane's 8 values
-  if constexpr (RAGGED) {
+  if constexpr (WIDE) {
+    // element loads at 64-bit addresses
+    auto at = [&](int u, int e) -> uint32_t {
+      const int64_t r = r0 + rr + 32 * u, c = c0 + 8 * ch + e;
+      if (r >= rows || c >= cols) return 0u;
+      if constexpr (F32) return reinterpret_cast<const uint32_t*>(x)[r * cols + c];
+      else return reinterpret_cast<const uint16_t*>(x)[r * cols + c];
+    };
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if constexpr (F32) {
+        v[u] = make_uint4(at(u, 0), at(u, 1), at(u, 2), at(u, 3));
+        vh[u] = make_uint4(at(u, 4), at(u, 5), at(u, 6), at(u, 7));
+      } else {
+        v[u] = make_uint4(at(u, 0) | at(u, 1) << 16, at(u, 2) | at(u, 3) << 16, at(u, 4) | at(u, 5) << 16,
+                          at(u, 6) | at(u, 7) << 16);
+      }
+    }
+  } else if constexpr (RAGGED) {
     // a descriptor per four rows (one wave's), so 32-bit offsets do for any x;
     // rows past the last fall outside it, columns past the last are cleared
     constexpr uint32_t kE = F32 ? 4u : 2u;
@@ -346,12 +370,12 @@ __global__ __launch_bounds__(kDualThreads) void quant_dual_kernel(DualJobs jobs)
 constexpr int64_t kDualMaxTiles = int64_t(1) << 23;   // slots fit one 1-D grid of 256-thread groups
 
 inline int dual_job(DualJob& j, const char* who, const void* x, int64_t rows, int64_t cols, uint8_t* q,
-                    float* s, uint8_t* q_t, float* s_t, bool xcd_ok, bool skm) {
+                    float* s, uint8_t* q_t, float* s_t, bool xcd_ok, bool skm,
+                    int64_t max_tiles = kDualMaxTiles) {
   const int64_t gx = (cols + 127) / 128, gy = (rows + 127) / 128;
-  if (gx * gy > kDualMaxTiles) {
+  if (gx * gy > max_tiles) {
     char msg[160];
-    snprintf(msg, sizeof msg, "%s: (rows / 128) x (cols / 128) must be <= %lld tiles", who,
-             (long long)kDualMaxTiles);
+    snprintf(msg, sizeof msg, "%s: (rows / 128) x (cols / 128) must be <= %lld tiles", who, (long long)max_tiles);
     return einval(msg);
   }
   j.x = reinterpret_cast<const uint4*>(x);
