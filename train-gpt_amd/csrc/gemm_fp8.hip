@@ -56,11 +56,15 @@ __device__ __forceinline__ v8i as_v8i(const u32x4_t& lo, const u32x4_t& hi) {
 
 
 // SKM: scales K-block-major (see gemm_fp8_nt_256_kernel).
-template <int TM, int TN, int BNS, bool OUT_F32, bool SKM>
+// What a GEMM stores: bf16, f32, or f32 holding the bf16 result (K-block-major
+// scales and one weight scale per column only: the FP8 linear's gradients).
+constexpr int kCBf16 = 0, kCF32 = 1, kCF32Of16 = 2;
+
+template <int TM, int TN, int BNS, int OUT, bool SKM>
 __global__ __launch_bounds__(256, 2) void gemm_fp8_nt_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ SA, const uint8_t* __restrict__ B,
     const float* __restrict__ SB, void* __restrict__ C, int M, int N, int K, int tiles_m,
-    int tiles_n, int round16) {
+    int tiles_n) {
   constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
   constexpr int LA = BM / 32, LB = BN / 32;          // 16-byte chunks per thread per K block
   constexpr int STAGE = (BM + BN) * 8;               // uint4 per stage (128 B per row)
@@ -175,8 +179,8 @@ __global__ __launch_bounds__(256, 2) void gemm_fp8_nt_kernel(
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + wm * TM * 16 + i * 16 + 4 * fg + r;
         if (m < M && n < N) {
-          if (OUT_F32)
-            reinterpret_cast<float*>(C)[(int64_t)m * N + n] = round16 ? round_bf16(acc[i][j][r]) : acc[i][j][r];
+          if (OUT != kCBf16)
+            reinterpret_cast<float*>(C)[(int64_t)m * N + n] = OUT == kCF32 ? acc[i][j][r] : round_bf16(acc[i][j][r]);
           else
             reinterpret_cast<__bf16*>(C)[(int64_t)m * N + n] = (__bf16)acc[i][j][r];
         }
@@ -340,8 +344,7 @@ __device__ __forceinline__ uint8_t* lat_pick(uint8_t* s0, uint8_t* s1, uint8_t* 
 // each element then copied out for the promotion; this file is built with
 // -amdgpu-mfma-vgpr-form, which keeps them in VGPRs and changes no other
 // kernel here.)
-// out: kLatBf16, kLatF32, or kLatF32Of16 (the bf16 result widened).
-constexpr int kLatBf16 = 0, kLatF32 = 1, kLatF32Of16 = 2;
+// out: kCBf16, kCF32 or kCF32Of16.
 template <int TM_, int TN, int WN, int OCC, int BNS, bool SKM>
 __global__ __launch_bounds__(128 * WN, OCC * WN / 2 > 1 ? OCC * WN / 2 : 1) void gemm_fp8_lat_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ SA, const uint8_t* __restrict__ B,
@@ -467,7 +470,7 @@ __global__ __launch_bounds__(128 * WN, OCC * WN / 2 > 1 ? OCC * WN / 2 : 1) void
   // workgroup's LDS
   __builtin_amdgcn_s_waitcnt(0x0070 | 0x0F00);      // vmcnt(0)
   const int mw = m0 + wm * 16 * TM, nw = n0 + wn * 16 * TNW;
-  if (out == kLatBf16 && vec_out) {
+  if (out == kCBf16 && vec_out) {
     // every wave is done with the stages before they hold results
     __builtin_amdgcn_s_waitcnt(0xC07F);             // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
@@ -495,23 +498,30 @@ __global__ __launch_bounds__(128 * WN, OCC * WN / 2 > 1 ? OCC * WN / 2 : 1) void
     }
     return;
   }
+  // the output's form is chosen once, outside the element loops (chosen at each
+  // element, odd widths ran up to 1.2x longer: 640 x 6899 over 128 6.8 -> 8.4 us)
+  auto put = [&](auto mode) {
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TNW; ++j) {
-      const int n = nw + j * 16 + fr;
+      for (int j = 0; j < TNW; ++j) {
+        const int n = nw + j * 16 + fr;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = mw + i * 16 + 4 * fg + r;
-        if (m < M && n < N) {
-          if (out != kLatBf16)
-            reinterpret_cast<float*>(C)[(int64_t)m * N + n] =
-                out == kLatF32Of16 ? round_bf16(acc[i][j][r]) : acc[i][j][r];
-          else
-            reinterpret_cast<__bf16*>(C)[(int64_t)m * N + n] = (__bf16)acc[i][j][r];
+        for (int r = 0; r < 4; ++r) {
+          const int m = mw + i * 16 + 4 * fg + r;
+          const float v = acc[i][j][r];
+          if (m < M && n < N) {
+            if (mode.value == kCBf16)
+              reinterpret_cast<__bf16*>(C)[(int64_t)m * N + n] = (__bf16)v;
+            else
+              reinterpret_cast<float*>(C)[(int64_t)m * N + n] = mode.value == kCF32Of16 ? round_bf16(v) : v;
+          }
         }
       }
-    }
+  };
+  if (out == kCBf16) put(IntC<kCBf16>{});
+  else if (out == kCF32) put(IntC<kCF32>{});
+  else put(IntC<kCF32Of16>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -801,16 +811,16 @@ __device__ __forceinline__ void w32_block(const W32Ctx& c, v16f (&acc)[2][4], W3
 // 16-byte slot, swapped when the row is odd) and store them whole.  A wave
 // reads back only what it wrote and LDS completes a wave's accesses in
 // order, so waiting for its own writes is enough.
-template <int S, bool OUT_F32>
+template <int S, int OUT>
 __device__ __forceinline__ void w32_store_tile(const v16f (&acc)[2][4], void* __restrict__ C, int M, int N,
-                                               int m0w, int n0w, int wave, int lane_in, int round16) {
+                                               int m0w, int n0w, int wave, int lane_in) {
   // an opaque copy of the lane index: the store addresses derive from it, so
   // the compiler cannot hoist them out of the tile loop (where they would
   // stay live across the K loop)
   int lane = lane_in;
   asm volatile("" : "+v"(lane));
   const int cl = lane & 31, g = lane >> 5;
-  if (!OUT_F32 && (N % 8) == 0) {
+  if (OUT == kCBf16 && (N % 8) == 0) {
     uint8_t* wbuf = (wave < 4 ? g256_a<S>() : g256_b<S>()) + (wave & 3) * 8192;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -852,17 +862,16 @@ __device__ __forceinline__ void w32_store_tile(const v16f (&acc)[2][4], void* __
       for (int q = 0; q < 4; ++q) {
         const int n = n0w + 32 * j + 8 * q + 4 * g;
         const v16f& v = acc[i][j];
-        if (OUT_F32) {
+        if (OUT != kCBf16) {
           float* dst = reinterpret_cast<float*>(C) + (int64_t)m * N + n;
-          float o[4];
-#pragma unroll
-          for (int t = 0; t < 4; ++t) o[t] = round16 ? round_bf16(v[4 * q + t]) : v[4 * q + t];
+          auto f32 = [](float x) { return OUT == kCF32 ? x : round_bf16(x); };
           if (vec_ok && n + 4 <= N) {
-            *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+            *reinterpret_cast<float4*>(dst) =
+                make_float4(f32(v[4 * q]), f32(v[4 * q + 1]), f32(v[4 * q + 2]), f32(v[4 * q + 3]));
           } else {
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-              if (n + t < N) dst[t] = o[t];
+              if (n + t < N) dst[t] = f32(v[4 * q + t]);
           }
         } else {
           __bf16* dst = reinterpret_cast<__bf16*>(C) + (int64_t)m * N + n;
@@ -889,11 +898,11 @@ __device__ __forceinline__ void w32_store_tile(const v16f (&acc)[2][4], void* __
 // row scales per loader lane group are then 256 contiguous bytes instead of
 // 64 rows K/32 bytes apart, which takes the scale copies from 64 cache lines
 // per instruction to two.
-template <int BNS, bool OUT_F32, bool SKM>
+template <int BNS, int OUT, bool SKM>
 __global__ __launch_bounds__(512, 1) void gemm_fp8_nt_256_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ SA, const uint8_t* __restrict__ B,
     const float* __restrict__ SB, void* __restrict__ C, int M, int N, int K, int tiles_m,
-    int tiles_n, int round16) {
+    int tiles_n) {
   W32Ctx c;
   const int tid = threadIdx.x, lane = tid & 63;
   c.wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: keeps descriptors in SGPRs
@@ -1029,8 +1038,7 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_nt_256_kernel(
     prev.p = v16f{};
     prev.sa = 0.0f;
     prev.sb = make_float4(0.f, 0.f, 0.f, 0.f);
-    w32_store_tile<S, OUT_F32>(acc, C, M, N, tm_cur * 256 + wm * 64, tn_cur * 256 + wn * 128, c.wave,
-                               lane, round16);
+    w32_store_tile<S, OUT>(acc, C, M, N, tm_cur * 256 + wm * 64, tn_cur * 256 + wn * 128, c.wave, lane);
     if (more) {
       // every wave is done with stage S before the next block's copies land there
       __syncthreads();
@@ -1050,27 +1058,27 @@ __global__ __launch_bounds__(512, 1) void gemm_fp8_nt_256_kernel(
   if (step < nsteps) one_step(IntC<0>{});
 }
 
-template <int BNS, bool OUT_F32, bool SKM>
+template <int BNS, int OUT, bool SKM>
 static int launch_gemm_256(const uint8_t* a_q, const float* a_s, const uint8_t* b_q,
-                           const float* b_s, void* c, int M, int N, int K, int r16, hipStream_t st) {
+                           const float* b_s, void* c, int M, int N, int K, hipStream_t st) {
   const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
   // one workgroup per CU (135 KiB of LDS each), looping over its tiles; the
   // grid stays a multiple of 8 so that a workgroup's slots share its XCD
   const int ntiles = tiles_m * tiles_n;
   const int slots = device_cus() & ~7;
   const int grid = ntiles <= slots || slots == 0 ? ntiles : slots;
-  hipLaunchKernelGGL((gemm_fp8_nt_256_kernel<BNS, OUT_F32, SKM>), dim3((unsigned)grid), dim3(512), 0, st,
-                     a_q, a_s, b_q, b_s, c, M, N, K, tiles_m, tiles_n, r16);
+  hipLaunchKernelGGL((gemm_fp8_nt_256_kernel<BNS, OUT, SKM>), dim3((unsigned)grid), dim3(512), 0, st,
+                     a_q, a_s, b_q, b_s, c, M, N, K, tiles_m, tiles_n);
   return check_launch("gemm_fp8_nt_256");
 }
 
-template <int TM, int TN, int BNS, bool OUT_F32, bool SKM>
+template <int TM, int TN, int BNS, int OUT, bool SKM>
 static int launch_gemm_cfg(const uint8_t* a_q, const float* a_s, const uint8_t* b_q,
-                           const float* b_s, void* c, int M, int N, int K, int r16, hipStream_t st) {
+                           const float* b_s, void* c, int M, int N, int K, hipStream_t st) {
   constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const size_t lds = (size_t)2 * (BM + BN) * 128 + (size_t)2 * (BM + BN) * 4;
-  auto kern = gemm_fp8_nt_kernel<TM, TN, BNS, OUT_F32, SKM>;
+  auto kern = gemm_fp8_nt_kernel<TM, TN, BNS, OUT, SKM>;
   // the dynamic-LDS limit is a per-device function attribute: set once per
   // device (thread-safe, see device_cus)
   constexpr int kMaxDev = 64;
@@ -1087,17 +1095,16 @@ static int launch_gemm_cfg(const uint8_t* a_q, const float* a_s, const uint8_t* 
     return TG_EHIP;
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), lds, st, a_q, a_s, b_q,
-                     b_s, c, M, N, K, tiles_m, tiles_n, r16);
+                     b_s, c, M, N, K, tiles_m, tiles_n);
   return check_launch("gemm_fp8_nt");
 }
 
 template <int TM, int TN, int WN, int OCC, bool SKM>
 static int launch_gemm_lat(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, const float* b_s,
-                           int b_scale_bn, void* c, bool f32, int M, int N, int K, int r16, hipStream_t st) {
+                           int b_scale_bn, void* c, int out, int M, int N, int K, hipStream_t st) {
   constexpr int BM = 32 * TM, BN = 32 * TN;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int vec = N % 8 == 0 && aligned(c, 16);
-  const int out = r16 ? kLatF32Of16 : f32 ? kLatF32 : kLatBf16;
   const dim3 grid((unsigned)(tiles_m * tiles_n)), block(128 * WN);
   if (b_scale_bn == 1)
     hipLaunchKernelGGL((gemm_fp8_lat_kernel<TM, TN, WN, OCC, 1, SKM>), grid, block, 0, st, a_q, a_s, b_q, b_s, c, M,
@@ -1164,12 +1171,13 @@ static int gemm_tile_of(int64_t m, int64_t n, int64_t nkb) {
   return best;
 }
 
-template <bool SKM>
+template <int OUT, bool SKM>
 static int launch_gemm_fp8_layout(const uint8_t* a_q, const float* a_s, const uint8_t* b_q,
-                                  const float* b_s, int b_scale_bn, void* c, bool f32, int m, int n,
-                                  int k, int r16, bool fits32, hipStream_t st) {
+                                  const float* b_s, int b_scale_bn, void* c, int m, int n, int k, bool fits32,
+                                  hipStream_t st) {
+  constexpr int BNS2 = OUT == kCF32Of16 ? 1 : 128;   // kCF32Of16 comes with b_scale_bn = 1 only
   if (fits32) {
-#define TG_LAT(...) launch_gemm_lat<__VA_ARGS__, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, st)
+#define TG_LAT(...) launch_gemm_lat<__VA_ARGS__, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, OUT, m, n, k, st)
     switch (gemm_tile_of(m, n, k / 128)) {
       case 1: return TG_LAT(4, 8, 4, 1);
       case 2: return TG_LAT(4, 6, 4, 1);
@@ -1180,32 +1188,25 @@ static int launch_gemm_fp8_layout(const uint8_t* a_q, const float* a_s, const ui
       default: break;
     }
 #undef TG_LAT
-    if (b_scale_bn == 1)
-      return f32 ? launch_gemm_256<1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
-                 : launch_gemm_256<1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
-    return f32 ? launch_gemm_256<128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
-               : launch_gemm_256<128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
+    return b_scale_bn == 1 ? launch_gemm_256<1, OUT, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
+                           : launch_gemm_256<BNS2, OUT, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
   }
-  // 128 x 128 or 128 x 96 tiles, whichever leaves the busiest CU the fewer
-  // outputs (tiles per CU, rounded up, times the tile's columns): C1's 2048 x
-  // 3072 is 384 tiles of 128 (two on half the CUs) or 512 of 96 (two on
-  // every CU), 10% faster
+  // operands past 2^31 bytes: 128 x 128 or 128 x 96 tiles, whichever leaves the
+  // busiest CU the fewer outputs (tiles per CU, rounded up, times the tile's columns)
   const int64_t cus = device_cus() > 0 ? device_cus() : 1;
   const int64_t tm = (m + 127) / 128;
   const int64_t load128 = (tm * ((n + 127) / 128) + cus - 1) / cus * 128;
   const int64_t load96 = (tm * ((n + 95) / 96) + cus - 1) / cus * 96;
-  if (load96 < load128) {
-    if (b_scale_bn == 1)
-      return f32 ? launch_gemm_cfg<4, 3, 1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
-                 : launch_gemm_cfg<4, 3, 1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
-    return f32 ? launch_gemm_cfg<4, 3, 128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
-               : launch_gemm_cfg<4, 3, 128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
-  }
-  if (b_scale_bn == 1)
-    return f32 ? launch_gemm_cfg<4, 4, 1, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
-               : launch_gemm_cfg<4, 4, 1, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
-  return f32 ? launch_gemm_cfg<4, 4, 128, true, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st)
-             : launch_gemm_cfg<4, 4, 128, false, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, r16, st);
+  if (load96 < load128)
+    return b_scale_bn == 1 ? launch_gemm_cfg<4, 3, 1, OUT, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
+                           : launch_gemm_cfg<4, 3, BNS2, OUT, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
+  return b_scale_bn == 1 ? launch_gemm_cfg<4, 4, 1, OUT, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st)
+                         : launch_gemm_cfg<4, 4, BNS2, OUT, SKM>(a_q, a_s, b_q, b_s, c, m, n, k, st);
+}
+
+// the tuned kernels take 32-bit buffer offsets; larger operands the VGPR-staged one
+static bool gemm_fits32(int64_t M, int64_t N, int64_t K) {
+  return (uint64_t)M * (uint64_t)K < (1ull << 31) && (uint64_t)N * (uint64_t)K < (1ull << 31);
 }
 
 int launch_gemm_fp8(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, const float* b_s,
@@ -1213,12 +1214,16 @@ int launch_gemm_fp8(const uint8_t* a_q, const float* a_s, const uint8_t* b_q, co
                     hipStream_t st, bool skm) {
   if (M == 0 || N == 0) return TG_OK;
   const int m = (int)M, n = (int)N, k = (int)K;
-  const int r16 = c_dtype == kOutF32OfBf16;   // f32 output holding the bf16 result
-  const bool f32 = c_dtype == TG_DTYPE_F32 || r16;
-  // the tuned kernels take 32-bit buffer offsets; larger operands the VGPR-staged one
-  const bool fits32 = (uint64_t)M * (uint64_t)K < (1ull << 31) && (uint64_t)N * (uint64_t)K < (1ull << 31);
-  return skm ? launch_gemm_fp8_layout<true>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, fits32, st)
-             : launch_gemm_fp8_layout<false>(a_q, a_s, b_q, b_s, b_scale_bn, c, f32, m, n, k, r16, fits32, st);
+  const bool fits32 = gemm_fits32(M, N, K);
+#define TG_LAYOUT(OUT, SKM) \
+  launch_gemm_fp8_layout<OUT, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, m, n, k, fits32, st)
+  if (c_dtype == kOutF32OfBf16) {   // f32 output holding the bf16 result
+    if (!skm || b_scale_bn != 1) return einval("gemm_fp8: f32 of bf16 needs K-block-major scales, one per column");
+    return TG_LAYOUT(kCF32Of16, true);
+  }
+  if (c_dtype == TG_DTYPE_F32) return skm ? TG_LAYOUT(kCF32, true) : TG_LAYOUT(kCF32, false);
+  return skm ? TG_LAYOUT(kCBf16, true) : TG_LAYOUT(kCBf16, false);
+#undef TG_LAYOUT
 }
 
 // ---------------------------------------------------------------------------
