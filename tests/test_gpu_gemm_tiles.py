@@ -1,12 +1,15 @@
 """The FP8 GEMM's tile choice changes no bit: every kernel adds a K block's
 product in the same order, so an output element is the same whichever tile
-computes it.  A row range of one operand is multiplied alone and as part of
-taller launches (which take other tiles), at the edges of the 32-, 64-, 128-
-and 256-row tiles and of their 64- to 256-column widths."""
+computes it.  Each tile is run on shapes of its own (gemm_tiles.py;
+test_gemm_tile_choice.py holds them to it) against launches of 32 x 64 tiles;
+and a row range of one operand is multiplied alone and as part of taller
+launches, at the edges of the 32- and 64-row tiles above all."""
 import pytest
 import torch
 
+import _tglib as L
 import fp8
+import gemm_tiles as G
 
 pytestmark = pytest.mark.gpu
 
@@ -44,7 +47,6 @@ def test_gemm_bits_do_not_depend_on_the_tile(dev, N, K, bn):
 
 def test_gemm_writes_nothing_past_c(dev):
     """Guard bytes after C stay, for widths that end inside a tile and a 16-byte piece."""
-    import _tglib as L
     for M, N, K in ((33, 65, 256), (70, 104, 384), (129, 1001, 128), (300, 72, 256)):
         a, sa, b, sb = _operands(dev, M, N, K, 1)
         buf = torch.full((M * N + 64,), 5.0, dtype=torch.bfloat16, device=dev)
@@ -52,3 +54,33 @@ def test_gemm_writes_nothing_past_c(dev):
                                        M, N, K, 128, L.stream_of(a)))
         assert torch.equal(buf[:M * N].reshape(M, N), fp8.scaled_matmul(a, sa, b, sb))
         assert bool((buf[M * N:] == 5.0).all())
+
+
+@pytest.mark.parametrize("bn", [1, 128])
+@pytest.mark.parametrize("M,N,K,km", [c for t in sorted(G.GEMM) for c in G.GEMM[t]])
+def test_every_tile_gives_the_bits_of_the_smallest(dev, M, N, K, km, bn):
+    """bf16 and f32 outputs of a launch against those of 256 x 512 pieces on 32 x 64 tiles, 64 rows of it against
+    float64, and nothing written past C."""
+    a, sa, b, sb = _operands(dev, M, N, K, bn)
+    fn = L.lib().tg_gemm_fp8_nt_km if km else L.lib().tg_gemm_fp8_nt
+    la, lb = (x.t().contiguous() if km else x for x in (sa, sb))
+    outs = []
+    for code, dt in ((L.TG_DTYPE_BF16, torch.bfloat16), (L.TG_DTYPE_F32, torch.float32)):
+        buf = torch.full((M * N + 64,), 5.0, dtype=dt, device=dev)
+        L.check(fn(a.data_ptr(), la.data_ptr(), b.data_ptr(), lb.data_ptr(), bn, buf.data_ptr(), code, M, N, K, 128,
+                   L.stream_of(a)))
+        assert bool((buf[M * N:] == 5.0).all())
+        outs.append(buf[:M * N].reshape(M, N))
+    c16, c32 = outs
+    assert torch.equal(c16, c32.to(torch.bfloat16))
+    assert G.tile_of(256, 512, K, False, f32=True) == (32, 64)
+    for m in range(0, M, 256):
+        for n in range(0, N, 512):
+            part = fp8.scaled_matmul(a[m:m + 256], sa[m:m + 256], b[n:n + 512], sb[n // bn:-(-(n + 512) // bn)],
+                                     b_scale_bn=bn, out_dtype=torch.float32)
+            assert torch.equal(part, c32[m:m + 256, n:n + 512]), (m, n)
+    rows = torch.linspace(0, M - 1, 64, device=dev).long()
+    ad = a[rows].view(torch.float8_e4m3fn).double() * sa[rows].double().repeat_interleave(128, 1)
+    bd = b.view(torch.float8_e4m3fn).double() * sb.double().repeat_interleave(bn, 0)[:N].repeat_interleave(128, 1)
+    ref = ad @ bd.t().contiguous()
+    assert float((c32[rows].double() - ref).abs().max()) <= 5e-5 * float(ref.abs().max())

@@ -8,6 +8,7 @@ import torch.nn.functional as F
 
 import _tglib as L
 import fp8
+import gemm_tiles as G
 
 pytestmark = pytest.mark.gpu
 
@@ -67,6 +68,15 @@ def test_linear_same_bits_as_general_path(dev, M, K, N, adt, bdt):
     ry, rda, rdb = _general(a.detach(), b.detach(), g)
     assert torch.equal(y, ry) and torch.equal(da, rda.to(adt)) and torch.equal(db, rdb.to(bdt))
     assert torch.equal(fp8._fp8_forward(a.detach(), b.detach(), 128), ry)
+
+
+@pytest.mark.parametrize("M,K,N", sorted(G.LINEAR_F32))
+def test_f32_linear_on_every_tile(dev, M, K, N):
+    """The f32 gradients hold the bf16 results, on each tile that a linear's dX and dW take."""
+    a, b, g = _inputs(dev, M, K, N, F32, F32)
+    da, db = fp8._linear_bwd(a, b, g)
+    _, rda, rdb = _general(a, b, g)
+    assert torch.equal(da, rda.float()) and torch.equal(db, rdb.float())
 
 
 @pytest.mark.parametrize("M,N", [(130, 257), (128, 256)])

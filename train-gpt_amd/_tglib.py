@@ -88,6 +88,11 @@ PREFILL_SIGNATURES = {
     "tg_prefill_kv": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp]),
 }
 
+# include/tg_fp8_tiles.h: the FP8 GEMM's tile choice
+TILE_SIGNATURES = {
+    "tg_gemm_fp8_tile": (_int, [_i64, _i64, _i64, _int, _int, _int, _vp, _vp]),
+}
+
 _lib = None
 
 
@@ -100,7 +105,8 @@ def lib():
                 f"{LIB_PATH} is missing: build it with `python train-gpt_amd/build.py` "
                 "(the FP8 hot path has no non-HIP implementation)")
         L = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in (*SIGNATURES.items(), *TRAIN_SIGNATURES.items(), *PREFILL_SIGNATURES.items()):
+        for name, (res, args) in (*SIGNATURES.items(), *TRAIN_SIGNATURES.items(), *PREFILL_SIGNATURES.items(),
+                                  *TILE_SIGNATURES.items()):
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args

@@ -30,6 +30,7 @@
 #include "tg_device.h"
 #include "tg_host.h"
 #include "gemm_tile.h"
+#include "../../include/tg_fp8_tiles.h"
 
 namespace tg {
 
@@ -1116,51 +1117,66 @@ static int launch_gemm_lat(const uint8_t* a_q, const float* a_s, const uint8_t* 
 }
 
 // The kernels that give one GEMM's bits, and what each costs.  A tile's time is
-// a fixed part (first round trip, epilogue, launch) plus a part per K block,
-// measured on 256 CUs at 18 and 72 blocks; `two` are the times of a CU's two
-// resident workgroups together, for the shapes that leave room for two.  The
-// 64-row and 32-row tiles of four waves hide one workgroup's round trips and
-// barriers behind the other's MFMAs; the 128-row tiles of eight waves read
-// fewer bytes per product, and the 256 x 256 persistent kernel fewest.
-// us, before (128-row tiles of 64 to 192 columns) -> now: 512 x 2304 x 9216 36.0
-// -> 29.9, 512 x 6912 x 2304 18.0 -> 16.4, 128 x 2304 x 9216 34.9 -> 16.7, 768 x
-// 3072 x 2048 15.9 -> 12.9, 2048 x 2304 x 2304 22.5 -> 20.8, 3000 x 2304 x 9216
-// (4096 x 4352 x 4096) 108 -> 95 (113 -> 104).
+// a fixed part (first round trip, epilogue, launch) plus a part per K block;
+// f2, b2 are the times of a CU's two resident workgroups together, for the
+// shapes that leave room for two.  The 64-row and 32-row tiles of four waves hide
+// one workgroup's round trips and barriers behind the other's MFMAs; the 128-row
+// tiles of eight waves read fewer bytes per product, and the 256 x 256
+// persistent kernel fewest.  Kept weights come from HBM: each K block then takes
+// k1 (one workgroup) or k2 (two) more, a third of the block's time where two
+// workgroups of 64 rows share a CU and next to nothing with 128 rows, whose eight
+// waves have more copies in flight.  odd: the element stores of a bf16 tile whose
+// rows are not 16-byte aligned (the 256 kernel's 2-byte stores cost it 33 us, 512
+// x 50257 against 50256 x 2304; a wider store beside the kept one takes registers
+// that the K loop needs: 5% to 4x slower).
+// The constants minimise the loss against the best tile over 2370 shapes on 256
+// CUs (64 to 9216 rows, 1 to 72 K blocks, every tile timed: weights rotated
+// through 640 MB, resident ones, and a training step's operands).  On 2370 others
+// the choice is 0.2% (rotated), 1.1% (resident kept weights) and 0.05% (training)
+// above the best tile on average, and no tile of the rule before it (128-row
+// tiles of 64 to 192 columns, 256 x 256 from 128 of them on) was more than 4%
+// faster with rotated weights.  us, that rule -> now: 512 x 2304 x 9216 36.0 ->
+// 29.9, 128 x 2304 x 9216 34.9 -> 16.7, 768 x 3072 x 2048 15.9 -> 12.9, 2048 x
+// 2304 x 2304 22.5 -> 20.8, 4096 x 4352 x 4096 113 -> 104; with rotated weights
+// 350 x 9216 x 2304 18.0 -> 18.1 (64 x 128 takes 20.3), 300 x 14336 x 4096 38.2
+// -> 38.0 (64 x 96 takes 44.5).
 struct GemmTile {
   int bm, bn, occ;
   float f1, b1, f2, b2;   // us: fixed and per K block, one and two workgroups on a CU
+  float k1, k2;           // us more per K block of a kept weight
+  float odd;              // us per tile of unaligned bf16 rows
 };
 constexpr GemmTile kGemmTiles[] = {
-    {256, 256, 1, 6.5f, 0.f, 0.f, 0.f},      // 0: gemm_fp8_nt_256_kernel (per block below)
-    {128, 256, 1, 7.5f, 1.22f, 0.f, 0.f},    // 1: lat <4, 8, 4, 1>
-    {128, 192, 1, 6.9f, 0.90f, 0.f, 0.f},    // 2: lat <4, 6, 4, 1>
-    {64, 128, 2, 3.8f, 0.446f, 4.3f, 0.634f},  // 3: lat <2, 4, 2, 2>
-    {64, 96, 2, 3.8f, 0.365f, 4.1f, 0.541f},   // 4: lat <2, 3, 2, 2>
-    {64, 64, 2, 3.6f, 0.267f, 3.9f, 0.459f},   // 5: lat <2, 2, 2, 2>
-    {32, 64, 2, 3.4f, 0.185f, 4.0f, 0.290f},   // 6: lat <1, 2, 2, 2>
+    {256, 256, 1, 6.5f, 1.28f, 0.f, 0.72f, 0.16f, 0.f, 33.f},      // 0: gemm_fp8_nt_256_kernel (b2: see below)
+    {128, 256, 1, 6.5f, 1.17f, 0.f, 0.f, 0.13f, 0.f, 0.6f},        // 1: lat <4, 8, 4, 1>
+    {128, 192, 1, 5.9f, 1.0f, 0.f, 0.f, 0.08f, 0.f, 0.6f},         // 2: lat <4, 6, 4, 1>
+    {64, 128, 2, 4.1f, 0.41f, 4.4f, 0.62f, 0.07f, 0.24f, 0.15f},   // 3: lat <2, 4, 2, 2>
+    {64, 96, 2, 4.0f, 0.37f, 4.1f, 0.56f, 0.06f, 0.22f, 0.1f},     // 4: lat <2, 3, 2, 2>
+    {64, 64, 2, 3.7f, 0.255f, 4.2f, 0.405f, 0.05f, 0.2f, 0.f},     // 5: lat <2, 2, 2, 2>
+    {32, 64, 2, 2.7f, 0.16f, 3.9f, 0.365f, 0.04f, 0.22f, 0.f},     // 6: lat <1, 2, 2, 2>
+    {128, 128, 1, 6.0f, 0.7f, 0.f, 0.f, 0.02f, 0.f, 0.3f},         // 7: lat <4, 4, 4, 1>
 };
 
 // The tile with the least modelled time.  Successive workgroups of a CU overlap
-// a launch's and a round trip's ~2 us.  The 256 kernel's block takes
-// 1.4 us on few CUs and 1.95 on all of them (the board's power), and output rows
-// that are not 16-byte aligned cost its tile 29 us more in 2-byte stores (512 x
-// 50257 against 50256 x 2304; a wider store beside the kept one takes registers
-// that the K loop needs: 5% to 4x slower).
-static int gemm_tile_of(int64_t m, int64_t n, int64_t nkb) {
-  const int64_t cus = device_cus() > 0 ? device_cus() : 1;
+// a launch's and a round trip's ~2 us.  The 256 kernel's block takes 1.28 us on
+// few CUs and b2 more on all of them (the board's power).  kept: row-major
+// scales, the layout of weights that are laid out once and multiplied many times
+// (the composites' own operands, just quantized, have K-block-major scales).
+static int gemm_tile_of(int64_t m, int64_t n, int64_t nkb, bool kept, bool bf16_out, int64_t cus) {
   int best = 0;
   double cost = 1e300;
   for (int i = 0; i < (int)(sizeof(kGemmTiles) / sizeof(kGemmTiles[0])); ++i) {
     const GemmTile& t = kGemmTiles[i];
     const int64_t wgs = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
-    const double r = (double)((wgs + cus - 1) / cus);
+    const int64_t ri = (wgs + cus - 1) / cus;
+    const double r = (double)ri, kb = (double)nkb, odd = bf16_out && n % 8 ? t.odd : 0.0;
+    const double k1 = kept ? t.k1 : 0.0, k2 = kept ? t.k2 : 0.0;
     double c;
     if (i == 0) {
-      const double fill = (double)wgs / (r * (double)cus), block = 1.4 + 0.55 * fill * fill;
-      c = r * (t.f1 + (n % 8 ? 29.0 : 0.0) + block * (double)nkb);
+      const double fill = (double)wgs / (r * (double)cus);
+      c = r * (t.f1 + odd + (t.b1 + t.b2 * fill * fill + k1) * kb);
     } else {
-      const double one = t.f1 + t.b1 * (double)nkb - 2.0, two = t.f2 + t.b2 * (double)nkb - 2.0;
-      const int64_t ri = (int64_t)r;
+      const double one = t.f1 + odd + (t.b1 + k1) * kb - 2.0, two = t.f2 + 2.0 * odd + (t.b2 + k2) * kb - 2.0;
       c = 2.0 + (t.occ == 2 ? (double)(ri / 2) * two + (double)(ri % 2) * one : r * one);
     }
     if (c < cost) {
@@ -1178,13 +1194,14 @@ static int launch_gemm_fp8_layout(const uint8_t* a_q, const float* a_s, const ui
   constexpr int BNS2 = OUT == kCF32Of16 ? 1 : 128;   // kCF32Of16 comes with b_scale_bn = 1 only
   if (fits32) {
 #define TG_LAT(...) launch_gemm_lat<__VA_ARGS__, SKM>(a_q, a_s, b_q, b_s, b_scale_bn, c, OUT, m, n, k, st)
-    switch (gemm_tile_of(m, n, k / 128)) {
+    switch (gemm_tile_of(m, n, k / 128, !SKM, OUT == kCBf16, device_cus() > 0 ? device_cus() : 1)) {
       case 1: return TG_LAT(4, 8, 4, 1);
       case 2: return TG_LAT(4, 6, 4, 1);
       case 3: return TG_LAT(2, 4, 2, 2);
       case 4: return TG_LAT(2, 3, 2, 2);
       case 5: return TG_LAT(2, 2, 2, 2);
       case 6: return TG_LAT(1, 2, 2, 2);
+      case 7: return TG_LAT(4, 4, 4, 1);
       default: break;
     }
 #undef TG_LAT
@@ -2191,6 +2208,19 @@ static int gemm_fp8_nt_entry(const char* who, const uint8_t* a_q, const float* a
     return launch_gemm_gb(a_q, a_s, b_q, b_s, b_scale_bn, c, c_dtype, M, N, K, block_k, as_stream(stream));
   if (!aligned(a_q, 16) || !aligned(b_q, 16)) return einval("gemm_fp8_nt: operands must be 16-byte aligned");
   return launch_gemm_fp8(a_q, a_s, b_q, b_s, b_scale_bn, c, c_dtype, M, N, K, as_stream(stream), skm);
+}
+
+extern "C" int tg_gemm_fp8_tile(int64_t M, int64_t N, int64_t K, int scales_km, int c_dtype, int cus, int* rows,
+                                int* cols) {
+  TG_TRY(check_gemm_args("gemm_fp8_tile", M, N, K, 128, 1));
+  if (c_dtype != TG_DTYPE_BF16 && c_dtype != TG_DTYPE_F32) return einval("gemm_fp8_tile: bad c_dtype");
+  if (cus <= 0) return einval("gemm_fp8_tile: cus must be positive");
+  if (!rows || !cols) return einval("gemm_fp8_tile: null pointer");
+  const bool tuned = gemm_fits32(M, N, K) && M > 0 && N > 0;
+  const int i = tuned ? gemm_tile_of(M, N, K / 128, !scales_km, c_dtype == TG_DTYPE_BF16, cus) : 0;
+  *rows = tuned ? kGemmTiles[i].bm : 0;
+  *cols = tuned ? kGemmTiles[i].bn : 0;
+  return TG_OK;
 }
 
 extern "C" int tg_gemm_fp8_nt(const uint8_t* a_q, const float* a_s, const uint8_t* b_q,
