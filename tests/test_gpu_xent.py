@@ -85,6 +85,13 @@ def test_xent_saturated_logits(dev):
     assert _grad_ok(logits.grad, g_ref)
 
 
+# rows of whole 16-byte words, shorter odd ones value by value, and odd ones as words from 3072 values on
+@pytest.mark.parametrize("cap", [CAP, 40.0])
+@pytest.mark.parametrize("V", [7, 513, 3064, 3071, 3072, 3073, 3079])
+def test_xent_row_forms(dev, V, cap):
+    test_xent_matches_float64(dev, 9, V, cap)
+
+
 @pytest.mark.parametrize("cap", [24.0, 25.0])
 def test_xent_table_range_edges(dev, cap):
     """Logits up to ~400 (past the table's 256) and down to 2^-30 (below its

@@ -79,10 +79,19 @@ __device__ __forceinline__ float block_lse(float m, float s) {
 // its own (their loads go out beside the words').  2048 x 50257, HBM-bound:
 // forward 40 us (5.1 TB/s), backward 90 us (4.6 TB/s); with 2-byte accesses for
 // every row that is not 16-byte aligned they took 112 and 181 us.
-struct RowSplit {
+// How a row is read (xent_mode): kElem, one value per thread and step; kWords,
+// rows of whole words; kSplit, any other row as words and single values.
+constexpr int kElem = 0, kWords = 1, kSplit = 2;
+template <int MODE> struct RowSplit {
   int head;            // values before the words
   int64_t n8, tail0;   // words; first value after them
   __device__ __forceinline__ RowSplit(const uint16_t* p, int64_t V) {
+    if (MODE == kWords) {
+      head = 0;
+      n8 = V >> 3;
+      tail0 = V;
+      return;
+    }
     const int64_t h = (int64_t)((0u - (uint32_t)(reinterpret_cast<uintptr_t>(p) >> 1)) & 7u);
     head = (int)(h < V ? h : V);
     n8 = (V - head) >> 3;
@@ -90,6 +99,7 @@ struct RowSplit {
   }
   // the single value of this thread, or -1: threads 0 .. 7 take the head, 8 .. 15 the tail
   __device__ __forceinline__ int64_t single(int64_t V) const {
+    if (MODE == kWords) return -1;
     const int64_t i = threadIdx.x < 8 ? (int64_t)threadIdx.x : tail0 + (int64_t)threadIdx.x - 8;
     return (threadIdx.x < 8 ? i < head : threadIdx.x < 16 && i < V) ? i : -1;
   }
@@ -116,6 +126,7 @@ __device__ __forceinline__ void lse_accum(const float* z, float& m, float& s) {
   lse_merge(m, s, zm, part);
 }
 
+template <int MODE>
 __global__ __launch_bounds__(kXentThreads) void xent_fwd_kernel(const uint16_t* __restrict__ logits,
                                                                const int64_t* __restrict__ tgt,
                                                                int64_t V, float cap, float inv_cap,
@@ -124,25 +135,30 @@ __global__ __launch_bounds__(kXentThreads) void xent_fwd_kernel(const uint16_t* 
   const int64_t row = blockIdx.x;
   const uint16_t* lr = logits + row * V;
   float m = -__builtin_inff(), s = 0.0f;
-  const RowSplit rs(lr, V);
-  const int64_t si = rs.single(V);
-  if (si >= 0) lse_merge(m, s, capped(__uint_as_float((uint32_t)lr[si] << 16), cap, inv_cap), 1.0f);
-  const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
-  const int64_t n8 = rs.n8;
-  int64_t c = threadIdx.x;
-  for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
-    uint4 w[kXentUnroll];
+  auto add1 = [&](int64_t i) { lse_merge(m, s, capped(__uint_as_float((uint32_t)lr[i] << 16), cap, inv_cap), 1.0f); };
+  if constexpr (MODE != kElem) {
+    const RowSplit<MODE> rs(lr, V);
+    const int64_t si = rs.single(V);
+    if (si >= 0) add1(si);
+    const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
+    const int64_t n8 = rs.n8;
+    int64_t c = threadIdx.x;
+    for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
+      uint4 w[kXentUnroll];
 #pragma unroll
-    for (int u = 0; u < kXentUnroll; ++u) w[u] = ldg_stream(p + c + u * kXentThreads);
-    float z[8 * kXentUnroll];
+      for (int u = 0; u < kXentUnroll; ++u) w[u] = ldg_stream(p + c + u * kXentThreads);
+      float z[8 * kXentUnroll];
 #pragma unroll
-    for (int u = 0; u < kXentUnroll; ++u) capped8(w[u], cap, inv_cap, z + 8 * u);
-    lse_accum<8 * kXentUnroll>(z, m, s);
-  }
-  for (; c < n8; c += kXentThreads) {
-    float z[8];
-    capped8(ldg_stream(p + c), cap, inv_cap, z);
-    lse_accum<8>(z, m, s);
+      for (int u = 0; u < kXentUnroll; ++u) capped8(w[u], cap, inv_cap, z + 8 * u);
+      lse_accum<8 * kXentUnroll>(z, m, s);
+    }
+    for (; c < n8; c += kXentThreads) {
+      float z[8];
+      capped8(ldg_stream(p + c), cap, inv_cap, z);
+      lse_accum<8>(z, m, s);
+    }
+  } else {
+    for (int64_t i = threadIdx.x; i < V; i += kXentThreads) add1(i);
   }
   const float lse = block_lse(m, s);
   if (threadIdx.x == 0) {
@@ -154,7 +170,7 @@ __global__ __launch_bounds__(kXentThreads) void xent_fwd_kernel(const uint16_t* 
   }
 }
 
-template <bool VEC>
+template <int MODE>
 __global__ __launch_bounds__(kXentThreads) void xent_bwd_kernel(const uint16_t* __restrict__ logits,
                                                                const int64_t* __restrict__ tgt,
                                                                const float* __restrict__ row_lse,
@@ -187,8 +203,8 @@ __global__ __launch_bounds__(kXentThreads) void xent_bwd_kernel(const uint16_t* 
   auto put1 = [&](int64_t i) {
     dr[i] = (uint16_t)(pack_bf16x2(grad(__uint_as_float((uint32_t)lr[i] << 16), i), 0.0f) & 0xFFFFu);
   };
-  if (VEC) {
-    const RowSplit rs(lr, V);
+  if constexpr (MODE != kElem) {
+    const RowSplit<MODE> rs(lr, V);
     const int64_t si = rs.single(V);
     if (si >= 0) put1(si);
     const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
@@ -276,6 +292,7 @@ __device__ __forceinline__ float block_sum_max(float s, uint32_t& mx, float* red
   return t;
 }
 
+template <int MODE>
 __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(8))) void xent_fwd_lut_kernel(const uint16_t* __restrict__ logits,
                                                                    const int64_t* __restrict__ tgt,
                                                                    int64_t rows, int64_t V, float cap,
@@ -294,28 +311,33 @@ __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(8)
       s += lut_at(lut, o0) + lut_at(lut, o1);
       mx = max(mx, max(m0, m1));
     };
-    const RowSplit rs(lr, V);
-    const int64_t si = rs.single(V);
-    if (si >= 0) {
+    auto add1 = [&](int64_t i) {
       uint32_t m;
-      s += lut_at(lut, lut_off<false>((uint32_t)lr[si], m));
-      mx = m;
-    }
-    const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
-    const int64_t n8 = rs.n8;
-    int64_t c = threadIdx.x;
-    for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
-      uint4 w[kXentUnroll];
+      s += lut_at(lut, lut_off<false>((uint32_t)lr[i], m));
+      mx = max(mx, m);
+    };
+    if constexpr (MODE != kElem) {
+      const RowSplit<MODE> rs(lr, V);
+      const int64_t si = rs.single(V);
+      if (si >= 0) add1(si);
+      const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
+      const int64_t n8 = rs.n8;
+      int64_t c = threadIdx.x;
+      for (; c + (kXentUnroll - 1) * kXentThreads < n8; c += kXentUnroll * kXentThreads) {
+        uint4 w[kXentUnroll];
 #pragma unroll
-      for (int u = 0; u < kXentUnroll; ++u) w[u] = ldg_stream(p + c + u * kXentThreads);
+        for (int u = 0; u < kXentUnroll; ++u) w[u] = ldg_stream(p + c + u * kXentThreads);
 #pragma unroll
-      for (int u = 0; u < kXentUnroll; ++u) {
-        add_word(w[u].x); add_word(w[u].y); add_word(w[u].z); add_word(w[u].w);
+        for (int u = 0; u < kXentUnroll; ++u) {
+          add_word(w[u].x); add_word(w[u].y); add_word(w[u].z); add_word(w[u].w);
+        }
       }
-    }
-    for (; c < n8; c += kXentThreads) {
-      const uint4 w = ldg_stream(p + c);
-      add_word(w.x); add_word(w.y); add_word(w.z); add_word(w.w);
+      for (; c < n8; c += kXentThreads) {
+        const uint4 w = ldg_stream(p + c);
+        add_word(w.x); add_word(w.y); add_word(w.z); add_word(w.w);
+      }
+    } else {
+      for (int64_t i = threadIdx.x; i < V; i += kXentThreads) add1(i);
     }
     const float S = block_sum_max(s, mx, red);
     if (threadIdx.x == 0) {
@@ -329,7 +351,7 @@ __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(8)
   }
 }
 
-template <bool VEC>
+template <int MODE>
 __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(6))) void xent_bwd_lut_kernel(const uint16_t* __restrict__ logits,
                                                                    const int64_t* __restrict__ tgt,
                                                                    const float* __restrict__ row_lse,
@@ -363,8 +385,8 @@ __global__ __launch_bounds__(kXentThreads) __attribute__((amdgpu_waves_per_eu(6)
       const float d = grad(lut_off<false>((uint32_t)lr[i], m), i);
       dr[i] = (uint16_t)(pack_bf16x2(d, 0.0f) & 0xFFFFu);
     };
-    if (VEC) {
-      const RowSplit rs(lr, V);
+    if constexpr (MODE != kElem) {
+      const RowSplit<MODE> rs(lr, V);
       const int64_t si = rs.single(V);
       if (si >= 0) put1(si);
       const uint4* p = reinterpret_cast<const uint4*>(lr + rs.head);
@@ -440,6 +462,25 @@ static int xent_check(const void* logits, const int64_t* tgt, int64_t rows, int6
   return TG_OK;
 }
 
+// How the rows are read.  16-byte accesses need the logits' and the gradient's
+// rows to cross 16-byte boundaries at the same elements: true of any two
+// 16-byte-aligned arrays (torch's), whatever the vocabulary; buffers offset
+// from each other keep the element-wise loop.  So do short rows: eight values
+// of one thread in turn take longer than one of each of 512 (odd vocabularies of
+// 1024 to 2047: backward 1.08x as words, of 4096 to 8191 0.90x; below 512 up to 1.7x).
+constexpr int64_t kSplitMin = 3072;
+static int xent_mode(const void* logits, const void* grad, int64_t vocab) {
+  if (vocab % 8 == 0 && aligned(logits, 16) && aligned(grad, 16)) return kWords;
+  const bool same = ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(grad)) & 15u) == 0;
+  return same && aligned(logits, 2) && vocab >= kSplitMin ? kSplit : kElem;
+}
+#define TG_XENT(mode, kern, grid, st, ...)                                                                  \
+  do {                                                                                                      \
+    if ((mode) == kWords) hipLaunchKernelGGL(kern<kWords>, grid, dim3(kXentThreads), 0, st, __VA_ARGS__);   \
+    else if ((mode) == kSplit) hipLaunchKernelGGL(kern<kSplit>, grid, dim3(kXentThreads), 0, st, __VA_ARGS__); \
+    else hipLaunchKernelGGL(kern<kElem>, grid, dim3(kXentThreads), 0, st, __VA_ARGS__);                     \
+  } while (0)
+
 extern "C" int tg_logit_cap_xent_fwd(const void* logits, const int64_t* targets, int64_t rows,
                                      int64_t vocab, float cap, float* row_loss, float* row_lse,
                                      void* stream) {
@@ -447,12 +488,13 @@ extern "C" int tg_logit_cap_xent_fwd(const void* logits, const int64_t* targets,
   if (rows == 0) return TG_OK;
   if (!row_loss || !row_lse) return einval("logit_cap_xent_fwd: null pointer");
   auto L = reinterpret_cast<const uint16_t*>(logits);
+  const int mode = xent_mode(logits, logits, vocab);
   if (cap <= kLutCapMax)
-    hipLaunchKernelGGL(xent_fwd_lut_kernel, dim3((unsigned)(rows < kLutGridFwd ? rows : kLutGridFwd)),
-                       dim3(kXentThreads), 0, as_stream(stream), L, targets, rows, vocab, cap, row_loss, row_lse);
+    TG_XENT(mode, xent_fwd_lut_kernel, dim3((unsigned)(rows < kLutGridFwd ? rows : kLutGridFwd)), as_stream(stream), L,
+            targets, rows, vocab, cap, row_loss, row_lse);
   else
-    hipLaunchKernelGGL(xent_fwd_kernel, dim3((unsigned)rows), dim3(kXentThreads), 0, as_stream(stream), L,
-                       targets, vocab, cap, 1.0f / cap, row_loss, row_lse);
+    TG_XENT(mode, xent_fwd_kernel, dim3((unsigned)rows), as_stream(stream), L, targets, vocab, cap, 1.0f / cap,
+            row_loss, row_lse);
   return check_launch("logit_cap_xent_fwd");
 }
 
@@ -463,31 +505,15 @@ extern "C" int tg_logit_cap_xent_bwd(const void* logits, const int64_t* targets,
   TG_TRY(xent_check(logits, targets, rows, vocab, cap));
   if (rows == 0) return TG_OK;
   if (!row_lse || !g || !dlogits) return einval("logit_cap_xent_bwd: null pointer");
-  // 16-byte accesses need the logits' and the gradient's rows to cross 16-byte
-  // boundaries at the same elements: true of any two 16-byte-aligned arrays
-  // (torch's), whatever the vocabulary; buffers offset from each other keep
-  // the element-wise loop
-  const bool vec = ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(dlogits)) & 15u) == 0 &&
-                   aligned(logits, 2);
   auto L = reinterpret_cast<const uint16_t*>(logits);
   auto D = reinterpret_cast<uint16_t*>(dlogits);
-  if (cap <= kLutCapMax) {
-    const dim3 grid((unsigned)(rows < kLutGridBwd ? rows : kLutGridBwd));
-    if (vec)
-      hipLaunchKernelGGL(xent_bwd_lut_kernel<true>, grid, dim3(kXentThreads), 0, as_stream(stream), L,
-                         targets, row_lse, g, g_scale, row_weight, rows, vocab, cap, D);
-    else
-      hipLaunchKernelGGL(xent_bwd_lut_kernel<false>, grid, dim3(kXentThreads), 0, as_stream(stream), L,
-                         targets, row_lse, g, g_scale, row_weight, rows, vocab, cap, D);
-    return check_launch("logit_cap_xent_bwd");
-  }
-  if (vec)
-    hipLaunchKernelGGL(xent_bwd_kernel<true>, dim3((unsigned)rows), dim3(kXentThreads), 0,
-                       as_stream(stream), L, targets, row_lse, g, g_scale, row_weight, vocab, cap,
-                       1.0f / cap, D);
+  const int mode = xent_mode(logits, dlogits, vocab);
+  if (cap <= kLutCapMax)
+    TG_XENT(mode, xent_bwd_lut_kernel, dim3((unsigned)(rows < kLutGridBwd ? rows : kLutGridBwd)), as_stream(stream), L,
+            targets, row_lse, g, g_scale, row_weight, rows, vocab, cap, D);
   else
-    hipLaunchKernelGGL(xent_bwd_kernel<false>, dim3((unsigned)rows), dim3(kXentThreads), 0,
-                       as_stream(stream), L, targets, row_lse, g, g_scale, row_weight, vocab, cap,
-                       1.0f / cap, D);
+    TG_XENT(mode, xent_bwd_kernel, dim3((unsigned)rows), as_stream(stream), L, targets, row_lse, g, g_scale, row_weight,
+            vocab, cap, 1.0f / cap, D);
   return check_launch("logit_cap_xent_bwd");
 }
+#undef TG_XENT
