@@ -186,10 +186,9 @@ __global__ __launch_bounds__(kAttnWaves * 64) void decode_attention_kernel(
   if (p < nfull) {
     load(B, p + 1);
     full(A);
-    last(B);
-  } else {
-    last(A);
+    A = B;                                                         // one copy of the last group's code
   }
+  last(A);
 
   // merge the 16 partial states (4 key rows x 4 waves) in a fixed order
   __shared__ float sm[16], sl[16];
