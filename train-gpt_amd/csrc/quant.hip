@@ -148,6 +148,7 @@ int launch_quant_tensors(const QuantTensor* t, int n, bool skm, hipStream_t st) 
     DualJobs jobs{};
     int cnt = 0, in = f32 ? kInF32 : kInVec;
     int64_t total = 0, widest = 0;
+    bool cols_only = true;
     for (int i = 0; i < n; ++i) {
       if ((t[i].x_dtype == TG_DTYPE_F32) != (f32 != 0) || t[i].rows == 0 || t[i].cols == 0) continue;
       if (cnt == 3) return einval("quantize: at most three tensors of a type");
@@ -155,6 +156,7 @@ int launch_quant_tensors(const QuantTensor* t, int n, bool skm, hipStream_t st) 
                       total % 8 == 0, skm, 0x7FFFFFFF));
       widest = t[i].cols > widest ? t[i].cols : widest;
       jobs.job[cnt].part = t[i].part;
+      cols_only = cols_only && t[i].part == 2;
       if (!f32) {
         const bool whole = t[i].rows % 128 == 0 && t[i].cols % 128 == 0 && aligned(t[i].x, 16);
         const bool words = t[i].cols % 2 == 0 && aligned(t[i].x, 4);
@@ -183,12 +185,18 @@ int launch_quant_tensors(const QuantTensor* t, int n, bool skm, hipStream_t st) 
     }
     const dim3 grid((unsigned)total);
     if (in == kInVec) hipLaunchKernelGGL((quant_dual_kernel<true, false>), grid, block, 0, st, jobs);
+    else if (f32)
+      hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInF32>), grid, block, 0, st, jobs);
+    // x.T alone by a kernel without the row half: one to seven columns, where its
+    // fixed cost is all there is, 5.0 us against 5.2
+    else if (in == kInBf16 && cols_only)
+      hipLaunchKernelGGL((quant_dual_kernel<false, true, false, true, kInBf16>), grid, block, 0, st, jobs);
     else if (in == kInBf16)
       hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInBf16>), grid, block, 0, st, jobs);
-    else if (in == kInBf16Any)
-      hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInBf16Any>), grid, block, 0, st, jobs);
+    else if (cols_only)
+      hipLaunchKernelGGL((quant_dual_kernel<false, true, false, true, kInBf16Any>), grid, block, 0, st, jobs);
     else
-      hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInF32>), grid, block, 0, st, jobs);
+      hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInBf16Any>), grid, block, 0, st, jobs);
     TG_TRY(check_launch("quant_tensors"));
   }
   return TG_OK;
