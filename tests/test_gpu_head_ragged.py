@@ -52,6 +52,23 @@ def test_gemm_bf16_ragged_rows_of_c(dev, M, N, off):
     assert bool((buf[:8 + off] == 9.0).all()) and bool((buf[8 + off + M * N:] == 9.0).all())
 
 
+# a wave's share of a row: 8, 16, 32 and 64 lanes to a row, one and two values left over, rows that end inside a batch
+# of eight stores, and rows that start on a word and between two
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("M", [1, 17, 66, 130])
+def test_gemm_bf16_narrow_rows_of_c(dev, M, off):
+    K = 64
+    for N in (1, 2, 3, 14, 15, 17, 18, 31, 33, 34, 63, 66, 97, 98, 113, 127, 129, 130, 131, 145, 161, 191, 194, 254, 290):
+        a = ((np.arange(M)[:, None] * 3 + np.arange(K)) % 5 - 2).astype(np.float32)
+        b = ((np.arange(N)[:, None] * 5 + 2 * np.arange(K)) % 7 - 3).astype(np.float32)
+        ta, tb = to_dev(ob.f32_to_bf16(a), dev), to_dev(ob.f32_to_bf16(b), dev)
+        buf = torch.full((M * N + 32,), 9.0, dtype=torch.bfloat16, device=dev)
+        c = buf[8 + off:8 + off + M * N]
+        L.check(L.lib().tg_gemm_bf16_nt(L.ptr(ta), L.ptr(tb), L.ptr(c), M, N, K, L.stream_of(ta)))
+        assert np.array_equal(bf16_bits(c.reshape(M, N)), ob.f32_to_bf16((a @ b.T).astype(np.float32))), N
+        assert bool((buf[:8 + off] == 9.0).all()) and bool((buf[8 + off + M * N:] == 9.0).all()), N
+
+
 # 192-wide tiles (few of them) at their edges, and 256-wide ones (a whole round);
 # 2, 6 and 10 slices of the four-stage ring
 @pytest.mark.parametrize("M,N,K", [(1, 192, 64), (255, 191, 64), (256, 200, 192), (257, 193, 192), (130, 384, 320),

@@ -203,13 +203,60 @@ __device__ __forceinline__ void q4_main_loop(const Q4Ctx& c, v4f (&acc)[4][NJ]) 
   }
 }
 
-// R rows of W = 16 NJ bf16 from LDS (256-byte rows, chunk c of row r at
-// c ^ (r & 15)) to C rows mw + r, columns nw .. nw + W - 1, by one wave; r0 is
-// the first row.  Rows of N % 8 == 0 go out as 16-byte pieces, W / 8 lanes per
-// row.  Other rows start at any even address: one row per instruction as up to
-// 64 consecutive 4-byte words from its first 4-byte boundary, and a single value
-// at either end where one is left over (2-byte stores of whole pieces touched
-// every line eight times).
+// R rows of cnt <= 128 bf16 from LDS (256-byte rows, chunk c of row r at c ^
+// (r & 15)) to C rows mw + r from column nw on, where they start at any even
+// address, by one wave; r0 (a multiple of 16) is the first row.  LW lanes to a
+// row: consecutive 4-byte words from its first 4-byte boundary, and a single
+// value at either end where one is left over; a lane without a value stores
+// past its descriptor's end, which is dropped, so no branch is taken.  Eight
+// instructions' words are read from LDS before the first is stored, in a loop
+// that is not unrolled: code that runs once waits for its own fetch.
+template <int R, int LW>
+__device__ __forceinline__ void q4_store_odd_rows(const uint8_t* l, __bf16* __restrict__ C, int M, int N, int mw,
+                                                  int nw, int cnt, int lane, int r0) {
+  constexpr int RPI = 64 / LW, IT = R / RPI, B = IT < 8 ? IT : 8;   // rows per instruction; instructions; a batch
+  constexpr uint32_t kDrop = 0xFFFFFFF0u;
+  const int sub = LW == 64 ? 0 : lane / LW, w = lane % LW, w1 = min(w + 1, 63);
+  auto word = [&](int r, int i) {
+    return *reinterpret_cast<const uint32_t*>(l + r * 256 + (((i >> 2) ^ (r & 15)) * 16) + (i & 3) * 4);
+  };
+#pragma unroll 1
+  for (int i0 = 0; i0 < IT; i0 += B) {
+    const int mb = __builtin_amdgcn_readfirstlane(mw + r0 + i0 * RPI), nb = __builtin_amdgcn_readfirstlane(nw);
+    if (mb >= M) break;
+    const int nrow = min(M - mb, B * RPI);
+    const uint8_t* first = reinterpret_cast<const uint8_t*>(C + (int64_t)mb * N + nb);
+    const uint32_t base = (uint32_t)(reinterpret_cast<uintptr_t>(first) & 3u);   // 0 or 2
+    const __amdgpu_buffer_rsrc_t rc = make_rsrc(first - base, (uint32_t)(((nrow - 1) * (int64_t)N + cnt) * 2) + base);
+    const bool singles = (N & 1) || base;   // else every row starts on a word and holds whole words
+    uint32_t own[B], next[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int r = r0 + (i0 + u) * RPI + sub;
+      own[u] = word(r, w);
+      next[u] = word(r, w1);
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int r = u * RPI + sub, o = (int)((base >> 1) + (uint32_t)(r & N)) & 1, n = (cnt - o) >> 1;
+      const uint32_t row = base + (uint32_t)r * (uint32_t)N * 2u, off = row + 2u * o + 4u * w;
+      const uint32_t v = o ? __builtin_amdgcn_alignbit(next[u], own[u], 16) : own[u];
+      const bool in = r < nrow;
+      __builtin_amdgcn_raw_buffer_store_b32(v, rc, in && w < n ? off : kDrop, 0, 0);
+      const bool tail = in && w == n && ((cnt - o) & 1), head = in && o && w == 0;
+      if (singles && LW == 8) {   // one lane may have both (two values in all)
+        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)v, rc, tail ? off : kDrop, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)own[u], rc, head ? row : kDrop, 0, 0);
+      } else if (singles) {
+        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(head ? own[u] : v), rc, head ? row : tail ? off : kDrop, 0, 0);
+      }
+    }
+  }
+}
+
+// The same for columns nw .. nw + W - 1 (W = 16 NJ, those below N) of any C.  Rows of
+// N % 8 == 0 go out as 16-byte pieces, W / 8 lanes per row; others as above
+// (2-byte stores of whole pieces touched every line eight times).
 template <int R, int NJ>
 __device__ __forceinline__ void q4_store_rows(const uint8_t* l, __bf16* __restrict__ C, int M, int N, int mw, int nw,
                                               int lane, int r0) {
@@ -227,21 +274,10 @@ __device__ __forceinline__ void q4_store_rows(const uint8_t* l, __bf16* __restri
   }
   const int cnt = min(16 * NJ, N - nw);
   if (cnt <= 0) return;
-  auto at = [&](int r, int e) {
-    return *reinterpret_cast<const uint16_t*>(l + r * PITCH + (((e >> 3) ^ (r & 15)) * 16) + (e & 7) * 2);
-  };
-#pragma unroll 4
-  for (int q = 0; q < R; ++q) {
-    const int r = r0 + q;
-    if (mw + r >= M) break;
-    uint16_t* dst = reinterpret_cast<uint16_t*>(C) + (int64_t)(mw + r) * N + nw;
-    const int o = (int)((reinterpret_cast<uintptr_t>(dst) >> 1) & 1);
-    const int e = 2 * lane + o;
-    const uint32_t lo = at(r, min(e, 127)), hi = at(r, min(e + 1, 127));
-    if (e + 1 < cnt) *reinterpret_cast<uint32_t*>(dst + e) = lo | (hi << 16);
-    else if (e < cnt) dst[e] = (uint16_t)lo;
-    if (o && lane == 0) dst[0] = at(r, 0);
-  }
+  if (cnt <= 16) q4_store_odd_rows<R, 8>(l, C, M, N, mw, nw, cnt, lane, r0);
+  else if (cnt <= 32) q4_store_odd_rows<R, 16>(l, C, M, N, mw, nw, cnt, lane, r0);
+  else if (cnt <= 64) q4_store_odd_rows<R, 32>(l, C, M, N, mw, nw, cnt, lane, r0);
+  else q4_store_odd_rows<R, 64>(l, C, M, N, mw, nw, cnt, lane, r0);
 }
 
 // Epilogue: lane (fr, fg) holds row i * 16 + fr and columns j * 16 + 4 fg .. +3
