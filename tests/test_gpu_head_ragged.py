@@ -37,6 +37,13 @@ def test_pack_any_even_address(dev, transpose, rows, cols, off):
     assert bool((y[out_rows * pitch:] == 7.0).all())
 
 
+# rows of fewer than 1024 output pieces, packed piece by piece over all rows, up to the edge (8120 -> 1016 pieces; 8184 -> 1024)
+@pytest.mark.parametrize("rows,cols,off", [(1, 64, 0), (7782, 64, 1), (5000, 65, 0), (300, 1, 1), (4, 8120, 1), (4, 8184, 1),
+                                           (1025, 1023, 0)])
+def test_pack_narrow_rows(dev, rows, cols, off):
+    test_pack_any_even_address(dev, 0, rows, cols, off)
+
+
 @pytest.mark.parametrize("M,N,off", [(3, 1, 0), (64, 127, 0), (65, 129, 1), (300, 258, 0), (257, 513, 1)])
 def test_gemm_bf16_ragged_rows_of_c(dev, M, N, off):
     """Output rows of any length and any even address: exact integer products,

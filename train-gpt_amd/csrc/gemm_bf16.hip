@@ -579,6 +579,32 @@ __global__ __launch_bounds__(256) void pack_bf16_rows_kernel(const uint16_t* __r
   }
 }
 
+// The same for rows narrower than a workgroup's 1024 pieces, over the pieces of
+// all rows in turn (one workgroup per row left most of its lanes idle: 7782 x 64
+// 11.2 us).
+__global__ __launch_bounds__(256) void pack_bf16_flat_kernel(const uint16_t* __restrict__ x,
+                                                             uint16_t* __restrict__ y, uint32_t total, int rows,
+                                                             int cols, uint32_t np) {
+  uint32_t base;
+  const __amdgpu_buffer_rsrc_t rx = u8_rsrc(x, (uint64_t)rows * (uint64_t)cols * 2u, base);
+  const uint32_t i0 = blockIdx.x * (256 * kRowPieces) + threadIdx.x;
+  U8Load l[kRowPieces];
+  uint32_t off[kRowPieces], p[kRowPieces];
+#pragma unroll
+  for (int u = 0; u < kRowPieces; ++u) {
+    const uint32_t i = min(i0 + 256 * u, total - 1), r = i / np;
+    p[u] = i - r * np;
+    off[u] = base + r * (uint32_t)cols * 2u + p[u] * 16u;
+    l[u] = u8_load(rx, off[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < kRowPieces; ++u) {
+    const uint32_t i = i0 + 256 * u;
+    if (i < total)
+      *reinterpret_cast<uint4*>(y + (int64_t)i * 8) = u8_first(u8_value(l[u], off[u]), (int64_t)cols - 8 * (int64_t)p[u]);
+  }
+}
+
 // Transposing pack of bf16 rows (16-byte-aligned ones, or with UA rows at any
 // even address, such as an odd vocabulary's): a 128 x 128 tile is loaded with 16-byte row loads into LDS
 // (pitch 272 B); lane p of a wave reads the column pair 2p, 2p + 1 one 32-bit
@@ -689,6 +715,12 @@ int launch_pack_bf16(const void* x, int x_dtype, int64_t rows, int64_t cols, int
     }
 #undef TG_PACK_T128
     return check_launch("pack_bf16_t128");
+  }
+  if (!transpose && wide && off32 && pitch / 8 < 256 * kRowPieces && rows * (pitch / 8) < 0x7FFFF000) {
+    const uint32_t np = (uint32_t)(pitch / 8), total = (uint32_t)rows * np;
+    hipLaunchKernelGGL(pack_bf16_flat_kernel, dim3((total + 256 * kRowPieces - 1) / (256 * kRowPieces)), dim3(256), 0, st,
+                       reinterpret_cast<const uint16_t*>(x), reinterpret_cast<uint16_t*>(y), total, r, c, np);
+    return check_launch("pack_bf16_flat");
   }
   if (!transpose && wide && off32) {
     const dim3 gr((unsigned)((pitch / 8 + 256 * kRowPieces - 1) / (256 * kRowPieces)),
