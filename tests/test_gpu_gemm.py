@@ -57,19 +57,19 @@ def test_layout_known_answer(dev):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 8, 128), (17, 40, 256), (130, 200, 384), (256, 256, 512),
-                                   # below 128 large tiles: the short-K ring kernel with 128 x 192
-                                   # tiles (C1; 1, 5 and 6 K blocks: no tail / a tail of 2 after a
-                                   # round of 3 stages), 128 x 128 (2048^2 on 256 CUs), 128 x 64 (few
-                                   # rows: 1 tile row over many CUs; 5 and 18 K blocks against 6
-                                   # stages) and N % 8 != 0 (element stores instead of staged rows)
+                                   # the short-K ring kernel on its 32- to 128-row tiles: 1, 2, 5,
+                                   # 6, 8 and 18 K blocks against its stages, N % 8 != 0 (element
+                                   # stores instead of staged rows).  Which tile a shape takes is
+                                   # modelled: gemm_tiles.py lists shapes for each of them, held to it by
+                                   # test_gemm_tile_choice.py and run in test_gpu_gemm_tiles.py
                                    (300, 136, 1024), (2048, 3072, 768), (2048, 3072, 640), (2048, 3072, 128),
                                    (2048, 2048, 256), (128, 6912, 2304), (640, 768, 640), (257, 1001, 640),
-                                   # >= 128 tiles of 256 x 256: the large-tile kernel, with ragged
-                                   # M / N edges and odd / even numbers of K blocks
+                                   # large outputs with ragged M / N edges and odd / even numbers of
+                                   # K blocks; the first two take the 256 x 256 kernel
                                    (2100, 4000, 384), (4096, 4096, 256), (3000, 2900, 640),
-                                   # more tiles than CUs: workgroups loop over 1-2 tiles, the next
-                                   # tile's first K block loaded during the current one's last;
-                                   # one K block per tile, and an odd count with N % 8 != 0
+                                   # more 256 x 256 tiles than CUs: workgroups of that kernel loop over
+                                   # 1-2 tiles, the next tile's first K block loaded during the current
+                                   # one's last (the first shape; N % 8 != 0 takes smaller tiles)
                                    (5000, 5000, 128), (4300, 4404, 384)])
 def test_scaled_gemm_random(dev, M, N, K):
     rng = np.random.default_rng(M * 7 + N)
@@ -123,9 +123,10 @@ def _structured_operands(M, N, K, bn):
 @pytest.mark.parametrize("bn", [1, 128])
 @pytest.mark.parametrize("M,N,K", [(5000, 5000, 384), (4300, 4404, 384), (8192, 8192, 2048)])
 def test_layout_known_answer_persistent_tiles(dev, M, N, K, bn):
-    """>= 128 tiles of 256 x 256 (the kernel bench.py times), with workgroups
-    walking several tiles, ragged edges and both weight-scale layouts; the C3
-    shape included.  Exact equality in f32, RNE of it in bf16."""
+    """Outputs of more 256 x 256 tiles than CUs (the kernel bench.py times,
+    where the tile rule takes it), with workgroups walking several tiles,
+    ragged edges and both weight-scale layouts; the C3 shape included.  Exact
+    equality in f32, RNE of it in bf16."""
     qa, sa, qb, sb, want = _structured_operands(M, N, K, bn)
     c32 = _gemm(qa, sa, qb, sb, dev, bn=bn, out=torch.float32).cpu().numpy()
     np.testing.assert_array_equal(c32, want.astype(np.float32))
@@ -137,10 +138,10 @@ def test_layout_known_answer_persistent_tiles(dev, M, N, K, bn):
                                       (200, 136, 384, 1), (96, 4404, 256, 128), (2048, 3072, 768, 1)])
 def test_gemm_km_same_bits(dev, M, N, K, bn):
     """tg_gemm_fp8_nt_km (scales K-block-major) = tg_gemm_fp8_nt on the
-    transposed scales, bit for bit, in bf16 and f32, on the persistent 256-tile
-    path (>= 128 tiles, ragged edges, both weight-scale layouts) and the
-    128-tile path.  (The composites use this path internally; their parity
-    tests cover it end to end.)"""
+    transposed scales, bit for bit, in bf16 and f32, large and small outputs,
+    ragged edges, both weight-scale layouts (the two entries price their
+    operands differently and may take different tiles).  (The composites use
+    this path internally; their parity tests cover it end to end.)"""
     import _tglib as L
     rng = np.random.default_rng(M + N + K + bn)
     qa, sa = fp8_ref.quantize_fp8(ob.bf16_to_f32(ob.randn_bf16(rng, (M, K))))
@@ -163,10 +164,9 @@ def test_gemm_km_same_bits(dev, M, N, K, bn):
 @pytest.mark.parametrize("M,K,N", [(200, 256, 200), (64, 384, 100), (300, 128, 1000), (2048, 768, 3072),
                                    (8192, 2048, 8192)])
 def test_composite_forward_same_bits_as_reference_layout(dev, M, K, N):
-    """tg_block_scaled_matmul (K-block-major scales in its workspace: the row
-    quantizer, the column quantizer's aligned, ragged and unaligned paths, and
-    both GEMM tile paths) = quantize_fp8 + scaled_matmul in the reference's
-    scale layout, bit for bit."""
+    """fp8.block_scaled_matmul (tg_linear_fwd: K-block-major scales in its
+    workspace, aligned, ragged and unaligned operands) = quantize_fp8 +
+    scaled_matmul in the reference's scale layout, bit for bit."""
     rng = np.random.default_rng(M + K + N)
     a = to_dev(ob.randn_bf16(rng, (M, K)), dev)
     b = to_dev(ob.randn_bf16(rng, (K, N), std=0.02), dev)
@@ -175,6 +175,50 @@ def test_composite_forward_same_bits_as_reference_layout(dev, M, K, N):
     qb, sb = fp8.quantize_fp8(b, transpose=True)
     want = fp8.scaled_matmul(qa.view(torch.uint8), sa, qb.view(torch.uint8), sb)
     assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
+def _quantized_product(x, y):
+    """scaled_matmul of x (R, K) and y (S, K), each quantized along its rows by itself."""
+    (qx, sx), (qy, sy) = fp8.quantize_fp8(x.contiguous()), fp8.quantize_fp8(y.contiguous())
+    return fp8.scaled_matmul(qx.view(torch.uint8), sx, qy.view(torch.uint8), sy)
+
+
+# whole tiles, ragged token counts and widths, rows of b that no 16-byte load takes, a single row and column
+@pytest.mark.parametrize("M,K,N", [(200, 256, 200), (64, 384, 100), (300, 128, 1000), (300, 256, 1001), (129, 384, 257),
+                                   (1, 128, 1), (127, 640, 130), (2048, 768, 3072)])
+def test_c_composite_forward(dev, M, K, N):
+    """tg_block_scaled_matmul through the C ABI at block_k 128: the bits of the separate quantizers and GEMM, the
+    float64 oracle within the bar, and nothing written past the output."""
+    import _tglib as L
+    rng = np.random.default_rng(3 * M + K + N)
+    ua, ub = ob.randn_bf16(rng, (M, K)), ob.randn_bf16(rng, (K, N), std=0.02)
+    a, b = to_dev(ua, dev), to_dev(ub, dev)
+    ws = torch.empty(L.lib().tg_block_scaled_matmul_workspace(M, N, K, 128), dtype=torch.uint8, device=dev)
+    buf = torch.full((M * N + 64,), 5.0, dtype=torch.bfloat16, device=dev)
+    L.check(L.lib().tg_block_scaled_matmul(L.ptr(a), L.ptr(b), L.ptr(buf), M, N, K, 128, L.ptr(ws), ws.numel(),
+                                           L.stream_of(a)))
+    y = buf[:M * N].reshape(M, N)
+    assert torch.equal(y, _quantized_product(a, b.t())) and bool((buf[M * N:] == 5.0).all())
+    _, ref, _, _ = fp8_ref.fp8_forward(ua, ub)
+    assert maxabs_rel(y, ref) <= TOL
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 128), (256, 384, 512), (512, 256, 768), (1024, 2304, 640)])
+def test_c_composite_backward(dev, M, N, K):
+    """tg_block_scaled_matmul_bwd_fp8 through the C ABI at block_k 128: dX and dW with the bits of the separate
+    quantizers and GEMM, and the float64 oracle within the bar."""
+    import _tglib as L
+    rng = np.random.default_rng(5 * M + N + K)
+    ua, ub, ug = ob.randn_bf16(rng, (M, K)), ob.randn_bf16(rng, (K, N), std=0.02), ob.randn_bf16(rng, (M, N), std=1e-3)
+    a, b, g = (to_dev(u, dev) for u in (ua, ub, ug))
+    ws = torch.empty(L.lib().tg_block_scaled_matmul_bwd_workspace(M, N, K, 128), dtype=torch.uint8, device=dev)
+    da, db = torch.empty_like(a), torch.empty_like(b)
+    L.check(L.lib().tg_block_scaled_matmul_bwd_fp8(L.ptr(a), L.ptr(b), L.ptr(g), L.ptr(da), L.ptr(db), M, N, K, 128,
+                                                   L.ptr(ws), ws.numel(), L.stream_of(a)))
+    assert torch.equal(da, _quantized_product(g, b))                     # g . b.T contracts N
+    assert torch.equal(db, _quantized_product(a.t(), g.t()))             # a.T . g contracts M
+    dx_ref, dw_ref, _ = fp8_ref.fp8_backward_fp8(ua, ub, ug)
+    assert maxabs_rel(da, dx_ref) <= TOL and maxabs_rel(db, dw_ref) <= TOL
 
 
 def test_block_scaled_matmul_c1(dev):
@@ -382,7 +426,7 @@ def test_fp8_backward_mode_switch_after_forward_raises(dev):
 
 
 def test_composite_forward_non_finite_operands(dev):
-    """NaN / +-inf in a and b through tg_block_scaled_matmul (fp8.py:50-78):
+    """NaN / +-inf in a and b through fp8.block_scaled_matmul (fp8.py:50-78):
     a NaN element gives its block a NaN scale, an infinite one an infinite
     scale and a NaN byte (inf / inf), so exactly the rows of a and the columns
     of b that hold one come out NaN (the oracle's float64 product); every

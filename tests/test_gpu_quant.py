@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+import _tglib as L
 import fp8
 from helpers import bf16_bits, f32_bits, same_scales, to_dev, u8
 from oracle import bf16 as ob
@@ -143,6 +144,26 @@ def test_quantize_dual_pair_equals_dual(dev, shapes):
                 assert torch.equal(g.view(torch.uint8), w.view(torch.uint8))
 
 
+def _km_outputs(x):
+    (R, C), u8, f32 = x.shape, torch.uint8, torch.float32
+    return [torch.empty(s, dtype=t, device=x.device)
+            for s, t in (((R, C), u8), ((C // 128, R), f32), ((C, R), u8), ((R // 128, C), f32))]
+
+
+def _dual_km(x):
+    """tg_quantize_dual_km: q, scales (C/128, R), q_t, scales_t (R/128, C)."""
+    o = _km_outputs(x)
+    L.check(L.lib().tg_quantize_dual_km(L.ptr(x), *x.shape, 128, *map(L.ptr, o), L.stream_of(x)))
+    return o
+
+
+def _dual_pair_km(x0, x1):
+    o0, o1 = _km_outputs(x0), _km_outputs(x1)
+    L.check(L.lib().tg_quantize_dual_pair_km(L.ptr(x0), *x0.shape, *map(L.ptr, o0), L.ptr(x1), *x1.shape, *map(L.ptr, o1),
+                                             128, L.stream_of(x0)))
+    return o0, o1
+
+
 @pytest.mark.parametrize("shape", [(128, 128), (256, 384), (1024, 640), (8192, 8192), (16384, 4096)])
 def test_quantize_dual_km_is_the_transposed_scale_layout(dev, shape):
     """tg_quantize_dual_km: the bytes of tg_quantize_dual, every scale array
@@ -153,7 +174,7 @@ def test_quantize_dual_km_is_the_transposed_scale_layout(dev, shape):
     x[:10, :128] = _special_rows(rng, 128)
     xd = to_dev(x, dev)
     q, s, qt, st = fp8.quantize_fp8_dual(xd)
-    kq, ks, kqt, kst = fp8._quantize_dual_km(xd, 128)
+    kq, ks, kqt, kst = _dual_km(xd)
     assert ks.shape == (shape[1] // 128, shape[0]) and kst.shape == (shape[0] // 128, shape[1])
     assert torch.equal(kq, q.view(torch.uint8)) and torch.equal(kqt, qt.view(torch.uint8))
     assert np.array_equal(f32_bits(ks), f32_bits(s).T) and np.array_equal(f32_bits(kst), f32_bits(st).T)
@@ -164,9 +185,9 @@ def test_quantize_dual_pair_km(dev, shapes):
     """tg_quantize_dual_pair_km = tg_quantize_dual_km on each tensor, bit for bit."""
     rng = np.random.default_rng(sum(map(sum, shapes)) + 5)
     xs = [to_dev(ob.randn_bf16(rng, s, std=0.02), dev) for s in shapes]
-    pair = fp8._quantize_dual_pair_km(xs[0], xs[1], 128)
+    pair = _dual_pair_km(*xs)
     for x, got in zip(xs, pair):
-        want = fp8._quantize_dual_km(x, 128)
+        want = _dual_km(x)
         for g, w in zip(got, want):
             assert np.array_equal(f32_bits(g), f32_bits(w)) if g.dtype == torch.float32 else torch.equal(g, w)
 

@@ -187,8 +187,8 @@ int launch_quant_tensors(const QuantTensor* t, int n, bool skm, hipStream_t st) 
     if (in == kInVec) hipLaunchKernelGGL((quant_dual_kernel<true, false>), grid, block, 0, st, jobs);
     else if (f32)
       hipLaunchKernelGGL((quant_dual_kernel<true, true, false, true, kInF32>), grid, block, 0, st, jobs);
-    // x.T alone by a kernel without the row half: one to seven columns, where its
-    // fixed cost is all there is, 5.0 us against 5.2
+    // x.T alone by a kernel without the row half: 384 rows of one to seven columns,
+    // where the fixed cost is all there is, 4.9 to 5.2 us against 5.1 to 5.3
     else if (in == kInBf16 && cols_only)
       hipLaunchKernelGGL((quant_dual_kernel<false, true, false, true, kInBf16>), grid, block, 0, st, jobs);
     else if (in == kInBf16)

@@ -36,8 +36,10 @@
 // (the FP8 backward on a token count or a width that no block divides): what
 // lies past x reads zero, which is the zero padding of a partial block, so q
 // rows are cp and q_t rows rp bytes wide (rows and cols rounded up to 128) and
-// no padded copy of x is made.  kInBf16: 16-byte-aligned bf16 rows; kInBf16Any:
-// bf16 rows at any even address (an odd width); kInF32: f32 rows, whose scale
+// no padded copy of x is made.  kInBf16: bf16 rows of an even width from a
+// 4-byte boundary on, so rows too start on one (read by buffer loads, which need
+// no more; not for 16-byte vector loads); kInBf16Any: bf16 rows at any even
+// address (an odd width); kInF32: f32 rows, whose scale
 // and quotient are IEEE divides and whose raw tile takes 65 KiB of LDS (row
 // pitch 130 words: the column reads, two values at a time, touch all 64 banks).
 // kInBf16Wide, kInF32Wide: the same tensors past 32-bit offsets or a 1-D grid

@@ -168,12 +168,6 @@ __device__ __forceinline__ uint32_t row16_max_u32(uint32_t v) {
   v = max(v, dpp_u32<0x140>(v));   // row_mirror
   return v;
 }
-// max over the 4 lanes of a quad
-__device__ __forceinline__ uint32_t quad_max_u32(uint32_t v) {
-  v = max(v, dpp_u32<0xB1>(v));
-  v = max(v, dpp_u32<0x4E>(v));
-  return v;
-}
 
 __device__ __forceinline__ double shfl_xor_f64(double v, int m) {
   int lo = __double2loint(v), hi = __double2hiint(v);

@@ -187,36 +187,6 @@ def quantize_fp8_dual_pair(x0: torch.Tensor, x1: torch.Tensor, block_k: int = DE
     return tuple((q.view(e4), s, qt.view(e4), st) for q, s, qt, st in outs)
 
 
-def _quantize_dual_km(x: torch.Tensor, block_k: int):
-    """quantize_fp8_dual with K-block-major scales (tg_quantize_dual_km): the
-    bytes of quantize_fp8_dual, scales stored transposed, (C/bk, R) and (R/bk, C)."""
-    R, C = x.shape
-    u8, f32 = torch.uint8, torch.float32
-    q = torch.empty((R, C), dtype=u8, device=x.device)
-    s = torch.empty((C // block_k, R), dtype=f32, device=x.device)
-    qt = torch.empty((C, R), dtype=u8, device=x.device)
-    st = torch.empty((R // block_k, C), dtype=f32, device=x.device)
-    _L.check(_L.lib().tg_quantize_dual_km(_L.ptr(x), R, C, block_k, _L.ptr(q), _L.ptr(s), _L.ptr(qt),
-                                          _L.ptr(st), _L.stream_of(x)))
-    return q, s, qt, st
-
-
-def _quantize_dual_pair_km(x0: torch.Tensor, x1: torch.Tensor, block_k: int):
-    """quantize_fp8_dual_pair with K-block-major scales (tg_quantize_dual_pair_km)."""
-    outs, args = [], []
-    u8, f32 = torch.uint8, torch.float32
-    for x in (x0, x1):
-        R, C = x.shape
-        o = (torch.empty((R, C), dtype=u8, device=x.device),
-             torch.empty((C // block_k, R), dtype=f32, device=x.device),
-             torch.empty((C, R), dtype=u8, device=x.device),
-             torch.empty((R // block_k, C), dtype=f32, device=x.device))
-        outs.append(o)
-        args += [_L.ptr(x), R, C] + [_L.ptr(v) for v in o]
-    _L.check(_L.lib().tg_quantize_dual_pair_km(*args, block_k, _L.stream_of(x0)))
-    return outs
-
-
 def scaled_matmul(a_q, a_s, b_q, b_s, b_scale_bn: int = 1, out_dtype=torch.bfloat16):
     """The scaled GEMM of fp8.py:70-76 on already-quantized operands ("NT"):
     a_q (M, K), b_q (N, K) e4m3fn; a_s (M, K/bk), b_s (N or ceil(N/128), K/bk)
@@ -331,11 +301,12 @@ def _fp8_backward(block_k, residuals, g):
     """Gradients of block_scaled_matmul: (da as a.dtype, db as b.dtype).
 
     BACKWARD_MODE "fp8": da = fwd(g, b.T), db = fwd(a.T, g) through FP8 MFMA.
-    N (da's contraction) and M (db's) need not divide by block_k: the operands
-    are zero-padded along them to a multiple of block_k.  Zeros change neither
-    a block's amax nor any product, so this is the FP8 rule with the last,
-    partial block quantized over its valid elements (fp8.py:39-47 defines only
-    whole blocks).
+    N (da's contraction) and M (db's) need not divide by block_k: the last,
+    partial block is quantized over its valid elements (fp8.py:39-47 defines
+    only whole blocks) and its products past them are zero.  tg_linear_bwd does
+    so at block_k 128; for other sizes the operands are zero-padded to a
+    multiple of block_k here, which changes neither a block's amax nor any
+    product.
     BACKWARD_MODE "bf16": fp8.py:85-98's straight-through rule, da = bf16(g) @
     bf16(b).T and db = bf16(a).T @ bf16(g), each a bf16 MFMA GEMM with fp32
     accumulation rounded once to bf16; block_k is unused, as in the reference.
