@@ -765,9 +765,10 @@ struct Q4Split {
 // times a split's slices plus 8 for its first round trip and its tile's store,
 // and for n > 1 the partial tiles written and read back (8 bytes per output and
 // split at ~5 TB/s) and the reduction's launch.  Measured:
-//   4096 x 2304 over 6912   144 tiles 142 us, 192 narrow ones 122; three splits
+//   4096 x 2304 over 6912   144 tiles 134 us, 192 narrow ones 118 (operands in the
+//                           caches; 176 and 152 with them from HBM); three splits
 //                           would move 226 MB of partial tiles
-//   512 x 768 over 3072     63 -> 54 us
+//   512 x 768 over 3072     55 -> 43 us
 //   4096 x 4096 over 4096   256 tiles 109 us, 352 narrow ones 152
 //   2048 x 50304 over 2304  1576 tiles 466 us, 2096 narrow ones 492
 //   2048 x 2304 over 50304  72 tiles 1219 us, three splits of them 479 + 12
